@@ -120,14 +120,5 @@ void fill_element_major(const DeviceLayout &L, int NpInt, const double *Q, doubl
   }
 }
 
-void read_element_major(const DeviceLayout &L, int NpInt, const double *h, double *Q) {
-  const int NV = 4 * NpInt, K = L.K;
-  for (int kk = 0; kk < L.K; ++kk) {
-    const int k = L.perm[kk];
-    for (int n = 0; n < 4; ++n)
-      for (int i = 0; i < NpInt; ++i) Q[size_t(n) * NpInt * K + size_t(i) * K + k] = h[size_t(kk) * NV + n * NpInt + i];
-  }
-}
-
 }  // namespace capi
 }  // namespace gocfd

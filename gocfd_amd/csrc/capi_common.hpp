@@ -70,6 +70,63 @@ struct StageTypeBuf {
   const void *ptr() const { return f.p ? static_cast<const void *>(f.p) : static_cast<const void *>(d.p); }
 };
 
+// Host states in the reference layout [4][NpInt][K] to and from the device's
+// element-major layout. The re-layout runs on the device: the host only
+// copies, through a device staging array of the reference layout's size and,
+// for states up to kPin bytes, one pinned host buffer. (On the host the
+// strided re-layout took 14 ms into and 18 ms out of the device at 80,000
+// triangles, order 4, 38 MB; the copies alone take 1.3 and 3.7 ms. A
+// pageable copy of 256 KB took 115 us where the pinned one and its host copy
+// take 14; from 4 MB on the pageable copy is as fast.) One transfer at a time:
+// calls on one handle are not re-entrant, and every entry point waits for its
+// stream before it returns.
+struct HostIo {
+  static constexpr size_t kPin = size_t(4) << 20;
+  DevBuf<double> stage;
+  double *pin = nullptr;
+  size_t npin = 0;
+  dev::Ctl *ctl = nullptr;  // behind the buffer, in the same pinned allocation
+  HostIo() = default;
+  HostIo(const HostIo &) = delete;
+  HostIo &operator=(const HostIo &) = delete;
+  ~HostIo() { if (pin) (void)hipHostFree(pin); }
+  void reserve(size_t vals) {
+    if (stage.n < vals) stage.alloc(vals);
+    const size_t bytes = vals * sizeof(double), want = bytes <= kPin ? bytes : 0;
+    if (!pin || npin < want) {
+      if (pin) (void)hipHostFree(pin);
+      pin = nullptr;
+      ctl = nullptr;
+      npin = 0;
+      HIPCHECK(hipHostMalloc(reinterpret_cast<void **>(&pin), want + sizeof(dev::Ctl), hipHostMallocDefault));
+      npin = want;
+      ctl = reinterpret_cast<dev::Ctl *>(reinterpret_cast<char *>(pin) + want);
+    }
+  }
+  // Q is free again on return; the re-layout may still run on the stream
+  void put(const double *Q, const int *perm, int K, int Kp, int NpInt, bool inert, double *dst, hipStream_t s) {
+    const size_t vals = size_t(K) * 4 * NpInt, bytes = vals * sizeof(double);
+    reserve(vals);
+    if (bytes <= kPin) {
+      std::memcpy(pin, Q, bytes);
+      HIPCHECK(hipMemcpyAsync(stage.p, pin, bytes, hipMemcpyHostToDevice, s));
+    } else {
+      HIPCHECK(hipMemcpyAsync(stage.p, Q, bytes, hipMemcpyHostToDevice, s));
+      HIPCHECK(hipStreamSynchronize(s));
+    }
+    HIPCHECK(dev::launch_gather_state(stage.p, perm, K, Kp, NpInt, inert, dst, s));
+  }
+  // Returns when Q is written
+  void get(const double *src, const int *perm, int K, int NpInt, double *Q, hipStream_t s) {
+    const size_t vals = size_t(K) * 4 * NpInt, bytes = vals * sizeof(double);
+    reserve(vals);
+    HIPCHECK(dev::launch_scatter_state(src, perm, K, NpInt, stage.p, s));
+    HIPCHECK(hipMemcpyAsync(bytes <= kPin ? pin : Q, stage.p, bytes, hipMemcpyDeviceToHost, s));
+    HIPCHECK(hipStreamSynchronize(s));
+    if (bytes <= kPin) std::memcpy(Q, pin, bytes);
+  }
+};
+
 // Freestream (model_problems/Euler2D/fluids.go:245-273)
 struct FreeStream {
   double gamma = 1.4, minf = 0, alpha = 0, q[4] = {1, 0, 0, 0}, pinf = 0, cinf = 0;
@@ -111,9 +168,8 @@ void check_device(int device, size_t lds_bytes);
 dev::Phys phys_of(const CaseStreams &fs, const gocfd_params &p);
 
 // Element-major FP64 device layout of a reference-layout state, padding
-// elements set to the inert state
+// elements set to the inert state (host side: an ensemble's initial states)
 void fill_element_major(const DeviceLayout &L, int NpInt, const double *Q, double *h);
-void read_element_major(const DeviceLayout &L, int NpInt, const double *h, double *Q);
 
 }  // namespace capi
 }  // namespace gocfd

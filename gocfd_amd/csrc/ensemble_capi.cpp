@@ -108,6 +108,7 @@ struct EnsGroup {
   DevBuf<int> code, nbr_slot, halo_elem, halo_face, wave_list, wave_cnt, wave_code, flux_list, flux_cnt, bnd_cnt, tile_case;
   // halo traces (without shock capturing): export lists and the two buffers
   DevBuf<int> xp_list, xp_dst, xp_cnt;
+  DevBuf<int> perm;                    // [Kp] device element -> element of its case (-1: padding)
   DevBuf<double> ht;
   StageTypeBuf flux_geo;
   void *q[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
@@ -140,6 +141,7 @@ struct gocfd_ensemble {
   std::vector<std::unique_ptr<EnsCase>> cases;
   std::vector<std::unique_ptr<EnsGroup>> groups;
   DevBuf<dev::CaseInfo> cinfo;
+  HostIo io;
   dev::Ctl *ctl = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr, fork = nullptr;
@@ -461,6 +463,7 @@ void build_group(gocfd_ensemble &h, EnsGroup &g) {
   std::vector<int> xp_list(size_t(g.ntiles) * g.Xmax, 0), xp_dst(size_t(g.ntiles) * g.Xmax, 0), xp_cnt(g.ntiles, 0);
   std::vector<double> flux_geo(size_t(g.ntiles) * g.Fmax * 4, 0.0);
   std::vector<double> q0(Kp * g.NV);
+  std::vector<int> perm(Kp, -1);
   for (int ci : g.cases) {
     const EnsCase &c = *h.cases[ci];
     const DeviceLayout &L = c.L;
@@ -506,6 +509,7 @@ void build_group(gocfd_ensemble &h, EnsGroup &g) {
         xp_dst[size_t(t0 + t) * g.Xmax + i] = (t0 + dt) * g.Fmax + di;
       }
     }
+    std::copy(L.perm.begin(), L.perm.end(), perm.begin() + o);
     fill_element_major(L, NpInt, c.Q0.data(), q0.data() + o * g.NV);
   }
   g.Jdet.upload(Jdet); g.Jinv.upload(Jinv); g.IInII.upload(IInII); g.Nx.upload(Nx); g.Ny.upload(Ny);
@@ -522,6 +526,7 @@ void build_group(gocfd_ensemble &h, EnsGroup &g) {
   g.flux_list.upload(flux_list); g.flux_cnt.upload(flux_cnt); g.bnd_cnt.upload(bnd_cnt);
   g.flux_geo.upload(flux_geo, h.prec, N);
   g.tile_case.upload(tile_case);
+  g.perm.upload(perm);
   if (!g.shock) {
     g.xp_list.upload(xp_list); g.xp_dst.upload(xp_dst); g.xp_cnt.upload(xp_cnt);
     g.ht.alloc(size_t(2) * g.ntiles * g.Fmax * NpEdge * 4);  // FP64 size, enough for either arithmetic
@@ -715,13 +720,10 @@ int gocfd_ensemble_get_state(gocfd_ensemble *h, int32_t c, double *Q) {
   GUARD_BEGIN
   if (!h || !Q || c < 0 || c >= int(h->cases.size())) return fail(GOCFD_ERR_ARG, "bad argument");
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   const EnsCase &cs = *h->cases[c];
   const EnsGroup &g = *h->groups[cs.group];
-  std::vector<double> buf(size_t(cs.L.Kp) * g.NV);
-  HIPCHECK(hipMemcpy(buf.data(), static_cast<double *>(g.q[0]) + size_t(cs.off) * g.NV,
-                     buf.size() * sizeof(double), hipMemcpyDeviceToHost));
-  read_element_major(cs.L, cs.d.ops.NpInt, buf.data(), Q);
+  h->io.get(static_cast<const double *>(g.q[0]) + size_t(cs.off) * g.NV, g.perm.p + cs.off, cs.L.K, cs.d.ops.NpInt, Q,
+            h->stream);
   return GOCFD_OK;
   GUARD_END
 }

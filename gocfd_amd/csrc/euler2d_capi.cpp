@@ -100,10 +100,8 @@ int gocfd_euler2d_create(const gocfd_mesh *mesh, const gocfd_params *p, gocfd_eu
   HIPCHECK(hipEventCreate(&h->ev1));
   const size_t nval = size_t(h->L.Kp) * h->NV;
   HIPCHECK(hipMalloc(&h->q[0], nval * sizeof(double)));
-  for (int s = 1; s < 5; ++s) {
-    HIPCHECK(hipMalloc(&h->q[s], nval * h->ssize));
-    HIPCHECK(hipMemset(h->q[s], 0, nval * h->ssize));
-  }
+  // every stage writes the whole of its output before the next one reads it
+  for (int s = 1; s < 5; ++s) HIPCHECK(hipMalloc(&h->q[s], nval * h->ssize));
   HIPCHECK(hipMalloc(&h->R, nval * sizeof(double)));
   HIPCHECK(hipMemset(h->R, 0, nval * sizeof(double)));
   HIPCHECK(hipMalloc(&h->ctl, sizeof(dev::Ctl)));
@@ -200,7 +198,6 @@ int gocfd_euler2d_get_state(gocfd_euler2d *h, double *Q) {
   if (!h || !Q) return fail(GOCFD_ERR_ARG, "null argument");
   NEED_DEVICE(h);
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   h->from_device(h->q[0], Q);
   return GOCFD_OK;
   GUARD_END
@@ -211,7 +208,6 @@ int gocfd_euler2d_get_residual(gocfd_euler2d *h, double *R) {
   if (!h || !R) return fail(GOCFD_ERR_ARG, "null argument");
   NEED_DEVICE(h);
   HIPCHECK(hipSetDevice(h->device));
-  HIPCHECK(hipStreamSynchronize(h->stream));
   h->from_device(h->R, R);
   return GOCFD_OK;
   GUARD_END
@@ -232,7 +228,6 @@ int gocfd_euler2d_rhs(gocfd_euler2d *h, const double *Q, double t, double *RHS) 
     HIPCHECK(dev::launch_fill_u64(h->sigV.p, h->sigV.n, 0ull, h->stream));
     HIPCHECK(dev::launch_fill_u64(h->epsV.p, h->epsV.n, 0ull, h->stream));
   }
-  HIPCHECK(hipStreamSynchronize(h->stream));
   h->from_device(h->rhs_out.p, RHS);
   return GOCFD_OK;
   GUARD_END
@@ -400,9 +395,9 @@ int gocfd_euler2d_vjp(gocfd_euler2d *h, int32_t nsteps, int32_t checkpoint_every
   capi::AdjointRunner &r = h->adjoint();
   const double t0 = h->current_time();
   const size_t tot = size_t(h->L.Kp) * h->NV;
-  DevBuf<double> lamN, lam0;
-  lamN.alloc(tot);
-  lam0.alloc(tot);
+  DevBuf<double> &lamN = h->deriv[0], &lam0 = h->deriv[1];
+  if (lamN.n < tot) lamN.alloc(tot);
+  if (lam0.n < tot) lam0.alloc(tot);
   h->to_device_zero_pad(dQn, lamN.p);
   double far[4];
   r.vjp(static_cast<const double *>(h->q[0]), t0, nsteps, checkpoint_every, lamN.p, lam0.p, far);
@@ -423,10 +418,9 @@ int gocfd_euler2d_jvp(gocfd_euler2d *h, int32_t nsteps, const double *dQ0, const
   capi::AdjointRunner &r = h->adjoint();
   const double t0 = h->current_time();
   const size_t tot = size_t(h->L.Kp) * h->NV;
-  DevBuf<double> dq0, qn, dqn;
-  dq0.alloc(tot);
-  qn.alloc(tot);
-  dqn.alloc(tot);
+  DevBuf<double> &dq0 = h->deriv[0], &qn = h->deriv[1], &dqn = h->deriv[2];
+  for (DevBuf<double> *b : {&dq0, &qn, &dqn})
+    if (b->n < tot) b->alloc(tot);
   h->to_device_zero_pad(dQ0, dq0.p);
   r.jvp(static_cast<const double *>(h->q[0]), dq0.p, dQinf, t0, nsteps, qn.p, dqn.p);
   if (Qn) h->from_device(qn.p, Qn);

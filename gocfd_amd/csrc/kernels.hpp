@@ -160,6 +160,14 @@ hipError_t launch_shock(int N, int prec, int pass, const StageArgs &a, hipStream
 hipError_t launch_ctl_init(Ctl *ctl, double time, hipStream_t s, int ncases = 1);
 hipError_t launch_fill_u64(unsigned long long *p, size_t n, unsigned long long v, hipStream_t s);
 hipError_t launch_fill_f64(double *p, size_t n, double v, hipStream_t s);
+// A state in the reference layout [4][NpInt][K] (device memory) -> the
+// device's element-major layout; padding elements (perm = -1) take the inert
+// state {1, 0, 0, 2.5}, or zero (cotangents and tangents). Every value of the
+// output is written.
+hipError_t launch_gather_state(const double *Q, const int *perm, int K, int Kp, int NpInt, bool inert, double *out,
+                               hipStream_t s);
+// The K real elements of an element-major state -> the reference layout
+hipError_t launch_scatter_state(const double *in, const int *perm, int K, int NpInt, double *Q, hipStream_t s);
 // Copy the order-N operators (DivInt^T [NpFlux][NpInt], FluxEdgeInterp
 // [3NpEdge][NpInt]) into the current device's constant memory.
 hipError_t upload_operators(int N, const double *divT, const double *interp);

@@ -106,6 +106,44 @@ __global__ void k_fill_f64(double *p, size_t n, double v) {
     p[i] = v;
 }
 
+__global__ void __launch_bounds__(256) k_gather_state(const double *__restrict__ Q, const int *__restrict__ perm,
+                                                      int K, int Kp, int NpInt, int inert, double *__restrict__ out) {
+  const int NV = 4 * NpInt;
+  const size_t n = size_t(Kp) * NV;
+  for (size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += size_t(gridDim.x) * blockDim.x) {
+    const int kk = int(idx / NV), r = int(idx - size_t(kk) * NV);
+    const int k = perm[kk];
+    double v = 0.0;
+    if (k >= 0) v = Q[size_t(r) * K + k];
+    else if (inert) v = r < NpInt ? 1.0 : r >= 3 * NpInt ? 2.5 : 0.0;
+    out[idx] = v;
+  }
+}
+
+__global__ void __launch_bounds__(256) k_scatter_state(const double *__restrict__ in, const int *__restrict__ perm,
+                                                       int K, int NpInt, double *__restrict__ Q) {
+  const int NV = 4 * NpInt;
+  const size_t n = size_t(K) * NV;
+  for (size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += size_t(gridDim.x) * blockDim.x) {
+    const int kk = int(idx / NV), r = int(idx - size_t(kk) * NV);
+    Q[size_t(r) * K + perm[kk]] = in[idx];
+  }
+}
+
+static int state_grid(size_t n) { return int(std::min<size_t>((n + 255) / 256, 8192)); }
+
+hipError_t launch_gather_state(const double *Q, const int *perm, int K, int Kp, int NpInt, bool inert, double *out,
+                               hipStream_t s) {
+  hipLaunchKernelGGL(k_gather_state, dim3(state_grid(size_t(Kp) * 4 * NpInt)), dim3(256), 0, s, Q, perm, K, Kp, NpInt,
+                     inert ? 1 : 0, out);
+  return hipGetLastError();
+}
+
+hipError_t launch_scatter_state(const double *in, const int *perm, int K, int NpInt, double *Q, hipStream_t s) {
+  hipLaunchKernelGGL(k_scatter_state, dim3(state_grid(size_t(K) * 4 * NpInt)), dim3(256), 0, s, in, perm, K, NpInt, Q);
+  return hipGetLastError();
+}
+
 hipError_t launch_ctl_init(Ctl *ctl, double time, hipStream_t s, int ncases) {
   hipLaunchKernelGGL(k_ctl_init, dim3((ncases + 63) / 64), dim3(64), 0, s, ctl, time, ncases);
   return hipGetLastError();

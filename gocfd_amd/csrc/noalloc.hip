@@ -28,40 +28,6 @@ constexpr int kMaxDevices = 64;
 double *g_scratch[kMaxDevices] = {};
 std::mutex g_scratch_mu;
 
-// Reference layout [4][NpInt][K] -> element-major [Kp][4 NpInt]; padding
-// elements (perm = -1) take the inert state {1, 0, 0, 2.5}, as the host-side
-// re-layout gives them. Every value of the output is written.
-__global__ void __launch_bounds__(256) k_gather_state(const double *__restrict__ Q, const int *__restrict__ perm,
-                                                      int K, int Kp, int NpInt, double *__restrict__ out) {
-  const int NV = 4 * NpInt;
-  const size_t n = size_t(Kp) * NV;
-  for (size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += size_t(gridDim.x) * blockDim.x) {
-    const int kk = int(idx / NV), r = int(idx - size_t(kk) * NV);
-    const int k = perm[kk];
-    double v;
-    if (k < 0) {
-      const int var = r / NpInt;
-      v = var == 0 ? 1.0 : var == 3 ? 2.5 : 0.0;
-    } else {
-      v = Q[size_t(r) * K + k];
-    }
-    out[idx] = v;
-  }
-}
-
-// Element-major RHS of the K real elements -> reference layout
-__global__ void __launch_bounds__(256) k_scatter_rhs(const double *__restrict__ in, const int *__restrict__ perm,
-                                                     int K, int NpInt, double *__restrict__ RHS) {
-  const int NV = 4 * NpInt;
-  const size_t n = size_t(K) * NV;
-  for (size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += size_t(gridDim.x) * blockDim.x) {
-    const int kk = int(idx / NV), r = int(idx - size_t(kk) * NV);
-    RHS[size_t(r) * K + perm[kk]] = in[idx];
-  }
-}
-
-int grid_for(size_t n) { return int(std::min<size_t>((n + 255) / 256, 8192)); }
-
 }  // namespace
 
 namespace gocfd {
@@ -98,18 +64,14 @@ extern "C" int gocfd_euler2d_rhs_noalloc(gocfd_euler2d *h, const double *Q, doub
   double *in = g_scratch[h->device], *out = in + vals;
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : h->stream;
   const int NpInt = h->d.ops.NpInt;
-  hipLaunchKernelGGL(k_gather_state, dim3(grid_for(vals)), dim3(256), 0, s, Q, h->perm.p, h->L.K, h->L.Kp, NpInt,
-                     in);
-  HIPCHECK(hipGetLastError());
+  HIPCHECK(dev::launch_gather_state(Q, h->perm.p, h->L.K, h->L.Kp, NpInt, true, in, s));
   dev::StageArgs a = h->rhs_args(in, t, out, s);
   h->launch_one_stage(a, s);
   if (h->shock) {  // the vertex buffers this evaluation used must be clear for the next stage
     HIPCHECK(dev::launch_fill_u64(h->sigV.p, h->sigV.n, 0ull, s));
     HIPCHECK(dev::launch_fill_u64(h->epsV.p, h->epsV.n, 0ull, s));
   }
-  const size_t nout = size_t(h->L.K) * h->NV;
-  hipLaunchKernelGGL(k_scatter_rhs, dim3(grid_for(nout)), dim3(256), 0, s, out, h->perm.p, h->L.K, NpInt, RHS);
-  HIPCHECK(hipGetLastError());
+  HIPCHECK(dev::launch_scatter_state(out, h->perm.p, h->L.K, NpInt, RHS, s));
   if (!stream) HIPCHECK(hipStreamSynchronize(s));
   return GOCFD_OK;
   GUARD_END
