@@ -95,6 +95,11 @@ void check_device(int device, size_t lds) {
                                           std::to_string(lds_max));
 }
 
+bool general_gamma(const dev::Phys &ph) {
+  auto is_14 = [](double g) { return std::fabs(1. / (g - 1.) - 2.5) < 1e-13; };
+  return !(is_14(ph.gamma) && is_14(ph.io[0].gamma) && is_14(ph.io[1].gamma));
+}
+
 dev::Phys phys_of(const CaseStreams &fs, const gocfd_params &p) {
   dev::Phys ph{};
   ph.gamma = fs.far.gamma; ph.minf = fs.far.minf; ph.pinf = fs.far.pinf; ph.cinf = fs.far.cinf;

@@ -165,6 +165,7 @@ void init_case(Discretisation &d, const gocfd_params &p, CaseStreams &fs, std::v
 void check_device(int device, size_t lds_bytes);
 
 // Physics constants of a case for the kernels
+bool general_gamma(const dev::Phys &ph);  // a far-field state whose gamma is not 1.4
 dev::Phys phys_of(const CaseStreams &fs, const gocfd_params &p);
 
 // Element-major FP64 device layout of a reference-layout state, padding

@@ -917,28 +917,39 @@ DeviceLayout build_device_layout(const Discretisation &d, int E, int TP) {
       }
     }
   }
-  // Non-shared faces per tile (the boundary loop of the stage kernel)
-  L.bnd_cnt.assign(L.ntiles, 0);
-  for (int kk = 0; kk < Kp; ++kk)
-    for (int f = 0; f < 3; ++f)
-      if ((L.face_code[size_t(f) * Kp + kk] & 15) != FK_Shared) ++L.bnd_cnt[kk / E];
+  // Boundary faces per tile, those with a boundary state first
+  auto has_state = [&](int code) { return (code & 15) == FK_Far || (code & 15) == FK_IVortex; };
+  L.bnd_ptr.assign(L.ntiles + 1, 0);
+  L.bst_cnt.assign(L.ntiles, 0);
+  for (int t = 0; t < L.ntiles; ++t) {
+    for (int pass = 0; pass < 2; ++pass)
+      for (int kk = t * E; kk < std::min(K, (t + 1) * E); ++kk)
+        for (int f = 0; f < 3; ++f) {
+          const size_t fi = size_t(f) * Kp + kk;
+          const int code = L.face_code[fi];
+          if ((code & 15) == FK_Shared || has_state(code) != (pass == 0)) continue;
+          if (pass == 0) ++L.bst_cnt[t];
+          L.bnd_item.push_back((kk % E) | (f << 8));
+          L.bnd_item.push_back(code);
+          for (double v : {L.Nx[fi], L.Ny[fi], L.IInII[fi], L.oohK[kk]}) L.bnd_geo.push_back(v);
+        }
+    L.bnd_ptr[t + 1] = int(L.bnd_item.size() / 2);
+  }
   // Faces whose owner-side trace enters the CFL wave-speed maximum, per tile
+  // (a face with a boundary state is always an owner, and its speed comes
+  // from the boundary items)
   std::vector<std::vector<int>> waves(L.ntiles);
   for (int kk = 0; kk < K; ++kk)
     for (int f = 0; f < 3; ++f)
-      if (L.face_code[size_t(f) * Kp + kk] & FC_WAVE) waves[kk / E].push_back((kk % E) | (f << 8));
+      if ((L.face_code[size_t(f) * Kp + kk] & FC_WAVE) && !has_state(L.face_code[size_t(f) * Kp + kk]))
+        waves[kk / E].push_back((kk % E) | (f << 8));
   L.Wmax = 1;
   for (auto &w : waves) L.Wmax = std::max<int>(L.Wmax, int(w.size()));
   L.wave_list.assign(size_t(L.ntiles) * L.Wmax, 0);
-  L.wave_code.assign(size_t(L.ntiles) * L.Wmax, 0);
   L.wave_cnt.assign(L.ntiles, 0);
   for (int t = 0; t < L.ntiles; ++t) {
     L.wave_cnt[t] = int(waves[t].size());
     std::copy(waves[t].begin(), waves[t].end(), L.wave_list.begin() + size_t(t) * L.Wmax);
-    for (size_t i = 0; i < waves[t].size(); ++i) {
-      const int w = waves[t][i];
-      L.wave_code[size_t(t) * L.Wmax + i] = L.face_code[size_t(w >> 8) * Kp + size_t(t) * E + (w & 255)];
-    }
   }
   L.Hmax = 1;
   for (auto &hl : halos) L.Hmax = std::max<int>(L.Hmax, int(hl.size()));

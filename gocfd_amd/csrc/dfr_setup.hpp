@@ -105,10 +105,11 @@ struct DeviceLayout {
   std::vector<int> nbr_elem;        // internal index of the neighbour (or -1)
   std::vector<double> Jdet, Jinv, IInII, Nx, Ny, oohK;  // geometry in internal order
   std::vector<int> halo_elem, halo_face;                // [ntiles x Hmax], -1 unused
-  int Wmax = 0;                                         // owned (wave-speed) faces per tile, max
+  // owned (wave-speed) faces per tile, without those that have a boundary
+  // state (whose speeds the boundary items give); Wmax: the most of a tile
+  int Wmax = 0;
   std::vector<int> wave_list;                           // [ntiles x Wmax]: e | face << 8
   std::vector<int> wave_cnt;                            // [ntiles]
-  std::vector<int> wave_code;                           // [ntiles x Wmax]: face_code of each wave_list face
   // Shared faces whose Riemann flux this tile evaluates: every face with an
   // out-of-tile neighbour, and the owner side of in-tile pairs (which also
   // fills the partner's slot). [ntiles x Fmax]: e | face << 8 | partner << 10
@@ -120,10 +121,13 @@ struct DeviceLayout {
   // partner's IInII negated (0 without partner)
   std::vector<double> flux_geo;
   std::vector<int> flux_cnt;                            // [ntiles]
-  // Faces of the tile's elements (padding included) that are not shared:
-  // boundary, inert and padding faces, whose flux the boundary loop sets.
-  // Tiles with none skip that loop. [ntiles]
-  std::vector<int> bnd_cnt;
+  // Faces of the tile's real elements that are not shared, tile after tile:
+  // the boundary faces, whose flux the boundary loop sets, those with a
+  // boundary state (far field, vortex) leading each tile's items. Items
+  // [bnd_ptr[t], bnd_ptr[t+1]): {e | face << 8, face_code} and the doubles
+  // {nx, ny, IInII, 1/hK}; bst_cnt [ntiles]: items with a boundary state.
+  std::vector<int> bnd_ptr, bst_cnt, bnd_item;
+  std::vector<double> bnd_geo;
   // Faces whose neighbour lies in another tile, per tile (the export list of
   // the halo traces): [ntiles x Xmax] e | face << 8, the halo-trace item slot
   // of the neighbour's face (its tile * Fmax + its flux-list item; the

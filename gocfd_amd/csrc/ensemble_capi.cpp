@@ -104,8 +104,9 @@ struct EnsGroup {
   double kappa = 0;
   int Nv = 0;                       // vertices of the group's cases
   std::vector<int> cases;
-  DevBuf<double> Jdet, Jinv, IInII, Nx, Ny, oohK, bxy, Interp64;
-  DevBuf<int> code, nbr_slot, halo_elem, halo_face, wave_list, wave_cnt, wave_code, flux_list, flux_cnt, bnd_cnt, tile_case;
+  DevBuf<double> Jdet, Jinv, IInII, Nx, Ny, oohK, bxy, Interp64, bnd_geo;
+  DevBuf<int> code, nbr_slot, halo_elem, halo_face, wave_list, wave_cnt, flux_list, flux_cnt, tile_case;
+  DevBuf<int> bnd_ptr, bst_cnt, bnd_item;
   // halo traces (without shock capturing): export lists and the two buffers
   DevBuf<int> xp_list, xp_dst, xp_cnt;
   DevBuf<int> perm;                    // [Kp] device element -> element of its case (-1: padding)
@@ -190,14 +191,17 @@ struct gocfd_ensemble {
     a.g.Jdet = g.Jdet.p; a.g.Jinv = g.Jinv.p; a.g.IInII = g.IInII.p; a.g.Nx = g.Nx.p; a.g.Ny = g.Ny.p;
     a.g.oohK = g.oohK.p; a.g.code = g.code.p; a.g.nbr_slot = g.nbr_slot.p;
     a.g.halo_elem = g.halo_elem.p; a.g.halo_face = g.halo_face.p; a.g.bxy = g.bxy.p;
-    a.g.wave_list = g.wave_list.p; a.g.wave_cnt = g.wave_cnt.p; a.g.wave_code = g.wave_code.p;
-    a.g.flux_list = g.flux_list.p; a.g.flux_cnt = g.flux_cnt.p; a.g.bnd_cnt = g.bnd_cnt.p;
+    a.g.wave_list = g.wave_list.p; a.g.wave_cnt = g.wave_cnt.p;
+    a.g.flux_list = g.flux_list.p; a.g.flux_cnt = g.flux_cnt.p;
+    a.g.bnd_ptr = g.bnd_ptr.p; a.g.bst_cnt = g.bst_cnt.p; a.g.bnd_item = g.bnd_item.p; a.g.bnd_geo = g.bnd_geo.p;
     a.g.flux_geo = g.flux_geo.ptr();
     a.g.xp_list = g.xp_list.p; a.g.xp_dst = g.xp_dst.p; a.g.xp_cnt = g.xp_cnt.p;
     a.ht = g.ht.p;
     a.Interp64 = g.Interp64.p;
     const EnsCase &c0 = *cases[g.cases[0]];
     a.ph = phys_of(c0.fs, c0.prm);
+    for (int ci : g.cases)
+      if (general_gamma(phys_of(cases[ci]->fs, cases[ci]->prm))) a.gen = 1;
     a.lts.on = g.lts ? 1 : 0;
     a.lts.fw = g.fw.p; a.lts.fwv = g.fwv.p; a.lts.wsrc = g.wsrc.p; a.lts.DTk = g.DTk.p; a.lts.DTv = g.DTv.p;
     if (g.shock) {
@@ -249,11 +253,12 @@ struct gocfd_ensemble {
         dev::MultiArgs m{};
         m.ngroups = int(mgroups.size());
         m.xcd_tiles = xcd_tiles;
+        for (int gi : mgroups) m.gen |= args(*groups[size_t(gi)]).gen;
         m.l = dev::MultiLaunch{s, step_index, int(gstage % 3), int(gstage & 1), int(gstage & 1)};
         int t0 = 0;
         for (size_t i = 0; i < mgroups.size(); ++i) {
           const EnsGroup &g = *groups[size_t(mgroups[i])];
-          m.g[i] = dev::MultiGroup{margs.p + i, t0, g.N, g.Fmax, g.Wmax + g.Xmax, g.lts ? 1 : 0};
+          m.g[i] = dev::MultiGroup{margs.p + i, t0, g.N, g.Fmax, g.Wmax + 2 * g.Xmax, g.lts ? 1 : 0};
           t0 += g.ntiles;
         }
         m.ntiles = t0;
@@ -459,7 +464,9 @@ void build_group(gocfd_ensemble &h, EnsGroup &g) {
   std::vector<int> code(3 * Kp), nbr_slot(3 * Kp), tile_case(g.ntiles);
   std::vector<int> halo_elem(size_t(g.ntiles) * g.Hmax, -1), halo_face(size_t(g.ntiles) * g.Hmax, 0);
   std::vector<int> wave_list(size_t(g.ntiles) * g.Wmax, 0), wave_cnt(g.ntiles, 0);
-  std::vector<int> flux_list(size_t(g.ntiles) * g.Fmax, 0), flux_cnt(g.ntiles, 0), bnd_cnt(g.ntiles, 0);
+  std::vector<int> flux_list(size_t(g.ntiles) * g.Fmax, 0), flux_cnt(g.ntiles, 0);
+  std::vector<int> bnd_ptr(1, 0), bst_cnt, bnd_item;
+  std::vector<double> bnd_geo;
   std::vector<int> xp_list(size_t(g.ntiles) * g.Xmax, 0), xp_dst(size_t(g.ntiles) * g.Xmax, 0), xp_cnt(g.ntiles, 0);
   std::vector<double> flux_geo(size_t(g.ntiles) * g.Fmax * 4, 0.0);
   std::vector<double> q0(Kp * g.NV);
@@ -495,7 +502,8 @@ void build_group(gocfd_ensemble &h, EnsGroup &g) {
       wave_cnt[t0 + t] = L.wave_cnt[t];
       for (int i = 0; i < L.wave_cnt[t]; ++i) wave_list[size_t(t0 + t) * g.Wmax + i] = L.wave_list[size_t(t) * L.Wmax + i];
       flux_cnt[t0 + t] = L.flux_cnt[t];
-      bnd_cnt[t0 + t] = L.bnd_cnt[t];
+      bst_cnt.push_back(L.bst_cnt[t]);
+      bnd_ptr.push_back(int(bnd_item.size() / 2) + L.bnd_ptr[t + 1] - L.bnd_ptr[0]);
       for (int i = 0; i < L.flux_cnt[t]; ++i) {
         flux_list[size_t(t0 + t) * g.Fmax + i] = L.flux_list[size_t(t) * L.Fmax + i];
         for (int c = 0; c < 4; ++c)
@@ -509,21 +517,22 @@ void build_group(gocfd_ensemble &h, EnsGroup &g) {
         xp_dst[size_t(t0 + t) * g.Xmax + i] = (t0 + dt) * g.Fmax + di;
       }
     }
+    for (size_t i = 0; i < L.bnd_item.size(); i += 2) {
+      int cd = L.bnd_item[i + 1];
+      if ((cd & 15) == FK_IVortex) cd = (cd & 0xff) | (((cd >> 8) + c.boff) << 8);
+      bnd_item.push_back(L.bnd_item[i]);
+      bnd_item.push_back(cd);
+    }
+    bnd_geo.insert(bnd_geo.end(), L.bnd_geo.begin(), L.bnd_geo.end());
     std::copy(L.perm.begin(), L.perm.end(), perm.begin() + o);
     fill_element_major(L, NpInt, c.Q0.data(), q0.data() + o * g.NV);
   }
   g.Jdet.upload(Jdet); g.Jinv.upload(Jinv); g.IInII.upload(IInII); g.Nx.upload(Nx); g.Ny.upload(Ny);
   g.oohK.upload(oohK); g.bxy.upload(bxy); g.code.upload(code); g.nbr_slot.upload(nbr_slot);
   g.halo_elem.upload(halo_elem); g.halo_face.upload(halo_face);
-  // the (group-offset) code of each wave-list face
-  std::vector<int> wave_code(size_t(g.ntiles) * g.Wmax, 0);
-  for (int t = 0; t < g.ntiles; ++t)
-    for (int i = 0; i < wave_cnt[t]; ++i) {
-      const int w = wave_list[size_t(t) * g.Wmax + i];
-      wave_code[size_t(t) * g.Wmax + i] = code[size_t(w >> 8) * Kp + size_t(t) * E + (w & 255)];
-    }
-  g.wave_list.upload(wave_list); g.wave_cnt.upload(wave_cnt); g.wave_code.upload(wave_code);
-  g.flux_list.upload(flux_list); g.flux_cnt.upload(flux_cnt); g.bnd_cnt.upload(bnd_cnt);
+  g.wave_list.upload(wave_list); g.wave_cnt.upload(wave_cnt);
+  g.flux_list.upload(flux_list); g.flux_cnt.upload(flux_cnt);
+  g.bnd_ptr.upload(bnd_ptr); g.bst_cnt.upload(bst_cnt); g.bnd_item.upload(bnd_item); g.bnd_geo.upload(bnd_geo);
   g.flux_geo.upload(flux_geo, h.prec, N);
   g.tile_case.upload(tile_case);
   g.perm.upload(perm);

@@ -111,8 +111,10 @@ int gocfd_euler2d_create(const gocfd_mesh *mesh, const gocfd_params *p, gocfd_eu
   h->bxy.upload(L.bpoint_xy);
   h->code.upload(L.face_code); h->nbr_slot.upload(L.nbr_slot);
   h->halo_elem.upload(L.halo_elem); h->halo_face.upload(L.halo_face);
-  h->wave_list.upload(L.wave_list); h->wave_cnt.upload(L.wave_cnt); h->wave_code.upload(L.wave_code);
-  h->flux_list.upload(L.flux_list); h->flux_cnt.upload(L.flux_cnt); h->bnd_cnt.upload(L.bnd_cnt);
+  h->wave_list.upload(L.wave_list); h->wave_cnt.upload(L.wave_cnt);
+  h->flux_list.upload(L.flux_list); h->flux_cnt.upload(L.flux_cnt);
+  h->bnd_ptr.upload(L.bnd_ptr); h->bst_cnt.upload(L.bst_cnt); h->bnd_item.upload(L.bnd_item);
+  h->bnd_geo.upload(L.bnd_geo);
   h->flux_geo.upload(L.flux_geo, h->prec, p->polynomial_order);
   h->perm.upload(L.perm);
   if (!h->shock) {

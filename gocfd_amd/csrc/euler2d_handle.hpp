@@ -37,8 +37,9 @@ struct gocfd_euler2d {
   void *R = nullptr;
   void *scratch_in = nullptr;
   DevBuf<double> rhs_out;
-  DevBuf<double> Jdet, Jinv, IInII, Nx, Ny, oohK, bxy, Interp64;
-  DevBuf<int> code, nbr_slot, halo_elem, halo_face, wave_list, wave_cnt, wave_code, flux_list, flux_cnt, bnd_cnt;
+  DevBuf<double> Jdet, Jinv, IInII, Nx, Ny, oohK, bxy, Interp64, bnd_geo;
+  DevBuf<int> code, nbr_slot, halo_elem, halo_face, wave_list, wave_cnt, flux_list, flux_cnt;
+  DevBuf<int> bnd_ptr, bst_cnt, bnd_item;
   HostIo io;
   DevBuf<double> deriv[3];  // states of a derivative call (kept for the next one)
   DevBuf<int> perm;  // [Kp] device element -> reference element (-1: padding)
@@ -91,8 +92,9 @@ struct gocfd_euler2d {
     a.g.Jdet = Jdet.p; a.g.Jinv = Jinv.p; a.g.IInII = IInII.p; a.g.Nx = Nx.p; a.g.Ny = Ny.p;
     a.g.oohK = oohK.p; a.g.code = code.p; a.g.nbr_slot = nbr_slot.p;
     a.g.halo_elem = halo_elem.p; a.g.halo_face = halo_face.p; a.g.bxy = bxy.p;
-    a.g.wave_list = wave_list.p; a.g.wave_cnt = wave_cnt.p; a.g.wave_code = wave_code.p;
-    a.g.flux_list = flux_list.p; a.g.flux_cnt = flux_cnt.p; a.g.bnd_cnt = bnd_cnt.p;
+    a.g.wave_list = wave_list.p; a.g.wave_cnt = wave_cnt.p;
+    a.g.flux_list = flux_list.p; a.g.flux_cnt = flux_cnt.p;
+    a.g.bnd_ptr = bnd_ptr.p; a.g.bst_cnt = bst_cnt.p; a.g.bnd_item = bnd_item.p; a.g.bnd_geo = bnd_geo.p;
     a.g.flux_geo = flux_geo.ptr();
     a.g.xp_list = xp_list.p; a.g.xp_dst = xp_dst.p; a.g.xp_cnt = xp_cnt.p;
     a.ht = ht.p;
@@ -114,6 +116,7 @@ struct gocfd_euler2d {
       a.sh.omega = 1. * double(d.N * d.N);
     }
     a.ph = phys_of(fs, prm);
+    a.gen = general_gamma(a.ph) ? 1 : 0;
     a.cases = cases.p;
     a.tile_case = tile_case.p;
     return a;

@@ -38,13 +38,17 @@ struct Geom {
   const double *Jdet, *Jinv, *IInII, *Nx, *Ny, *oohK;  // [Kp], [4][Kp], [3][Kp] x3, [Kp]
   const int *code, *nbr_slot;                          // [3][Kp]
   const int *halo_elem, *halo_face;                    // [ntiles][Hmax]
+  // owned faces without a boundary state
   const int *wave_list, *wave_cnt;                     // [ntiles][Wmax], [ntiles]
-  const int *wave_code;                                // [ntiles][Wmax]: code of each wave_list face
   const int *flux_list, *flux_cnt;                     // [ntiles][Fmax], [ntiles]
   // per flux-list item, in the stage arithmetic type: owner normal (nx, ny),
   // this side's signed IInII, the in-tile partner's IInII negated
   const void *flux_geo;                                // [ntiles][Fmax][4]
-  const int *bnd_cnt;                                  // [ntiles] non-shared faces
+  // Boundary faces, tile after tile (items [bnd_ptr[t], bnd_ptr[t+1])): {e |
+  // face << 8, face code}, {nx, ny, IInII, 1/hK}; the first bst_cnt[t] have a
+  // boundary state (far field, vortex)
+  const int *bnd_ptr, *bst_cnt, *bnd_item;
+  const double *bnd_geo;
   const double *bxy;                                   // IVortex boundary points
   // Faces whose neighbour lies in another tile, per tile: after a stage the
   // tile writes its traces of the new state there into the neighbour's face
@@ -122,6 +126,7 @@ struct StageArgs {
   int step_index;      // steps since the state was set (selects time parity)
   int ring;            // global stage counter mod 3
   int par2;            // global stage counter mod 2
+  int gen;             // 1: a case's gamma is not 1.4 (the boundary state needs a power)
   int hpar;            // halo-trace buffer holding this stage's input traces
   // Halo-trace buffers [2][ntiles Fmax][NpEdge][4] in the stage arithmetic
   // type (without shock capturing): by tile and flux-list item, the traces
@@ -182,13 +187,14 @@ struct MultiGroup {
   const StageArgs *a;   // the group's arguments (device memory)
   int tile0;            // its first tile in the launch's numbering
   int N;
-  int Fmax, WXmax, lts; // its LDS layout (host side)
+  int Fmax, WXints, lts; // its LDS layout (host side)
 };
 struct MultiLaunch {
   int stage, step_index, ring, par2, hpar;
 };
 struct MultiArgs {
   int ngroups, ntiles, xcd_tiles;
+  int gen;  // a group's gen
   MultiLaunch l;
   MultiGroup g[kMultiMax];
 };

@@ -283,7 +283,7 @@ __device__ __forceinline__ void atomic_max_bits(unsigned long long *p, double v)
   if (b > *reinterpret_cast<volatile unsigned long long *>(p)) atomicMax(p, b);
 }
 
-template <class C>
+template <bool GEN, class C>
 __device__ __forceinline__ void boundary_state(int kind, const Phys &ph, const double *bxy, int bidx,
                                                int NpEdge, int pp, double t, const C own[4],
                                                double nx, double ny, double qb[4]) {
@@ -302,7 +302,7 @@ __device__ __forceinline__ void boundary_state(int kind, const Phys &ph, const d
     const double *xy = bxy + 2 * (size_t(bidx) * NpEdge + pp);
     ivortex_state(t, xy[0], xy[1], qf);
   }
-  riemann_bc(gam, minf, pinf, cinf, qi, qf, nx, ny, qb);
+  riemann_bc<double, double, GEN>(gam, minf, pinf, cinf, qi, qf, nx, ny, qb);
 }
 
 // Wave speed (|U| + c) / hK of a face point (StoreEdgeAggregates, edges.go:264-272)
@@ -319,8 +319,8 @@ __device__ __forceinline__ double point_speed(double g, const double q[4], doubl
 // 32 bytes), the Riemann
 // items' geometry [Fmax][4] and the elements' metric terms [6][kTile];
 // without shock capturing, phase G's lists: the elements' 1/hK [kTile]
-// (FP64), the owned faces with their codes [2][Wmax] and the export items
-// with their destinations [2][Xmax] (ints); local time stepping adds the
+// (FP64), the owned faces [Wmax] and the export items with their
+// destinations [2][Xmax] (ints; WXints = Wmax + 2 Xmax); local time stepping adds the
 // element dt and face-speed buffers.
 template <int N>
 __host__ __device__ constexpr size_t lds_trace_bytes(size_t csize, int Hmax, bool mf) {
@@ -328,9 +328,9 @@ __host__ __device__ constexpr size_t lds_trace_bytes(size_t csize, int Hmax, boo
                    4 * (size_t(Shape<N>::NF) * kTP + size_t(Shape<N>::NpEdge) * Hmax)) + 31) / 32 * 32;
 }
 template <int N>
-__host__ __device__ constexpr size_t lds_tile_bytes(size_t csize, int Hmax, int Fmax, int WXmax, bool mf) {
+__host__ __device__ constexpr size_t lds_tile_bytes(size_t csize, int Hmax, int Fmax, int WXints, bool mf) {
   return lds_trace_bytes<N>(csize, Hmax, mf) + csize * (4 * size_t(Fmax) + 6 * kTile) +
-         (WXmax > 0 ? (sizeof(double) * kTile + 2 * sizeof(int) * size_t(WXmax) + 15) / 16 * 16 : 0);
+         (WXints > 0 ? (sizeof(double) * kTile + sizeof(int) * size_t(WXints) + 15) / 16 * 16 : 0);
 }
 constexpr size_t lds_lts_bytes = sizeof(double) * kTile + sizeof(unsigned long long) * 3 * kTile;
 
@@ -366,16 +366,25 @@ __device__ __forceinline__ bool step_skipped(const StageLaunch &l, const Ctl *ct
 #ifndef GOCFD_WAVES_F64
 #define GOCFD_WAVES_F64 3
 #endif
-template <class S, bool LAST, bool SHOCK>
+// No stage kernel may spill vector registers: with scalar registers spilled to
+// vector lanes as well, this compiler (clang 22, ROCm 7.2) puts a block's
+// vector spill stores among the lane writes at the head of the block, before
+// the exec mask is restored, so the lanes that were off (those without a
+// Riemann item) store nothing and reload garbage -- addresses among it. The
+// build's spill counts are checked by a test. GEN (a gamma other than 1.4)
+// needs the registers of pow, so it takes one wave per SIMD less; so does
+// Roe-ER at order 4 in FP64.
+template <int N, class S, int FLUX, bool LAST, bool SHOCK, bool GEN>
 struct StageWaves {
-  static constexpr int value =
-      SHOCK ? 1 : sizeof(S) == 4 ? (LAST ? GOCFD_WAVES_F32_LAST : GOCFD_WAVES_F32) : GOCFD_WAVES_F64;
+  static constexpr int value = SHOCK            ? 1
+                               : sizeof(S) == 4 ? (LAST || GEN ? GOCFD_WAVES_F32_LAST : GOCFD_WAVES_F32)
+                                                : (N == 4 && (GEN || FLUX == 3) ? 2 : GOCFD_WAVES_F64);
 };
 
 // S: storage of the stage states q1..q4; SIN: storage of this stage's
 // input (q0 at stage 0 and for the RHS evaluation, else S). q0 and the
 // stage-3 RHS R, which accumulate the step, are always FP64.
-template <int N, class S, class SIN, class C, int FLUX, bool LAST, bool SHOCK>
+template <int N, class S, class SIN, class C, int FLUX, bool LAST, bool SHOCK, bool GEN>
 __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch &l, const int tile) {
   using Sh = Shape<N>;
   constexpr int NpInt = Sh::NpInt, NpEdge = Sh::NpEdge, NF = Sh::NF, NV = Sh::NV, NR = Sh::NR;
@@ -401,12 +410,11 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   // phase G's lists (without shock capturing)
   double *sOK = reinterpret_cast<double *>(sJ + 6 * E);  // [E] 1/hK
   int *sWP = reinterpret_cast<int *>(sOK + E);           // [Wmax] owned faces e | f << 8
-  int *sWC = sWP + a.Wmax;                               // [Wmax] their codes
-  int *sXP = sWC + a.Wmax, *sXD = sXP + a.Xmax;          // [Xmax] export items, destinations
+  int *sXP = sWP + a.Wmax, *sXD = sXP + a.Xmax;          // [Xmax] export items, destinations
   // local time stepping only: element dt and per-face speed maxima, after
   // the tile buffers (the launch adds their bytes only when LTS is on)
   double *sDT = reinterpret_cast<double *>(
-      smem_raw + lds_tile_bytes<N>(sizeof(C), HX ? 0 : a.Hmax, a.Fmax, HX ? a.Wmax + a.Xmax : 0, MF));
+      smem_raw + lds_tile_bytes<N>(sizeof(C), HX ? 0 : a.Hmax, a.Fmax, HX ? a.Wmax + 2 * a.Xmax : 0, MF));
   unsigned long long *sWf = reinterpret_cast<unsigned long long *>(sDT + kTile);
   __shared__ double red[kThreads / 64];
 
@@ -439,22 +447,20 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     jm0 = c == 0 ? a.g.Jdet[k0 + e] : a.g.Jinv[size_t(c - 1) * Kp + k0 + e];
     if (c == 0) jm1 = a.g.Jinv[3 * size_t(Kp) + k0 + e];
   }
-  // phase G's lists (owned faces, their codes, 1/hK; export items)
+  // phase G's lists (owned faces, 1/hK; export items)
   const int nwc = HX ? a.g.wave_cnt[tile] : 0, nxc = HX ? a.g.xp_cnt[tile] : 0;
-  int gw = 0, gc = 0, gx = 0, gd = 0;
+  int gw = 0, gx = 0, gd = 0;
   double gok = 0.;
   if constexpr (HX) {
-    if (tid < a.Wmax) {
-      gw = a.g.wave_list[size_t(tile) * a.Wmax + tid];
-      gc = a.g.wave_code[size_t(tile) * a.Wmax + tid];
-    }
+    if (tid < a.Wmax) gw = a.g.wave_list[size_t(tile) * a.Wmax + tid];
     if (tid < a.Xmax) {
       gx = a.g.xp_list[size_t(tile) * a.Xmax + tid];
       gd = a.g.xp_dst[size_t(tile) * a.Xmax + tid];
     }
     if (tid < E) gok = a.g.oohK[k0 + tid];
   }
-  const int nbnd = a.g.bnd_cnt[tile];  // non-shared faces: the boundary loop runs only if any
+  // boundary faces: their loops run only if any
+  const int bnd0 = a.g.bnd_ptr[tile], nbnd = a.g.bnd_ptr[tile + 1] - bnd0;
   int hk0 = -1, hf0 = 0;
   if (!HX && tid < a.Hmax * 4) {
     const int h = tid % a.Hmax;
@@ -535,10 +541,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   }
   if (tid < a.Fmax) sFG[tid] = fgv;
   if constexpr (HX) {
-    if (tid < a.Wmax) {
-      sWP[tid] = gw;
-      sWC[tid] = gc;
-    }
+    if (tid < a.Wmax) sWP[tid] = gw;
     if (tid < a.Xmax) {
       sXP[tid] = gx;
       sXD[tid] = gd;
@@ -709,21 +712,21 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     }
   }
 #pragma unroll 1
-  for (int it = tid; it < (nbnd > 0 ? E * NF : 0); it += kThreads) {
-    const int e = it % E, p = it / E, f = p / NpEdge, pp = p - f * NpEdge;
-    const size_t fi = size_t(f) * Kp + k0 + e;
-    const int code = a.g.code[fi];
+  for (int it = tid; it < nbnd * NpEdge; it += kThreads) {
+    const int w = it / NpEdge, pp = it - w * NpEdge;
+    const int packed = a.g.bnd_item[2 * size_t(bnd0 + w)], code = a.g.bnd_item[2 * size_t(bnd0 + w) + 1];
+    const double *geo = a.g.bnd_geo + 4 * size_t(bnd0 + w);
+    const double nxd = geo[0], nyd = geo[1], wd = geo[2];
+    const int e = packed & 255, f = packed >> 8, p = f * NpEdge + pp;
     const int kind = code & 15;
-    if (kind == FK_Shared) continue;
     C own[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) own[c] = sT[c * TS + p * kTP + e];
-    const double nxd = a.g.Nx[fi], nyd = a.g.Ny[fi];
     const C nx = C(nxd), ny = C(nyd);
     C F[4] = {C(0), C(0), C(0), C(0)};
     if (kind == FK_Far || kind == FK_IVortex) {
       double qb[4];
-      boundary_state(kind, ph, a.g.bxy, code >> 8, NpEdge, pp, time, own, nxd, nyd, qb);
+      boundary_state<GEN>(kind, ph, a.g.bxy, code >> 8, NpEdge, pp, time, own, nxd, nyd, qb);
       const C q[4] = {C(qb[0]), C(qb[1]), C(qb[2]), C(qb[3])};
       C Fx[4], Fy[4];
       flux_xy(g, q, Fx, Fy);
@@ -750,9 +753,20 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
         }
       }
     }
-    const C w = C(a.g.IInII[fi]);
+    const C wn = C(wd);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) sT[c * TS + p * kTP + e] = F[c] * w;
+    for (int c = 0; c < 4; ++c) sT[c * TS + p * kTP + e] = F[c] * wn;
+  }
+  // padding elements (the case's last tile): zero flux, so that they keep
+  // their inert state
+  const int nreal = min(E, ci.k_end - k0);
+  if (nreal < E) {
+    for (int it = tid; it < E * NF; it += kThreads) {
+      const int e = it % E, p = it / E;
+      if (e >= nreal)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) sT[c * TS + p * kTP + e] = C(0);
+    }
   }
   __syncthreads();
 
@@ -937,7 +951,6 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     S *q3 = static_cast<S *>(a.q3) + base;
     S *q4 = static_cast<S *>(a.q4) + base;
     double *Rr = static_cast<double *>(a.R) + base;
-    const int nreal = min(E, ci.k_end - k0);
     if constexpr (MF) {
       // the lane's values: variable c at point MS::point(krow, j) of element
       // me; the divergence is rq, the stage input qv, which takes the new
@@ -1125,21 +1138,32 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
         const int w = it / NpEdge, pp = it - w * NpEdge;
         const int packed = sWP[w];
         const int e = packed & 255, f = packed >> 8, p = f * NpEdge + pp;
-        const int kk = k0 + e;
-        const size_t fi = size_t(f) * Kp + kk;
-        const int code = sWC[w];
-        const int kind = code & 15;
-        C own[4];
+        double q[4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) own[c] = sT[c * TS + p * kTP + e];
-        double q[4] = {double(own[0]), double(own[1]), double(own[2]), double(own[3])};
-        if (kind == FK_Far || kind == FK_IVortex)
-          boundary_state(kind, ph, a.g.bxy, code >> 8, NpEdge, pp, tnext, own, a.g.Nx[fi], a.g.Ny[fi], q);
+        for (int c = 0; c < 4; ++c) q[c] = double(sT[c * TS + p * kTP + e]);
         const double wsp = point_speed(ph.gamma, q, sOK[e]);
         if (!(wsp == wsp)) bad = 1;
         wl = fmax(wl, wsp);
         if (lts) atomicMax(&sWf[e * 3 + f], bits(wsp));
       }
+    }
+    // the faces with a boundary state: the speed of that state
+    const int nbs = a.g.bst_cnt[tile] * NpEdge;
+#pragma unroll 1
+    for (int it = tid; it < nbs; it += kThreads) {
+      const int w = it / NpEdge, pp = it - w * NpEdge;
+      const int packed = a.g.bnd_item[2 * size_t(bnd0 + w)], code = a.g.bnd_item[2 * size_t(bnd0 + w) + 1];
+      const double *geo = a.g.bnd_geo + 4 * size_t(bnd0 + w);
+      const int e = packed & 255, f = packed >> 8, p = f * NpEdge + pp;
+      C own[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) own[c] = sT[c * TS + p * kTP + e];
+      double q[4];
+      boundary_state<GEN>(code & 15, ph, a.g.bxy, code >> 8, NpEdge, pp, tnext, own, geo[0], geo[1], q);
+      const double wsp = point_speed(ph.gamma, q, geo[3]);
+      if (!(wsp == wsp)) bad = 1;
+      wl = fmax(wl, wsp);
+      if (lts) atomicMax(&sWf[e * 3 + f], bits(wsp));
     }
     V4 *hout = static_cast<V4 *>(a.ht) + size_t(l.hpar ^ 1) * a.ntiles * a.Fmax * NpEdge;
 #pragma unroll
@@ -1166,6 +1190,11 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
         const int e = packed & 255, f = packed >> 8;
         fw[size_t(f) * Kp + k0 + e] = from_bits(sWf[e * 3 + f]);
       }
+      for (int w = tid; w < a.g.bst_cnt[tile]; w += kThreads) {
+        const int packed = a.g.bnd_item[2 * size_t(bnd0 + w)];
+        const int e = packed & 255, f = packed >> 8;
+        fw[size_t(f) * Kp + k0 + e] = from_bits(sWf[e * 3 + f]);
+      }
     }
   }
   if (tid == 0) {
@@ -1187,8 +1216,8 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   }
 }
 
-template <int N, class S, class SIN, class C, int FLUX, bool LAST, bool SHOCK>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(StageWaves<S, LAST, SHOCK>::value)))
+template <int N, class S, class SIN, class C, int FLUX, bool LAST, bool SHOCK, bool GEN>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(StageWaves<N, S, FLUX, LAST, SHOCK, GEN>::value)))
 k_stage(StageArgs) {
   // The argument is read through a pointer into the kernel-argument segment
   // (the struct is the only explicit argument, at offset 0): each field is
@@ -1197,52 +1226,65 @@ k_stage(StageArgs) {
   const StageArgs &a = *(const StageArgs *)__builtin_amdgcn_kernarg_segment_ptr();
   const int tile = tile_of_block(a.xcd_tiles);
   if (tile >= a.ntiles) return;
-  stage_tile<N, S, SIN, C, FLUX, LAST, SHOCK>(a, launch_of(a), tile);
+  stage_tile<N, S, SIN, C, FLUX, LAST, SHOCK, GEN>(a, launch_of(a), tile);
 }
 
-// Wave speeds of the current state (start of a step sequence): one thread per
-// (element, face), traces straight from HBM; each face's maximum goes to its
-// case's control block (an atomic per face: this runs once per sequence) and,
-// for local time stepping, to the per-face speed buffer.
+// Wave speeds of the current state (start of a step sequence): a workgroup
+// per tile, thread (face, element), traces straight from HBM; one maximum per
+// tile goes to its case's control block (an atomic per face serialised on one
+// address: 110 to 330 us at 80,000 to 320,000 triangles), and each face's to
+// the per-face speed buffer of local time stepping.
+constexpr int kProThreads = 3 * kTile;
 template <int N, class S>
-__global__ void __launch_bounds__(256) k_prologue(StageArgs a) {
+__global__ void __launch_bounds__(kProThreads) k_prologue(StageArgs a) {
   using Sh = Shape<N>;
   constexpr int NpInt = Sh::NpInt, NpEdge = Sh::NpEdge, NV = Sh::NV;
-  const int it = blockIdx.x * blockDim.x + threadIdx.x;
-  const int kk = it / 3, f = it - 3 * kk;
-  if (kk >= a.Kp) return;
-  const int cs = a.tile_case[kk / kTile];
+  __shared__ double red[kProThreads / 64];
+  const int tile = blockIdx.x, f = threadIdx.x / kTile, kk = tile * kTile + int(threadIdx.x) % kTile;
+  const int cs = a.tile_case[tile];
   const CaseInfo &ci = a.cases[cs];
-  if (kk >= ci.k_end) return;
   Ctl *ctl = a.ctl + cs;
   const double *Itp = a.Interp64;
   const size_t fi = size_t(f) * a.Kp + kk;
   const int code = a.g.code[fi];
-  if (!(code & FC_WAVE)) return;
-  const S *q = static_cast<const S *>(a.qs) + size_t(kk) * NV;
+  const bool on = kk < ci.k_end && (code & FC_WAVE);
   double wl = 0.0;
   int bad = 0;
-  for (int pp = 0; pp < NpEdge; ++pp) {
-    const int p = f * NpEdge + pp;
-    double tr[4];
-    for (int n = 0; n < 4; ++n) {
-      double t = 0;
-      for (int i = 0; i < NpInt; ++i) t += Itp[p * NpInt + i] * double(q[n * NpInt + i]);
-      tr[n] = t;
+  if (on) {
+    const S *q = static_cast<const S *>(a.qs) + size_t(kk) * NV;
+    double u[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) u[i] = double(q[i]);
+    for (int pp = 0; pp < NpEdge; ++pp) {
+      const int p = f * NpEdge + pp;
+      double tr[4];
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        double t = 0;
+#pragma unroll
+        for (int i = 0; i < NpInt; ++i) t += Itp[p * NpInt + i] * u[n * NpInt + i];
+        tr[n] = t;
+      }
+      const int kind = code & 15;
+      if (kind == FK_Far || kind == FK_IVortex) {
+        const double own[4] = {tr[0], tr[1], tr[2], tr[3]};
+        boundary_state<true>(kind, ci.ph, a.g.bxy, code >> 8, NpEdge, pp, ctl->time[a.step_index & 1], own,
+                       a.g.Nx[fi], a.g.Ny[fi], tr);
+      }
+      const double w = point_speed(ci.ph.gamma, tr, a.g.oohK[kk]);
+      if (!(w == w)) bad = 1;
+      wl = fmax(wl, w);
     }
-    const int kind = code & 15;
-    if (kind == FK_Far || kind == FK_IVortex) {
-      const double own[4] = {tr[0], tr[1], tr[2], tr[3]};
-      boundary_state(kind, ci.ph, a.g.bxy, code >> 8, NpEdge, pp, ctl->time[a.step_index & 1], own,
-                     a.g.Nx[fi], a.g.Ny[fi], tr);
-    }
-    const double w = point_speed(ci.ph.gamma, tr, a.g.oohK[kk]);
-    if (!(w == w)) bad = 1;
-    wl = fmax(wl, w);
+    if (a.lts.on) a.lts.fw[size_t(a.par2) * 3 * a.Kp + fi] = wl;
   }
-  if (a.lts.on) a.lts.fw[size_t(a.par2) * 3 * a.Kp + fi] = wl;
-  atomic_max_bits(&ctl->wmax[a.ring], wl);
-  if (bad) atomicOr(&ctl->nan, 1);
+  wl = wave_max(wl);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = wl;
+  bad = __syncthreads_or(bad);
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kProThreads / 64; ++w) wl = fmax(wl, red[w]);
+    atomic_max_bits(&ctl->wmax[a.ring], wl);
+    if (bad) atomicOr(&ctl->nan, 1);
+  }
 }
 
 // Halo traces of a state set outside the step sequence (a restart, an RHS
@@ -1528,7 +1570,7 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
                        double(sTr[(2 * NF + p) * E + e]), double(sTr[(3 * NF + p) * E + e])};
         if (kind == FK_Far || kind == FK_IVortex) {
           const double own[4] = {q[0], q[1], q[2], q[3]};
-          boundary_state(kind, ci.ph, a.g.bxy, code >> 8, NpEdge, pp, time, own, a.g.Nx[fi], a.g.Ny[fi], q);
+          boundary_state<true>(kind, ci.ph, a.g.bxy, code >> 8, NpEdge, pp, time, own, a.g.Nx[fi], a.g.Ny[fi], q);
         }
         const double sp = point_speed(ci.ph.gamma, q, oohK);
         if (!(sp == sp)) bad = 1;
@@ -1690,42 +1732,48 @@ __global__ void __launch_bounds__(256) k_shock_grad_act(StageArgs a) {
 // ---- launchers ----
 
 template <int N>
-size_t lds_bytes_n(size_t csize, int Hmax, int Fmax, int WXmax, bool lts, bool mf) {
-  return lds_tile_bytes<N>(csize, Hmax, Fmax, WXmax, mf) + (lts ? lds_lts_bytes : 0);
+size_t lds_bytes_n(size_t csize, int Hmax, int Fmax, int WXints, bool lts, bool mf) {
+  return lds_tile_bytes<N>(csize, Hmax, Fmax, WXints, mf) + (lts ? lds_lts_bytes : 0);
 }
 
-template <int N, class S, class SIN, class C, int FLUX, bool LAST, bool SHOCK>
+template <int N, class S, class SIN, class C, int FLUX, bool LAST, bool SHOCK, bool GEN>
 hipError_t launch_stage_t(const StageArgs &a, hipStream_t s) {
   // one thread stages each list item into LDS
   if (a.Fmax > kThreads || (!SHOCK && (a.Wmax > kThreads || a.Xmax > kThreads))) return hipErrorInvalidValue;
-  const size_t lds = lds_bytes_n<N>(sizeof(C), SHOCK ? a.Hmax : 0, a.Fmax, SHOCK ? 0 : a.Wmax + a.Xmax,
+  const size_t lds = lds_bytes_n<N>(sizeof(C), SHOCK ? a.Hmax : 0, a.Fmax, SHOCK ? 0 : a.Wmax + 2 * a.Xmax,
                                     a.lts.on != 0, UseMfma<N, C, SHOCK>::value);
   static size_t attr_bytes = 0;  // dynamic LDS the kernel is currently allowed
   if (lds > 64 * 1024 && lds > attr_bytes) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_stage<N, S, SIN, C, FLUX, LAST, SHOCK>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_stage<N, S, SIN, C, FLUX, LAST, SHOCK, GEN>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     attr_bytes = lds;
   }
   const int q = (a.ntiles + 7) / 8;
-  hipLaunchKernelGGL((k_stage<N, S, SIN, C, FLUX, LAST, SHOCK>), dim3(8 * q), dim3(kThreads), lds, s, a);
+  hipLaunchKernelGGL((k_stage<N, S, SIN, C, FLUX, LAST, SHOCK, GEN>), dim3(8 * q), dim3(kThreads), lds, s, a);
   return hipGetLastError();
 }
 
-template <int N, class S, class C, int FLUX, bool SHOCK>
+template <int N, class S, class C, int FLUX, bool SHOCK, bool GEN>
 hipError_t launch_stage_l(const StageArgs &a, hipStream_t s) {
-  if (a.stage == 4) return launch_stage_t<N, S, S, C, FLUX, true, SHOCK>(a, s);
-  if (a.stage <= 0) return launch_stage_t<N, S, double, C, FLUX, false, SHOCK>(a, s);  // input q0
-  return launch_stage_t<N, S, S, C, FLUX, false, SHOCK>(a, s);
+  if (a.stage == 4) return launch_stage_t<N, S, S, C, FLUX, true, SHOCK, GEN>(a, s);
+  if (a.stage <= 0) return launch_stage_t<N, S, double, C, FLUX, false, SHOCK, GEN>(a, s);  // input q0
+  return launch_stage_t<N, S, S, C, FLUX, false, SHOCK, GEN>(a, s);
+}
+
+template <int N, class S, class C, int FLUX, bool SHOCK>
+hipError_t launch_stage_g(const StageArgs &a, hipStream_t s) {
+  if (a.gen) return launch_stage_l<N, S, C, FLUX, SHOCK, true>(a, s);
+  return launch_stage_l<N, S, C, FLUX, SHOCK, false>(a, s);
 }
 
 template <int N, class S, class C, bool SHOCK>
 hipError_t launch_stage_f(const StageArgs &a, hipStream_t s) {
   switch (a.ph.flux) {
-    case 0: return launch_stage_l<N, S, C, 0, SHOCK>(a, s);
-    case 1: return launch_stage_l<N, S, C, 1, SHOCK>(a, s);
-    case 2: return launch_stage_l<N, S, C, 2, SHOCK>(a, s);
-    case 3: return launch_stage_l<N, S, C, 3, SHOCK>(a, s);
+    case 0: return launch_stage_g<N, S, C, 0, SHOCK>(a, s);
+    case 1: return launch_stage_g<N, S, C, 1, SHOCK>(a, s);
+    case 2: return launch_stage_g<N, S, C, 2, SHOCK>(a, s);
+    case 3: return launch_stage_g<N, S, C, 3, SHOCK>(a, s);
   }
   return hipErrorInvalidValue;
 }
@@ -1749,10 +1797,8 @@ hipError_t launch_stage_n(int prec, int shock, const StageArgs &a, hipStream_t s
 
 template <int N>
 hipError_t launch_prologue_n(int prec, const StageArgs &a, hipStream_t s) {
-  const long items = long(a.Kp) * 3;
-  const int blocks = int((items + 255) / 256);
   (void)prec;  // the prologue reads q0, which is FP64 in every precision
-  hipLaunchKernelGGL((k_prologue<N, double>), dim3(blocks), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((k_prologue<N, double>), dim3(a.ntiles), dim3(kProThreads), 0, s, a);
   return hipGetLastError();
 }
 
@@ -1889,9 +1935,10 @@ namespace dev {
 template <int N, class S>
 using MultiC = typename std::conditional<(sizeof(S) == 8 || N <= 1), double, float>::type;
 
-// KIND 0: stage 0 (input q0), 1: stages 1-3, 2: stage 4
-template <class S, int FLUX, int KIND>
-__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(StageWaves<S, KIND == 2, false>::value)))
+// KIND 0: stage 0 (input q0), 1: stages 1-3, 2: stage 4. Two waves per SIMD:
+// the five orders' bodies in one kernel spill vector registers at three.
+template <class S, int FLUX, int KIND, bool GEN>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 k_stage_multi(MultiArgs m) {
   const int t = tile_of_block(m.xcd_tiles);
   if (t >= m.ntiles) return;
@@ -1905,15 +1952,15 @@ k_stage_multi(MultiArgs m) {
   using SIN = typename std::conditional<KIND == 0, double, S>::type;
   constexpr bool LAST = KIND == 2;
   switch (m.g[g].N) {
-    case 0: stage_tile<0, S, SIN, MultiC<0, S>, FLUX, LAST, false>(a, l, tile); break;
-    case 1: stage_tile<1, S, SIN, MultiC<1, S>, FLUX, LAST, false>(a, l, tile); break;
-    case 2: stage_tile<2, S, SIN, MultiC<2, S>, FLUX, LAST, false>(a, l, tile); break;
-    case 3: stage_tile<3, S, SIN, MultiC<3, S>, FLUX, LAST, false>(a, l, tile); break;
-    default: stage_tile<4, S, SIN, MultiC<4, S>, FLUX, LAST, false>(a, l, tile); break;
+    case 0: stage_tile<0, S, SIN, MultiC<0, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
+    case 1: stage_tile<1, S, SIN, MultiC<1, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
+    case 2: stage_tile<2, S, SIN, MultiC<2, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
+    case 3: stage_tile<3, S, SIN, MultiC<3, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
+    default: stage_tile<4, S, SIN, MultiC<4, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
   }
 }
 
-template <class S, int FLUX, int KIND>
+template <class S, int FLUX, int KIND, bool GEN>
 static hipError_t launch_multi_k(const MultiArgs &m, hipStream_t s) {
   size_t lds = 0;
   for (int g = 0; g < m.ngroups; ++g) {
@@ -1921,40 +1968,39 @@ static hipError_t launch_multi_k(const MultiArgs &m, hipStream_t s) {
     const size_t cs = sizeof(S) == 8 || G.N <= 1 ? sizeof(double) : sizeof(float);
     size_t b = 0;
     switch (G.N) {
-      case 0: b = lds_bytes_n<0>(cs, 0, G.Fmax, G.WXmax, G.lts != 0, false); break;
-      case 1: b = lds_bytes_n<1>(cs, 0, G.Fmax, G.WXmax, G.lts != 0, false); break;
-      case 2: b = lds_bytes_n<2>(cs, 0, G.Fmax, G.WXmax, G.lts != 0, false); break;
-      case 3: b = lds_bytes_n<3>(cs, 0, G.Fmax, G.WXmax, G.lts != 0, true); break;
-      default: b = lds_bytes_n<4>(cs, 0, G.Fmax, G.WXmax, G.lts != 0, true); break;
+      case 0: b = lds_bytes_n<0>(cs, 0, G.Fmax, G.WXints, G.lts != 0, false); break;
+      case 1: b = lds_bytes_n<1>(cs, 0, G.Fmax, G.WXints, G.lts != 0, false); break;
+      case 2: b = lds_bytes_n<2>(cs, 0, G.Fmax, G.WXints, G.lts != 0, false); break;
+      case 3: b = lds_bytes_n<3>(cs, 0, G.Fmax, G.WXints, G.lts != 0, true); break;
+      default: b = lds_bytes_n<4>(cs, 0, G.Fmax, G.WXints, G.lts != 0, true); break;
     }
     lds = std::max(lds, b);
   }
   static size_t attr_bytes = 0;  // dynamic LDS the kernel is currently allowed
   if (lds > 64 * 1024 && lds > attr_bytes) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_stage_multi<S, FLUX, KIND>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_stage_multi<S, FLUX, KIND, GEN>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     attr_bytes = lds;
   }
   const int q = (m.ntiles + 7) / 8;
-  hipLaunchKernelGGL((k_stage_multi<S, FLUX, KIND>), dim3(8 * q), dim3(kThreads), lds, s, m);
+  hipLaunchKernelGGL((k_stage_multi<S, FLUX, KIND, GEN>), dim3(8 * q), dim3(kThreads), lds, s, m);
   return hipGetLastError();
 }
 
 template <>
 hipError_t launch_stage_multi_f<GOCFD_MULTI_FLUX>(int prec, const MultiArgs &m, hipStream_t s) {
-  // FP64 only: the FP32 variant faulted the GPU in its first run and stays
-  // off until that is explained
+  // FP64 only: the FP32 variant (switched off) spilled vector registers,
+  // which this compiler can place wrongly; see StageWaves
   if (prec != 0) return hipErrorNotSupported;
   for (int g = 0; g < m.ngroups; ++g)
-    if (m.g[g].Fmax > kThreads || m.g[g].WXmax > 2 * kThreads) return hipErrorInvalidValue;
+    if (m.g[g].Fmax > kThreads || m.g[g].WXints > 3 * kThreads) return hipErrorInvalidValue;
   const int kind = m.l.stage == 0 ? 0 : m.l.stage == 4 ? 2 : 1;
-  if (prec == 0) {
-    if (kind == 0) return launch_multi_k<double, GOCFD_MULTI_FLUX, 0>(m, s);
-    if (kind == 2) return launch_multi_k<double, GOCFD_MULTI_FLUX, 2>(m, s);
-    return launch_multi_k<double, GOCFD_MULTI_FLUX, 1>(m, s);
-  }
-  return hipErrorNotSupported;
+  if (kind == 0)
+    return m.gen ? launch_multi_k<double, GOCFD_MULTI_FLUX, 0, true>(m, s) : launch_multi_k<double, GOCFD_MULTI_FLUX, 0, false>(m, s);
+  if (kind == 2)
+    return m.gen ? launch_multi_k<double, GOCFD_MULTI_FLUX, 2, true>(m, s) : launch_multi_k<double, GOCFD_MULTI_FLUX, 2, false>(m, s);
+  return m.gen ? launch_multi_k<double, GOCFD_MULTI_FLUX, 1, true>(m, s) : launch_multi_k<double, GOCFD_MULTI_FLUX, 1, false>(m, s);
 }
 
 template <>
