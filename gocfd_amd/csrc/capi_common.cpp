@@ -114,14 +114,14 @@ dev::Phys phys_of(const CaseStreams &fs, const gocfd_params &p) {
   return ph;
 }
 
-void fill_element_major(const DeviceLayout &L, int NpInt, const double *Q, double *h) {
+void fill_tiles(const DeviceLayout &L, int NpInt, const double *Q, double *h) {
   const double pad[4] = {1.0, 0.0, 0.0, 2.5};
   const int NV = 4 * NpInt, K = L.K;
   for (int kk = 0; kk < L.Kp; ++kk) {
     const int k = L.perm[kk];
     for (int n = 0; n < 4; ++n)
       for (int i = 0; i < NpInt; ++i)
-        h[size_t(kk) * NV + n * NpInt + i] = k < 0 ? pad[n] : Q[size_t(n) * NpInt * K + size_t(i) * K + k];
+        h[dev::state_at(kk, n * NpInt + i, NV)] = k < 0 ? pad[n] : Q[size_t(n) * NpInt * K + size_t(i) * K + k];
   }
 }
 

@@ -71,7 +71,7 @@ struct StageTypeBuf {
 };
 
 // Host states in the reference layout [4][NpInt][K] to and from the device's
-// element-major layout. The re-layout runs on the device: the host only
+// tile layout (or element-major, tiled = false). The re-layout runs on the device: the host only
 // copies, through a device staging array of the reference layout's size and,
 // for states up to kPin bytes, one pinned host buffer. (On the host the
 // strided re-layout took 14 ms into and 18 ms out of the device at 80,000
@@ -104,7 +104,7 @@ struct HostIo {
     }
   }
   // Q is free again on return; the re-layout may still run on the stream
-  void put(const double *Q, const int *perm, int K, int Kp, int NpInt, bool inert, double *dst, hipStream_t s) {
+  void put(const double *Q, const int *perm, int K, int Kp, int NpInt, bool tiled, bool inert, double *dst, hipStream_t s) {
     const size_t vals = size_t(K) * 4 * NpInt, bytes = vals * sizeof(double);
     reserve(vals);
     if (bytes <= kPin) {
@@ -114,13 +114,13 @@ struct HostIo {
       HIPCHECK(hipMemcpyAsync(stage.p, Q, bytes, hipMemcpyHostToDevice, s));
       HIPCHECK(hipStreamSynchronize(s));
     }
-    HIPCHECK(dev::launch_gather_state(stage.p, perm, K, Kp, NpInt, inert, dst, s));
+    HIPCHECK(dev::launch_gather_state(stage.p, perm, K, Kp, NpInt, tiled, inert, dst, s));
   }
   // Returns when Q is written
-  void get(const double *src, const int *perm, int K, int NpInt, double *Q, hipStream_t s) {
+  void get(const double *src, const int *perm, int K, int NpInt, bool tiled, double *Q, hipStream_t s) {
     const size_t vals = size_t(K) * 4 * NpInt, bytes = vals * sizeof(double);
     reserve(vals);
-    HIPCHECK(dev::launch_scatter_state(src, perm, K, NpInt, stage.p, s));
+    HIPCHECK(dev::launch_scatter_state(src, perm, K, NpInt, tiled, stage.p, s));
     HIPCHECK(hipMemcpyAsync(bytes <= kPin ? pin : Q, stage.p, bytes, hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
     if (bytes <= kPin) std::memcpy(Q, pin, bytes);
@@ -168,9 +168,9 @@ void check_device(int device, size_t lds_bytes);
 bool general_gamma(const dev::Phys &ph);  // a far-field state whose gamma is not 1.4
 dev::Phys phys_of(const CaseStreams &fs, const gocfd_params &p);
 
-// Element-major FP64 device layout of a reference-layout state, padding
-// elements set to the inert state (host side: an ensemble's initial states)
-void fill_element_major(const DeviceLayout &L, int NpInt, const double *Q, double *h);
+// Tile layout (dev::state_at) of a reference-layout state, padding elements
+// set to the inert state (host side: an ensemble's initial states)
+void fill_tiles(const DeviceLayout &L, int NpInt, const double *Q, double *h);
 
 }  // namespace capi
 }  // namespace gocfd

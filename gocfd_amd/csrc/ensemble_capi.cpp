@@ -114,7 +114,7 @@ struct EnsGroup {
   StageTypeBuf flux_geo;
   void *q[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   void *R = nullptr;
-  std::vector<double> q0_init;         // initial element-major state (tuning restores it)
+  std::vector<double> q0_init;         // initial state, tile layout (tuning restores it)
   // local time stepping
   DevBuf<double> fw, fwv, DTk, DTv;
   DevBuf<int> wsrc;
@@ -525,7 +525,7 @@ void build_group(gocfd_ensemble &h, EnsGroup &g) {
     }
     bnd_geo.insert(bnd_geo.end(), L.bnd_geo.begin(), L.bnd_geo.end());
     std::copy(L.perm.begin(), L.perm.end(), perm.begin() + o);
-    fill_element_major(L, NpInt, c.Q0.data(), q0.data() + o * g.NV);
+    fill_tiles(L, NpInt, c.Q0.data(), q0.data() + o * g.NV);
   }
   g.Jdet.upload(Jdet); g.Jinv.upload(Jinv); g.IInII.upload(IInII); g.Nx.upload(Nx); g.Ny.upload(Ny);
   g.oohK.upload(oohK); g.bxy.upload(bxy); g.code.upload(code); g.nbr_slot.upload(nbr_slot);
@@ -731,7 +731,7 @@ int gocfd_ensemble_get_state(gocfd_ensemble *h, int32_t c, double *Q) {
   HIPCHECK(hipSetDevice(h->device));
   const EnsCase &cs = *h->cases[c];
   const EnsGroup &g = *h->groups[cs.group];
-  h->io.get(static_cast<const double *>(g.q[0]) + size_t(cs.off) * g.NV, g.perm.p + cs.off, cs.L.K, cs.d.ops.NpInt, Q,
+  h->io.get(static_cast<const double *>(g.q[0]) + size_t(cs.off) * g.NV, g.perm.p + cs.off, cs.L.K, cs.d.ops.NpInt, true, Q,
             h->stream);
   return GOCFD_OK;
   GUARD_END

@@ -400,10 +400,10 @@ int gocfd_euler2d_vjp(gocfd_euler2d *h, int32_t nsteps, int32_t checkpoint_every
   DevBuf<double> &lamN = h->deriv[0], &lam0 = h->deriv[1];
   if (lamN.n < tot) lamN.alloc(tot);
   if (lam0.n < tot) lam0.alloc(tot);
-  h->to_device_zero_pad(dQn, lamN.p);
+  h->to_device_deriv(dQn, lamN.p);
   double far[4];
-  r.vjp(static_cast<const double *>(h->q[0]), t0, nsteps, checkpoint_every, lamN.p, lam0.p, far);
-  h->from_device(lam0.p, dQ0);
+  r.vjp(h->state_deriv(), t0, nsteps, checkpoint_every, lamN.p, lam0.p, far);
+  h->from_device_deriv(lam0.p, dQ0);
   if (dQinf) for (int c = 0; c < 4; ++c) dQinf[c] = far[c];
   return GOCFD_OK;
   GUARD_END
@@ -423,10 +423,10 @@ int gocfd_euler2d_jvp(gocfd_euler2d *h, int32_t nsteps, const double *dQ0, const
   DevBuf<double> &dq0 = h->deriv[0], &qn = h->deriv[1], &dqn = h->deriv[2];
   for (DevBuf<double> *b : {&dq0, &qn, &dqn})
     if (b->n < tot) b->alloc(tot);
-  h->to_device_zero_pad(dQ0, dq0.p);
-  r.jvp(static_cast<const double *>(h->q[0]), dq0.p, dQinf, t0, nsteps, qn.p, dqn.p);
-  if (Qn) h->from_device(qn.p, Qn);
-  h->from_device(dqn.p, dQn);
+  h->to_device_deriv(dQ0, dq0.p);
+  r.jvp(h->state_deriv(), dq0.p, dQinf, t0, nsteps, qn.p, dqn.p);
+  if (Qn) h->from_device_deriv(qn.p, Qn);
+  h->from_device_deriv(dqn.p, dQn);
   return GOCFD_OK;
   GUARD_END
 }

@@ -32,7 +32,7 @@ struct gocfd_euler2d {
   size_t ssize = 8;  // bytes per stored stage-state value (q1..q4); q0 and R are FP64
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  // state (element-major, Kp * NV values of the storage type)
+  // state (tile layout, dev::state_at: Kp * NV values of the storage type)
   void *q[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
   void *R = nullptr;
   void *scratch_in = nullptr;
@@ -41,7 +41,7 @@ struct gocfd_euler2d {
   DevBuf<int> code, nbr_slot, halo_elem, halo_face, wave_list, wave_cnt, flux_list, flux_cnt;
   DevBuf<int> bnd_ptr, bst_cnt, bnd_item;
   HostIo io;
-  DevBuf<double> deriv[3];  // states of a derivative call (kept for the next one)
+  DevBuf<double> deriv[3], q0_deriv;  // states of a derivative call, element-major (kept for the next one)
   DevBuf<int> perm;  // [Kp] device element -> reference element (-1: padding)
   StageTypeBuf flux_geo;
   // halo traces (without shock capturing): export lists and the two buffers
@@ -122,19 +122,25 @@ struct gocfd_euler2d {
     return a;
   }
 
-  // reference layout [4][NpInt][K] (double) <-> element-major FP64 device
-  // buffer (q0 and the RHS-evaluation input) on the handle's stream
+  // reference layout [4][NpInt][K] (double) <-> FP64 device buffer in the
+  // tile layout (q0 and the RHS-evaluation input) on the handle's stream
   void to_device(const double *Q, void *dst) {
-    io.put(Q, perm.p, L.K, L.Kp, d.ops.NpInt, true, static_cast<double *>(dst), stream);
+    io.put(Q, perm.p, L.K, L.Kp, d.ops.NpInt, true, true, static_cast<double *>(dst), stream);
   }
-  // reference-layout cotangent or tangent -> element-major device buffer,
-  // zero on the padding elements
-  void to_device_zero_pad(const double *Q, void *dst) {
-    io.put(Q, perm.p, L.K, L.Kp, d.ops.NpInt, false, static_cast<double *>(dst), stream);
-  }
-  // element-major FP64 device buffer -> reference layout; returns when Q is written
+  // returns when Q is written
   void from_device(const void *src, double *Q) {
-    io.get(static_cast<const double *>(src), perm.p, L.K, d.ops.NpInt, Q, stream);
+    io.get(static_cast<const double *>(src), perm.p, L.K, d.ops.NpInt, true, Q, stream);
+  }
+  // The derivative kernels' element-major buffers: a cotangent or tangent,
+  // zero on the padding elements; the way back; and the current state
+  void to_device_deriv(const double *Q, double *dst) {
+    io.put(Q, perm.p, L.K, L.Kp, d.ops.NpInt, false, false, dst, stream);
+  }
+  void from_device_deriv(const double *src, double *Q) { io.get(src, perm.p, L.K, d.ops.NpInt, false, Q, stream); }
+  const double *state_deriv() {
+    if (q0_deriv.n < size_t(L.Kp) * NV) q0_deriv.alloc(size_t(L.Kp) * NV);
+    HIPCHECK(dev::launch_element_major(static_cast<const double *>(q[0]), L.Kp, d.ops.NpInt, q0_deriv.p, stream));
+    return q0_deriv.p;
   }
 
   // The control block after the stream's work so far (through pinned memory:
@@ -196,7 +202,7 @@ struct gocfd_euler2d {
     }
   }
 
-  // Arguments of an RHS evaluation of the element-major FP64 state qs into
+  // Arguments of an RHS evaluation of the FP64 state qs (tile layout) into
   // out, with its halo traces in the buffer the next stage does not read
   // (the one the last stage read); on stream s
   dev::StageArgs rhs_args(const void *qs, double t, double *out, hipStream_t s) {

@@ -19,6 +19,12 @@ constexpr int kThreads = 4 * kTile; // threads per workgroup: one per (element, 
 // LDS banks (a 64-element pitch put them all on one)
 constexpr int kTP = kTile + 4;
 static_assert(kThreads % 64 == 0, "whole wavefronts per workgroup");
+// Place of value r = variable * NpInt + point of element kk in a state array:
+// tile after tile, within a tile [4 NpInt][kTile], so that the lanes of a
+// wave, which hold consecutive elements, touch consecutive values
+__host__ __device__ constexpr size_t state_at(int kk, int r, int NV) {
+  return (size_t(kk / kTile) * NV + r) * kTile + kk % kTile;
+}
 
 // Device control block. Time is double-buffered by step parity and the wave
 // speed maxima live in rings of three slots indexed by the global stage
@@ -134,9 +140,9 @@ struct StageArgs {
   // the neighbour's tile
   void *ht;
   double t_rhs;        // time for the RHS-only evaluation
-  void *qs;            // stage input state (element-major)
+  void *qs;            // stage input state (tile layout, state_at)
   void *q0, *q1, *q2, *q3, *q4, *R;
-  double *rhs_out;     // RHS-only output (element-major, double)
+  double *rhs_out;     // RHS-only output (tile layout, double)
   Ctl *ctl;            // control blocks, one per case
   const CaseInfo *cases;
   const int *tile_case;  // [ntiles] case of each tile
@@ -166,13 +172,17 @@ hipError_t launch_ctl_init(Ctl *ctl, double time, hipStream_t s, int ncases = 1)
 hipError_t launch_fill_u64(unsigned long long *p, size_t n, unsigned long long v, hipStream_t s);
 hipError_t launch_fill_f64(double *p, size_t n, double v, hipStream_t s);
 // A state in the reference layout [4][NpInt][K] (device memory) -> the
-// device's element-major layout; padding elements (perm = -1) take the inert
+// device's tile layout (state_at) or element-major [Kp][4 NpInt] (tiled =
+// false: the derivative kernels); padding elements (perm = -1) take the inert
 // state {1, 0, 0, 2.5}, or zero (cotangents and tangents). Every value of the
 // output is written.
-hipError_t launch_gather_state(const double *Q, const int *perm, int K, int Kp, int NpInt, bool inert, double *out,
-                               hipStream_t s);
-// The K real elements of an element-major state -> the reference layout
-hipError_t launch_scatter_state(const double *in, const int *perm, int K, int NpInt, double *Q, hipStream_t s);
+hipError_t launch_gather_state(const double *Q, const int *perm, int K, int Kp, int NpInt, bool tiled, bool inert,
+                               double *out, hipStream_t s);
+// The K real elements of a device state -> the reference layout
+hipError_t launch_scatter_state(const double *in, const int *perm, int K, int NpInt, bool tiled, double *Q,
+                                hipStream_t s);
+// A tile-layout state -> element-major
+hipError_t launch_element_major(const double *in, int Kp, int NpInt, double *out, hipStream_t s);
 // Copy the order-N operators (DivInt^T [NpFlux][NpInt], FluxEdgeInterp
 // [3NpEdge][NpInt]) into the current device's constant memory.
 hipError_t upload_operators(int N, const double *divT, const double *interp);

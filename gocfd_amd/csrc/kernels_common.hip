@@ -68,14 +68,13 @@ hipError_t upload_operators(int N, const double *divT, const double *interp) {
 #undef CALL
 }
 
-// Dynamic LDS of the stage kernel, at most: the tile state [NV][kTile+1],
-// the trace/flux buffer [4][3 NpEdge kTP + NpEdge Hmax] (the halo part
+// Dynamic LDS of the stage kernel, at most: the trace/flux buffer [4][3 NpEdge kTP + NpEdge Hmax] (the halo part
 // only with shock capturing), the Riemann items' geometry and the metric.
 size_t stage_lds_bytes(int N, int prec, int Hmax) {
   if (N < 0 || N > 4) return 0;
   const size_t cs = prec == 0 ? sizeof(double) : sizeof(float);
-  const size_t NpInt = size_t(N + 1) * (N + 2) / 2, NpEdge = size_t(N) + 2;
-  return (cs * (4 * NpInt * (kTile + 1) + 4 * (3 * NpEdge * kTP + NpEdge * size_t(Hmax))) + 31) / 32 * 32 +
+  const size_t NpEdge = size_t(N) + 2;
+  return (cs * 4 * (3 * NpEdge * kTP + NpEdge * size_t(Hmax)) + 31) / 32 * 32 +
          cs * (4 * 3 * kTile + 6 * kTile) +                                  // item geometry (Fmax <= 3 kTile), metric
          sizeof(double) * kTile + 2 * sizeof(int) * 6 * kTile +              // phase G lists (Wmax, Xmax <= 3 kTile)
          sizeof(double) * kTile + sizeof(unsigned long long) * 3 * kTile;  // with the LTS buffers
@@ -106,12 +105,27 @@ __global__ void k_fill_f64(double *p, size_t n, double v) {
     p[i] = v;
 }
 
+// Output index -> (element, value): in the tile layout neighbouring threads
+// take neighbouring elements of one value
+__device__ __forceinline__ void state_of(size_t idx, int NV, bool tiled, int &kk, int &r) {
+  if (tiled) {
+    const size_t row = idx / kTile, tile = row / NV;
+    r = int(row - tile * NV);
+    kk = int(tile) * kTile + int(idx % kTile);
+  } else {
+    kk = int(idx / NV);
+    r = int(idx - size_t(kk) * NV);
+  }
+}
+
 __global__ void __launch_bounds__(256) k_gather_state(const double *__restrict__ Q, const int *__restrict__ perm,
-                                                      int K, int Kp, int NpInt, int inert, double *__restrict__ out) {
+                                                      int K, int Kp, int NpInt, int tiled, int inert,
+                                                      double *__restrict__ out) {
   const int NV = 4 * NpInt;
   const size_t n = size_t(Kp) * NV;
   for (size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += size_t(gridDim.x) * blockDim.x) {
-    const int kk = int(idx / NV), r = int(idx - size_t(kk) * NV);
+    int kk, r;
+    state_of(idx, NV, tiled, kk, r);
     const int k = perm[kk];
     double v = 0.0;
     if (k >= 0) v = Q[size_t(r) * K + k];
@@ -121,26 +135,45 @@ __global__ void __launch_bounds__(256) k_gather_state(const double *__restrict__
 }
 
 __global__ void __launch_bounds__(256) k_scatter_state(const double *__restrict__ in, const int *__restrict__ perm,
-                                                       int K, int NpInt, double *__restrict__ Q) {
+                                                       int K, int Kp, int NpInt, int tiled, double *__restrict__ Q) {
   const int NV = 4 * NpInt;
-  const size_t n = size_t(K) * NV;
+  const size_t n = size_t(Kp) * NV;
+  for (size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += size_t(gridDim.x) * blockDim.x) {
+    int kk, r;
+    state_of(idx, NV, tiled, kk, r);
+    if (kk < K) Q[size_t(r) * K + perm[kk]] = in[idx];
+  }
+}
+
+__global__ void __launch_bounds__(256) k_element_major(const double *__restrict__ in, int Kp, int NpInt,
+                                                       double *__restrict__ out) {
+  const int NV = 4 * NpInt;
+  const size_t n = size_t(Kp) * NV;
   for (size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += size_t(gridDim.x) * blockDim.x) {
     const int kk = int(idx / NV), r = int(idx - size_t(kk) * NV);
-    Q[size_t(r) * K + perm[kk]] = in[idx];
+    out[idx] = in[state_at(kk, r, NV)];
   }
 }
 
 static int state_grid(size_t n) { return int(std::min<size_t>((n + 255) / 256, 8192)); }
 
-hipError_t launch_gather_state(const double *Q, const int *perm, int K, int Kp, int NpInt, bool inert, double *out,
-                               hipStream_t s) {
+hipError_t launch_gather_state(const double *Q, const int *perm, int K, int Kp, int NpInt, bool tiled, bool inert,
+                               double *out, hipStream_t s) {
   hipLaunchKernelGGL(k_gather_state, dim3(state_grid(size_t(Kp) * 4 * NpInt)), dim3(256), 0, s, Q, perm, K, Kp, NpInt,
-                     inert ? 1 : 0, out);
+                     tiled ? 1 : 0, inert ? 1 : 0, out);
   return hipGetLastError();
 }
 
-hipError_t launch_scatter_state(const double *in, const int *perm, int K, int NpInt, double *Q, hipStream_t s) {
-  hipLaunchKernelGGL(k_scatter_state, dim3(state_grid(size_t(K) * 4 * NpInt)), dim3(256), 0, s, in, perm, K, NpInt, Q);
+hipError_t launch_scatter_state(const double *in, const int *perm, int K, int NpInt, bool tiled, double *Q,
+                                hipStream_t s) {
+  const int Kp = (K + kTile - 1) / kTile * kTile;
+  hipLaunchKernelGGL(k_scatter_state, dim3(state_grid(size_t(Kp) * 4 * NpInt)), dim3(256), 0, s, in, perm, K, Kp, NpInt,
+                     tiled ? 1 : 0, Q);
+  return hipGetLastError();
+}
+
+hipError_t launch_element_major(const double *in, int Kp, int NpInt, double *out, hipStream_t s) {
+  hipLaunchKernelGGL(k_element_major, dim3(state_grid(size_t(Kp) * 4 * NpInt)), dim3(256), 0, s, in, Kp, NpInt, out);
   return hipGetLastError();
 }
 

@@ -1,7 +1,7 @@
 // RHS of a device-resident state without any device allocation
 // (gocfd_euler2d_rhs_noalloc, include/gocfd_euler2d.h), for callers that
 // cannot allocate: code under HIP graph capture, serving loops, harnesses
-// that forbid hipMalloc. The element-major staging of the input state and of
+// that forbid hipMalloc. The tile-layout staging of the input state and of
 // the RHS lives in one file-scope device array, `scratch`, of fixed size;
 // each device that loads the library holds its own copy until the process
 // ends, and every call on that device shares it.
@@ -64,14 +64,14 @@ extern "C" int gocfd_euler2d_rhs_noalloc(gocfd_euler2d *h, const double *Q, doub
   double *in = g_scratch[h->device], *out = in + vals;
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : h->stream;
   const int NpInt = h->d.ops.NpInt;
-  HIPCHECK(dev::launch_gather_state(Q, h->perm.p, h->L.K, h->L.Kp, NpInt, true, in, s));
+  HIPCHECK(dev::launch_gather_state(Q, h->perm.p, h->L.K, h->L.Kp, NpInt, true, true, in, s));
   dev::StageArgs a = h->rhs_args(in, t, out, s);
   h->launch_one_stage(a, s);
   if (h->shock) {  // the vertex buffers this evaluation used must be clear for the next stage
     HIPCHECK(dev::launch_fill_u64(h->sigV.p, h->sigV.n, 0ull, s));
     HIPCHECK(dev::launch_fill_u64(h->epsV.p, h->epsV.n, 0ull, s));
   }
-  HIPCHECK(dev::launch_scatter_state(out, h->perm.p, h->L.K, NpInt, RHS, s));
+  HIPCHECK(dev::launch_scatter_state(out, h->perm.p, h->L.K, NpInt, true, RHS, s));
   if (!stream) HIPCHECK(hipStreamSynchronize(s));
   return GOCFD_OK;
   GUARD_END

@@ -5,10 +5,11 @@
 // memory.
 //
 // One stage launch per Runge-Kutta stage. A workgroup owns a tile of kTile
-// consecutive elements (Hilbert order), whose element-major state is one
-// contiguous chunk of HBM. Per stage and tile:
-//   A. load the stage state (into LDS, or on the matrix-core path into the
-//      registers of the lanes that use it); face traces by the
+// consecutive elements (Hilbert order), whose state is one contiguous chunk of
+// HBM, the 64 elements' values of one variable and point side by side. Per
+// stage and tile:
+//   A. load the stage state into the registers of the lanes that use it;
+//      face traces by the
 //      FluxEdgeInterp contraction (model_problems/Euler2D/edges.go:485-491)
 //      for the tile's faces; the cross-tile neighbour traces from the
 //      halo-trace buffer, or with shock capturing interpolated from the
@@ -138,45 +139,26 @@ struct MfShape {
   }
 };
 
-// The lane's KI values of one variable of its element (matrix-core path);
-// row points at the variable's NpInt values in HBM. An FP32 lane holds four
-// consecutive points 4 krow + j: one vector access of the run starting at
-// min(4 krow, NpInt - 4) (points past NpInt repeat the last one on loads and
-// are not stored). FP64 lanes hold points krow + 4 j, one access each.
-template <class T>
-struct Run4 {
-  T v[4];
-};
+// The lane's KI values of one variable of its element (matrix-core path):
+// row points at the variable's first value of the element, consecutive points
+// lie kTile values apart. A wave's access to one point covers 16 consecutive
+// elements for each of four points: whole 128-byte lines in FP64. (With the
+// element's points contiguous instead, every lane touched a line of its own:
+// 17.7 million cache accesses per FP64 stage at order 4, 80,000 elements, and
+// 38 in the last one, 53 and 80 % of the cycles.) Points past NpInt repeat
+// the last one on loads and are not stored.
 template <int N, class C, class T>
 __device__ __forceinline__ void lane_load(const T *row, int krow, T (&out)[MfShape<N, C>::KI]) {
-  constexpr int NpInt = Shape<N>::NpInt, KI = MfShape<N, C>::KI;
-  if constexpr (sizeof(C) == 4) {
-    static_assert(KI == 4 && NpInt >= 4, "FP32 lanes hold four consecutive points");
-    const int o = min(4 * krow, NpInt - 4);
-    const Run4<T> r = *reinterpret_cast<const Run4<T> *>(row + o);
+  constexpr int NpInt = Shape<N>::NpInt;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = min(4 * krow + j, NpInt - 1) - o;
-      out[j] = d == 0 ? r.v[0] : d == 1 ? r.v[1] : d == 2 ? r.v[2] : r.v[3];
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < KI; ++j) out[j] = row[min(MfShape<N, C>::point(krow, j), NpInt - 1)];
-  }
+  for (int j = 0; j < MfShape<N, C>::KI; ++j) out[j] = row[min(MfShape<N, C>::point(krow, j), NpInt - 1) * kTile];
 }
 template <int N, class C, class T>
 __device__ __forceinline__ void lane_store(T *row, int krow, const T (&val)[MfShape<N, C>::KI]) {
-  constexpr int NpInt = Shape<N>::NpInt, KI = MfShape<N, C>::KI;
-  if constexpr (sizeof(C) == 4) {
-    if (4 * krow + 3 < NpInt) {
-      *reinterpret_cast<Run4<T> *>(row + 4 * krow) = Run4<T>{{val[0], val[1], val[2], val[3]}};
-      return;
-    }
-  }
 #pragma unroll
-  for (int j = 0; j < KI; ++j) {
+  for (int j = 0; j < MfShape<N, C>::KI; ++j) {
     const int i = MfShape<N, C>::point(krow, j);
-    if (i < NpInt) row[i] = val[j];
+    if (i < Shape<N>::NpInt) row[i * kTile] = val[j];
   }
 }
 
@@ -313,23 +295,22 @@ __device__ __forceinline__ double point_speed(double g, const double q[4], doubl
   return oohK * (U + c);
 }
 
-// Dynamic LDS of the stage kernel: the tile state [NV][kTile+1] (not on the
-// matrix-core path, whose state stays in registers) and the trace/flux
-// buffer [4][3 NpEdge kTP + NpEdge Hmax] (rows of kTP elements; rounded to
-// 32 bytes), the Riemann
+// Dynamic LDS of the stage kernel: the trace/flux buffer [4][3 NpEdge kTP +
+// NpEdge Hmax] (rows of kTP elements; rounded to 32 bytes; before the traces
+// it holds the tile state of the VALU path for the interior flux), the Riemann
 // items' geometry [Fmax][4] and the elements' metric terms [6][kTile];
 // without shock capturing, phase G's lists: the elements' 1/hK [kTile]
 // (FP64), the owned faces [Wmax] and the export items with their
 // destinations [2][Xmax] (ints; WXints = Wmax + 2 Xmax); local time stepping adds the
 // element dt and face-speed buffers.
 template <int N>
-__host__ __device__ constexpr size_t lds_trace_bytes(size_t csize, int Hmax, bool mf) {
-  return (csize * ((mf ? 0 : size_t(Shape<N>::NV) * (kTile + 1)) +
-                   4 * (size_t(Shape<N>::NF) * kTP + size_t(Shape<N>::NpEdge) * Hmax)) + 31) / 32 * 32;
+__host__ __device__ constexpr size_t lds_trace_bytes(size_t csize, int Hmax) {
+  static_assert(4 * Shape<N>::NF * kTP >= Shape<N>::NV * kTile, "the state fits the trace buffer");
+  return (csize * 4 * (size_t(Shape<N>::NF) * kTP + size_t(Shape<N>::NpEdge) * Hmax) + 31) / 32 * 32;
 }
 template <int N>
-__host__ __device__ constexpr size_t lds_tile_bytes(size_t csize, int Hmax, int Fmax, int WXints, bool mf) {
-  return lds_trace_bytes<N>(csize, Hmax, mf) + csize * (4 * size_t(Fmax) + 6 * kTile) +
+__host__ __device__ constexpr size_t lds_tile_bytes(size_t csize, int Hmax, int Fmax, int WXints) {
+  return lds_trace_bytes<N>(csize, Hmax) + csize * (4 * size_t(Fmax) + 6 * kTile) +
          (WXints > 0 ? (sizeof(double) * kTile + sizeof(int) * size_t(WXints) + 15) / 16 * 16 : 0);
 }
 constexpr size_t lds_lts_bytes = sizeof(double) * kTile + sizeof(unsigned long long) * 3 * kTile;
@@ -356,7 +337,10 @@ __device__ __forceinline__ bool step_skipped(const StageLaunch &l, const Ctl *ct
 
 // Waves per SIMD the register allocator targets. On the matrix-core path an
 // FP64 tile needs about 45 KB of LDS at N=4 (three workgroups per CU) and
-// fits 168 VGPRs; the FP32 stages fit 128 VGPRs without spilling.
+// fits 168 VGPRs; the FP32 stages fit 128 VGPRs without spilling. On the VALU
+// path the tile's state stays in its threads' registers: the order-2 FP64
+// stage fits 128 VGPRs and 27 KB of LDS, four workgroups per CU (with a state
+// buffer in LDS: 40 KB, three).
 #ifndef GOCFD_WAVES_F32
 #define GOCFD_WAVES_F32 4
 #endif
@@ -381,6 +365,52 @@ struct StageWaves {
                                                 : (N == 4 && (GEN || FLUX == 3) ? 2 : GOCFD_WAVES_F64);
 };
 
+// a x + b y with one rounding order, a x + round(b y), in every instantiation
+// (left to the compiler it depends on the surrounding blocks)
+template <class C>
+__device__ __forceinline__ C dot2(C a, C x, C b, C y) {
+#pragma clang fp contract(off)
+  const C t = b * y;
+  return fma(a, x, t);
+}
+
+// Stage 4 of SSP54 (euler.go:555-565): R = -q0 + a q2 + b q3 + c q4 + d dt R3 +
+// e dt RHS, on the VALU path with FP32 stage states. A last bit of q0 can
+// move the next rounding to an FP32 stage state by 6e-8, so the roundings of
+// the sum are pinned: the products with q2 and q3 are rounded for the last
+// three of every NpInt values of the tile in element order (split), fused for
+// the others.
+__device__ __forceinline__ double ssp_last_f32(bool split, double q0, double q2, double q3, double q4, double dtR3,
+                                               double dtR) {
+#pragma clang fp contract(off)
+  const double p2 = 0.517231671970585 * q2, p3 = 0.096059710526146 * q3;
+  double r = split ? (p2 - q0) + p3 : fma(0.096059710526146, q3, fma(0.517231671970585, q2, -q0));
+  r = fma(0.386708617503269, q4, r);
+  r = fma(0.063692468666290, dtR3, r);
+  return fma(0.226007483236906, dtR, r);
+}
+
+// Stages 0..3 on the VALU path (euler.go:511-545), roundings pinned for the
+// same reason: c dt RHS + (a q0 + round(b q_s))
+__device__ __forceinline__ double ssp_mid(int stage, double q0, double qs, double dtR) {
+#pragma clang fp contract(off)
+  switch (stage) {
+    case 0: return fma(0.391752226571890, dtR, qs);
+    case 1: return fma(0.368410593050371, dtR, fma(0.444370493651235, q0, 0.555629506348765 * qs));
+    case 2: return fma(0.251891774271694, dtR, fma(0.620101851488403, q0, 0.379898148511597 * qs));
+    default: return fma(0.544974750228521, dtR, fma(0.178079954393132, q0, 0.821920045606868 * qs));
+  }
+}
+
+// What bounds it and why this layout. With element-major tiles (an element's
+// 4 NpInt values contiguous) the order-2 stage staged its tile through LDS with
+// index arithmetic per value (VALU busy 55 %, three workgroups per CU) and the
+// matrix-core path's lanes each touched a line of their own. With the elements
+// side by side each thread or lane loads and stores its own values, whole lines
+// per wave, and the combination E is lane-local. Whole runs with their state
+// transfers, boundary lists included: order 2 FP64, 320,000 elements, 50 steps
+// 106 -> 33.7 ms; order 4, 80,000 elements, 100 steps in FP64 66.1 -> 32.9 ms,
+// in FP32 58.4 -> 25.6 ms.
 // S: storage of the stage states q1..q4; SIN: storage of this stage's
 // input (q0 at stage 0 and for the RHS evaluation, else S). q0 and the
 // stage-3 RHS R, which accumulate the step, are always FP64.
@@ -388,7 +418,7 @@ template <int N, class S, class SIN, class C, int FLUX, bool LAST, bool SHOCK, b
 __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch &l, const int tile) {
   using Sh = Shape<N>;
   constexpr int NpInt = Sh::NpInt, NpEdge = Sh::NpEdge, NF = Sh::NF, NV = Sh::NV, NR = Sh::NR;
-  constexpr int E = kTile, P = kTile + 1;
+  constexpr int E = kTile;
   static_assert(kThreads == 4 * kTile, "one thread per (element, variable)");
   extern __shared__ __align__(16) unsigned char smem_raw[];
   // Without shock capturing the traces of cross-tile neighbours come from
@@ -397,15 +427,16 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   // previous stage) each tile interpolates them from the neighbours' state
   // into a halo part of the trace buffer.
   constexpr bool HX = !SHOCK;
-  // Matrix-core path: the state stays in registers (no sQ, no sR)
+  // The state stays in registers: on the matrix-core path those of the lanes
+  // that hold its points in the MFMA layout, otherwise those of the thread of
+  // its (element, variable)
   constexpr bool MF = UseMfma<N, C, SHOCK>::value;
   using V4 = typename Vec4<C>::type;
-  C *sQ = reinterpret_cast<C *>(smem_raw);  // [NV][P] (VALU path)
   const int TS = NF * kTP + (HX ? 0 : NpEdge * a.Hmax);
-  C *sT = MF ? sQ : sQ + NV * P;             // [4][TS]: traces, then fluxes
-  C *sR = sT;                                // [NV][P]: RHS (aliases sT; VALU path)
+  C *sT = reinterpret_cast<C *>(smem_raw);  // [4][TS]: traces, then fluxes
+  C *sQ = sT;                               // [NV][E]: the tile state, before the traces (VALU path)
   // the Riemann items' geometry and the metric terms (Jdet, Jinv[4], -1/Jdet)
-  V4 *sFG = reinterpret_cast<V4 *>(smem_raw + lds_trace_bytes<N>(sizeof(C), HX ? 0 : a.Hmax, MF));  // [Fmax]
+  V4 *sFG = reinterpret_cast<V4 *>(smem_raw + lds_trace_bytes<N>(sizeof(C), HX ? 0 : a.Hmax));  // [Fmax]
   C *sJ = reinterpret_cast<C *>(sFG + a.Fmax);                                                 // [6][E]
   // phase G's lists (without shock capturing)
   double *sOK = reinterpret_cast<double *>(sJ + 6 * E);  // [E] 1/hK
@@ -414,7 +445,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   // local time stepping only: element dt and per-face speed maxima, after
   // the tile buffers (the launch adds their bytes only when LTS is on)
   double *sDT = reinterpret_cast<double *>(
-      smem_raw + lds_tile_bytes<N>(sizeof(C), HX ? 0 : a.Hmax, a.Fmax, HX ? a.Wmax + 2 * a.Xmax : 0, MF));
+      smem_raw + lds_tile_bytes<N>(sizeof(C), HX ? 0 : a.Hmax, a.Fmax, HX ? a.Wmax + 2 * a.Xmax : 0));
   unsigned long long *sWf = reinterpret_cast<unsigned long long *>(sDT + kTile);
   __shared__ double red[kThreads / 64];
 
@@ -468,46 +499,47 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     hf0 = a.g.halo_face[size_t(tile) * a.Hmax + h];
   }
 
-  // ---- A: tile state -> LDS (coalesced, contiguous chunk), or on the
-  // matrix-core path to the registers of the lanes that use it ----
-  // Every load is issued before the first LDS store, so a thread's LPT
-  // loads are in flight together.
-  constexpr int LPT = (E * NV + kThreads - 1) / kThreads;
+  // ---- A: tile state -> the registers of the lanes that use it ----
+  // Every load is issued before the first LDS store, so a thread's loads are
+  // in flight together; the tile's values [4 NpInt][E] put a wave's elements
+  // next to each other.
   using MS = MfShape<N, C>;
   constexpr int KI = MF ? MS::KI : 1;
   const int lane = tid & 63, krow = lane >> 4;
   const int me = (tid >> 6) * 16 + (lane & 15);  // element of the lane (matrix-core path)
-  SIN v[MF ? 1 : LPT];
+  const int te = tid % E, tn = tid / E;  // (element, variable) of this thread (VALU path)
+  const size_t tb = size_t(k0) * NV;     // the tile's values
+  const size_t vb = tb + size_t(tn * NpInt) * E + te;  // the thread's first (VALU path), the next E apart
+  constexpr int VP = MF ? 1 : NpInt;
+  C q[VP];      // VALU path: the thread's variable at its element's points
   C qv[4][KI];  // matrix-core path: the variables at points MS::point(krow, j)
   if constexpr (MF) {
     // a point past NpInt repeats the last one (a finite operand for the zero
     // columns of the A fragments)
-    const SIN *qe = qs + size_t(k0 + me) * NV;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       SIN r[KI];
-      lane_load<N, C>(qe + c * NpInt, krow, r);
+      lane_load<N, C>(qs + tb + size_t(c * NpInt) * E + me, krow, r);
 #pragma unroll
       for (int j = 0; j < KI; ++j) qv[c][j] = C(r[j]);
     }
   } else {
-    const SIN *qt = qs + size_t(k0) * NV;
 #pragma unroll
-    for (int j = 0; j < LPT; ++j) {
-      const int idx = tid + j * kThreads;
-      v[j] = (idx < E * NV) ? qt[idx] : S(0);
-    }
+    for (int i = 0; i < NpInt; ++i) q[i] = C(qs[vb + size_t(i) * E]);
   }
   // the neighbour traces of the cross-tile faces, under the state loads:
   // the cross-tile faces lead the flux list and their traces sit at the
   // tile's item slots, so these loads need nothing else loaded first (items
   // below Xmax that are not cross-tile read slots they never use)
-  V4 hx[HX ? ITB : 1];
+  // (the thread's first HXN items: 85 cross-tile faces at order 4, twice what
+  // a tile of a Hilbert-ordered mesh has; a tile with more loads the rest at
+  // their use, and the registers of three waves per SIMD suffice)
+  constexpr int HXN = ITB < 2 ? ITB : 2;
+  V4 hx[HX ? HXN : 1];
+  const V4 *hin = static_cast<const V4 *>(a.ht) + (size_t(l.hpar) * a.ntiles + tile) * a.Fmax * NpEdge;
   if constexpr (HX) {
-    const V4 *hin = static_cast<const V4 *>(a.ht) + size_t(l.hpar) * a.ntiles * a.Fmax * NpEdge +
-                    size_t(tile) * a.Fmax * NpEdge;
 #pragma unroll
-    for (int j = 0; j < ITB; ++j) {
+    for (int j = 0; j < HXN; ++j) {
       const int it = tid + j * kThreads;
       hx[j] = V4{C(0), C(0), C(0), C(0)};
       if (it < a.Xmax * NpEdge) hx[j] = hin[it];
@@ -531,13 +563,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   const C g = C(ph.gamma);
   if constexpr (!MF) {
 #pragma unroll
-    for (int j = 0; j < LPT; ++j) {
-      const int idx = tid + j * kThreads;
-      if (idx < E * NV) {
-        const int e = idx / NV, r = idx - e * NV;
-        sQ[r * P + e] = C(v[j]);
-      }
-    }
+    for (int i = 0; i < NpInt; ++i) sQ[(tn * NpInt + i) * E + te] = q[i];
   }
   if (tid < a.Fmax) sFG[tid] = fgv;
   if constexpr (HX) {
@@ -566,11 +592,36 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     if (l.stage == 4 && first && threadIdx.x == 0) ctl->time[par ^ 1] = time;
     return;
   }
-  const int te = tid % E, tn = tid / E;  // (element, variable) of this thread (VALU path)
+  // VALU path: the interior flux's part of the divergence (phase C) while
+  // the trace buffer holds the tile state, whose four variables it needs at
+  // each point; then the traces take its place. (A state buffer of its own
+  // would cost 12 KB at order 2 in FP64: three workgroups per CU, not four.)
+  C acc[VP];
+  bool act = false;  // shock capturing: eps*grad Q is nonzero somewhere in the element
   if constexpr (!MF) {
-    C q[NpInt];
+    const int kk = k0 + te;
+    if constexpr (SHOCK) act = a.sh.active[kk] != 0;
+    const C Jdc = sJ[te], J0 = sJ[E + te], J1 = sJ[2 * E + te], J2 = sJ[3 * E + te], J3 = sJ[4 * E + te];
 #pragma unroll
-    for (int i = 0; i < NpInt; ++i) q[i] = sQ[(tn * NpInt + i) * P + te];
+    for (int i = 0; i < NpInt; ++i) acc[i] = C(0);
+#pragma unroll 1
+    for (int j = 0; j < NpInt; ++j) {
+      const C r0 = sQ[(0 * NpInt + j) * E + te], r1 = sQ[(1 * NpInt + j) * E + te];
+      const C r2 = sQ[(2 * NpInt + j) * E + te], r3 = sQ[(3 * NpInt + j) * E + te];
+      C Fx, Fy;
+      flux_component(tn, g, r0, r1, r2, r3, Fx, Fy);
+      if constexpr (SHOCK) {
+        if (act) {
+          const C *dX = static_cast<const C *>(a.sh.diss) + size_t(tn * 2 * NR + j) * Kp + kk;
+          Fx -= dX[0];
+          Fy -= dX[size_t(NR) * Kp];
+        }
+      }
+      const C Fr = Jdc * dot2(J0, Fx, J1, Fy), Fs = Jdc * dot2(J2, Fx, J3, Fy);
+#pragma unroll
+      for (int i = 0; i < NpInt; ++i) acc[i] += DvT[j * NpInt + i] * Fr + DvT[(NpInt + j) * NpInt + i] * Fs;
+    }
+    __syncthreads();  // every thread has read the state
 #pragma unroll 2
     for (int p = 0; p < NF; ++p) {
       C t = C(0);
@@ -584,16 +635,16 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     const int kh = it == tid ? hk0 : a.g.halo_elem[size_t(tile) * a.Hmax + h];
     if (kh < 0) continue;
     const int f = it == tid ? hf0 : a.g.halo_face[size_t(tile) * a.Hmax + h];
-    const SIN *qn = qs + size_t(kh) * NV + n * NpInt;
-    C q[NpInt];
+    const SIN *qn = qs + state_at(kh, n * NpInt, NV);
+    C qh[NpInt];
 #pragma unroll
-    for (int i = 0; i < NpInt; ++i) q[i] = C(qn[i]);
+    for (int i = 0; i < NpInt; ++i) qh[i] = C(qn[i * E]);
 #pragma unroll
     for (int pp = 0; pp < NpEdge; ++pp) {
       const C *row = Itp + (f * NpEdge + pp) * NpInt;
       C t = C(0);
 #pragma unroll
-      for (int i = 0; i < NpInt; ++i) t += row[i] * q[i];
+      for (int i = 0; i < NpInt; ++i) t += row[i] * qh[i];
       sT[n * TS + NF * kTP + h * NpEdge + pp] = t;
     }
   }
@@ -610,7 +661,10 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   // the tile has been read; in FP64 until the thread's last item. Boundary
   // faces follow in a rolled loop: a boundary face point reads and writes
   // only its own LDS slot.
-  C fl[SHOCK || sizeof(C) == 8 ? ITB : 1][4];
+  // (the first three in FP64, the usual tile's all: more would not fit the
+  // registers of three waves per SIMD at order 4)
+  constexpr int HOLDN = SHOCK ? ITB : sizeof(C) == 8 ? (ITB < 3 ? ITB : 3) : 0;
+  C fl[HOLDN > 0 ? HOLDN : 1][4];
 #pragma unroll
   for (int j = 0; j < ITB; ++j) {
     const int it = tid + j * kThreads;
@@ -630,7 +684,15 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
       for (int c = 0; c < 4; ++c) {
         own[c] = sT[c * TS + p * kTP + e];
         oth[c] = sT[c * TS + idx];
-        if (xt) oth[c] = hx[j][c];
+      }
+      if (HX && j < HXN) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (xt) oth[c] = hx[HX ? (j < HXN ? j : 0) : 0][c];
+      } else if (xt) {
+        const V4 h = hin[it];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) oth[c] = h[c];
       }
       const C nx = gq[0], ny = gq[1];
       const bool owner = packed & (1 << 12);
@@ -664,7 +726,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
           }
         }
       }
-      if constexpr (!SHOCK && sizeof(C) == 4) {
+      if (j >= HOLDN) {
         // Without shock capturing each trace slot of the tile is read by
         // exactly one item (an in-tile pair by its owner item at point pp,
         // which reads and writes the partner's point NpEdge-1-pp; a
@@ -682,16 +744,15 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
         }
       } else {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) fl[j][c] = F[c];
+        for (int c = 0; c < 4; ++c) fl[j < HOLDN ? j : 0][c] = F[c];
       }
     }
   }
   // results held until every item of the thread is done (FP64), or until
   // every trace of the tile has been read (shock capturing: a barrier)
-  constexpr bool HOLD = SHOCK || sizeof(C) == 8;
   if constexpr (SHOCK) __syncthreads();
 #pragma unroll
-  for (int j = 0; j < (HOLD ? ITB : 0); ++j) {
+  for (int j = 0; j < HOLDN; ++j) {
     const int it = tid + j * kThreads;
     if (it < nfl) {
       const int w = it / NpEdge, pp = it - w * NpEdge;
@@ -776,9 +837,9 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   double q0p[PF ? 4 : 1][PF ? KI : 1];
   if constexpr (PF) {
     if (l.stage >= 1) {
-      const double *q0e = static_cast<const double *>(a.q0) + size_t(k0 + me) * NV;
+      const double *q0e = static_cast<const double *>(a.q0) + tb + me;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) lane_load<N, C>(q0e + c * NpInt, krow, q0p[c]);
+      for (int c = 0; c < 4; ++c) lane_load<N, C>(q0e + c * NpInt * E, krow, q0p[c]);
     }
   }
   // ---- C: interior flux + divergence ----
@@ -818,31 +879,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
 #pragma unroll
     for (int c = 0; c < 4; ++c) rq[c] = rq[c] * moojd;
   } else {
-    // VALU: thread (element te, variable tn)
-    const int kk = k0 + te;
-    bool act = false;  // shock capturing: eps*grad Q is nonzero somewhere in the element
-    if constexpr (SHOCK) act = a.sh.active[kk] != 0;
-    const C Jdc = sJ[te], J0 = sJ[E + te], J1 = sJ[2 * E + te], J2 = sJ[3 * E + te], J3 = sJ[4 * E + te];
-    C acc[NpInt];
-#pragma unroll
-    for (int i = 0; i < NpInt; ++i) acc[i] = C(0);
-#pragma unroll 1
-    for (int j = 0; j < NpInt; ++j) {
-      const C r0 = sQ[(0 * NpInt + j) * P + te], r1 = sQ[(1 * NpInt + j) * P + te];
-      const C r2 = sQ[(2 * NpInt + j) * P + te], r3 = sQ[(3 * NpInt + j) * P + te];
-      C Fx, Fy;
-      flux_component(tn, g, r0, r1, r2, r3, Fx, Fy);
-      if constexpr (SHOCK) {
-        if (act) {
-          const C *dX = static_cast<const C *>(a.sh.diss) + size_t(tn * 2 * NR + j) * Kp + kk;
-          Fx -= dX[0];
-          Fy -= dX[size_t(NR) * Kp];
-        }
-      }
-      const C Fr = Jdc * (J0 * Fx + J1 * Fy), Fs = Jdc * (J2 * Fx + J3 * Fy);
-#pragma unroll
-      for (int i = 0; i < NpInt; ++i) acc[i] += DvT[j * NpInt + i] * Fr + DvT[(NpInt + j) * NpInt + i] * Fs;
-    }
+    // VALU: thread (element te, variable tn); the face fluxes
 #pragma unroll 2
     for (int p = 0; p < NF; ++p) {
       const C Fe = sT[tn * TS + p * kTP + te];
@@ -855,7 +892,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     if constexpr (SHOCK) {
       // modal filter of the RHS (limitAndFilterSolution dissipation.go:606-622)
       ConstD *V = shock_ops_c(a.sh) + Sh::oV, *Vi = shock_ops_c(a.sh) + Sh::oVi, *mf = shock_ops_c(a.sh) + Sh::omf;
-      const double fac = 1. - sin(0.5 * M_PI * a.sh.sigma[kk]);
+      const double fac = 1. - sin(0.5 * M_PI * a.sh.sigma[k0 + te]);
       double m[NpInt];
 #pragma unroll
       for (int i = 0; i < NpInt; ++i) {
@@ -872,27 +909,21 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
         acc[i] = C(t);
       }
     }
-    __syncthreads();  // every thread has read its fluxes; sR may now overwrite sT
-#pragma unroll
-    for (int i = 0; i < NpInt; ++i) sR[(tn * NpInt + i) * P + te] = acc[i];
   }
-  if constexpr (!MF) __syncthreads();
 
   if (rhs_only) {
-    double *out = l.rhs_out + size_t(k0) * NV;
+    double *out = l.rhs_out + tb;
     if constexpr (MF) {
 #pragma unroll
       for (int j = 0; j < KI; ++j) {
         const int i = MS::point(krow, j);
         if (i < NpInt)
 #pragma unroll
-          for (int c = 0; c < 4; ++c) out[size_t(me) * NV + c * NpInt + i] = double(rq[c][j]);
+          for (int c = 0; c < 4; ++c) out[(c * NpInt + i) * E + me] = double(rq[c][j]);
       }
     } else {
-      for (int idx = tid; idx < E * NV; idx += kThreads) {
-        const int e = idx / NV, r = idx - e * NV;
-        out[idx] = double(sR[r * P + e]);
-      }
+#pragma unroll
+      for (int i = 0; i < NpInt; ++i) l.rhs_out[vb + size_t(i) * E] = double(acc[i]);
     }
     return;
   }
@@ -942,9 +973,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   }
   int bad = 0;
   {
-    // The operands of this stage are loaded for all LPT values of the
-    // thread first, then combined and stored.
-    const size_t base = size_t(k0) * NV;
+    const size_t base = MF ? tb + me : vb;
     double *q0 = static_cast<double *>(a.q0) + base;
     S *q1 = static_cast<S *>(a.q1) + base;
     S *q2 = static_cast<S *>(a.q2) + base;
@@ -955,7 +984,6 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
       // the lane's values: variable c at point MS::point(krow, j) of element
       // me; the divergence is rq, the stage input qv, which takes the new
       // state for phase F (a repeated point keeps its finite old value)
-      const size_t eb = size_t(me) * NV;
       const double dte = lts ? sDT[me] : dt;
       const bool real = me < nreal;
       if constexpr (LAST) {
@@ -963,10 +991,10 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
         for (int c = 0; c < 4; ++c) {
           double v0[KI], vR[KI];
           S v2[KI], v3[KI];
-          lane_load<N, C>(q0 + eb + c * NpInt, krow, v0);
-          lane_load<N, C>(q2 + eb + c * NpInt, krow, v2);
-          lane_load<N, C>(q3 + eb + c * NpInt, krow, v3);
-          lane_load<N, C>(Rr + eb + c * NpInt, krow, vR);
+          lane_load<N, C>(q0 + c * NpInt * E, krow, v0);
+          lane_load<N, C>(q2 + c * NpInt * E, krow, v2);
+          lane_load<N, C>(q3 + c * NpInt * E, krow, v3);
+          lane_load<N, C>(Rr + c * NpInt * E, krow, vR);
 #pragma unroll
           for (int j = 0; j < KI; ++j) {
             const double dtR = dte * double(rq[c][j]);
@@ -980,8 +1008,8 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
               if (real && !(v0[j] == v0[j])) bad = 1;
             }
           }
-          lane_store<N, C>(Rr + eb + c * NpInt, krow, vR);
-          lane_store<N, C>(q0 + eb + c * NpInt, krow, v0);
+          lane_store<N, C>(Rr + c * NpInt * E, krow, vR);
+          lane_store<N, C>(q0 + c * NpInt * E, krow, v0);
         }
       } else {
         double v0[4][KI];
@@ -992,7 +1020,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
             for (int j = 0; j < KI; ++j) v0[c][j] = q0p[c][j];  // loaded under phase C
         } else if (stage >= 1) {
 #pragma unroll
-          for (int c = 0; c < 4; ++c) lane_load<N, C>(q0 + eb + c * NpInt, krow, v0[c]);
+          for (int c = 0; c < 4; ++c) lane_load<N, C>(q0 + c * NpInt * E, krow, v0[c]);
         }
         S *qn = stage == 0 ? q1 : stage == 1 ? q2 : stage == 2 ? q3 : q4;
 #pragma unroll
@@ -1016,88 +1044,60 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
               if (real && !(nv[j] == nv[j])) bad = 1;
             }
           }
-          lane_store<N, C>(qn + eb + c * NpInt, krow, nv);
-          if (stage == 3) lane_store<N, C>(Rr + eb + c * NpInt, krow, rh);
+          lane_store<N, C>(qn + c * NpInt * E, krow, nv);
+          if (stage == 3) lane_store<N, C>(Rr + c * NpInt * E, krow, rh);
         }
-      }
-    } else if constexpr (LAST) {
-      // stage 4: R = -q0 + a q2 + b q3 + c q4 + d dt R3 + e dt RHS, q0 += R;
-      // with FP32 stage states the four operand arrays are loaded in two
-      // halves (the register budget of three waves per SIMD)
-      constexpr int CH = sizeof(S) == 4 ? (LPT + 1) / 2 : LPT;
-#pragma unroll
-      for (int j0 = 0; j0 < LPT; j0 += CH) {
-      double v0[CH], vR[CH];
-      S v2[CH], v3[CH];
-#pragma unroll
-      for (int jj = 0; jj < CH; ++jj) {
-        const int idx = tid + (j0 + jj) * kThreads;
-        const bool ok = j0 + jj < LPT && idx < E * NV;
-        v0[jj] = ok ? q0[idx] : 0.0;
-        v2[jj] = ok ? q2[idx] : S(0);
-        v3[jj] = ok ? q3[idx] : S(0);
-        vR[jj] = ok ? Rr[idx] : 0.0;
-      }
-#pragma unroll
-      for (int jj = 0; jj < CH; ++jj) {
-        const int j = j0 + jj;
-        const int idx = tid + j * kThreads;
-        if (j >= LPT) continue;
-        if (idx >= E * NV) continue;
-        const int e = idx / NV, r = idx - e * NV;
-        const double dte = lts ? sDT[e] : dt;
-        const double dtR = dte * double(sR[r * P + e]);
-        const double qsv = double(sQ[r * P + e]);
-        const double q0v = double(v0[jj]);
-        const double dtR3 = dte * double(vR[jj]);
-        const double Rn = -q0v + 0.517231671970585 * double(v2[jj]) + 0.096059710526146 * double(v3[jj]) +
-                          0.386708617503269 * qsv + 0.063692468666290 * dtR3 + 0.226007483236906 * dtR;
-        Rr[idx] = Rn;
-        const double nv = q0v + Rn;
-        q0[idx] = nv;
-        sQ[r * P + e] = C(nv);
-        if (e < nreal && !(nv == nv)) bad = 1;
-      }
       }
     } else {
-      double v0[LPT];
-      if (stage >= 1) {
+      // the thread's values: variable tn at the points of element te; the
+      // operands in chunks of CH points (the last stage has four arrays of
+      // them), each loaded before it is combined and stored
+      const double dte = lts ? sDT[te] : dt;
+      const bool real = te < nreal;
+      constexpr int CH = NpInt <= 6 ? NpInt : 5;
+      S *qn = stage == 0 ? q1 : stage == 1 ? q2 : stage == 2 ? q3 : q4;
 #pragma unroll
-        for (int j = 0; j < LPT; ++j) {
-          const int idx = tid + j * kThreads;
-          v0[j] = (idx < E * NV) ? q0[idx] : 0.0;
-        }
-      }
+      for (int i0 = 0; i0 < NpInt; i0 += CH) {
+        double v0[CH], vR[LAST ? CH : 1];
+        S v2[LAST ? CH : 1], v3[LAST ? CH : 1];
 #pragma unroll
-      for (int j = 0; j < LPT; ++j) {
-        const int idx = tid + j * kThreads;
-        if (idx >= E * NV) continue;
-        const int e = idx / NV, r = idx - e * NV;
-        const double rhs = double(sR[r * P + e]);
-        const double qsv = double(sQ[r * P + e]);
-        const double dtR = (lts ? sDT[e] : dt) * rhs;
-        S nv;
-        switch (stage) {
-          case 0:
-            nv = S(qsv + 0.391752226571890 * dtR);
-            q1[idx] = nv;
-            break;
-          case 1:
-            nv = S(0.444370493651235 * double(v0[j]) + 0.555629506348765 * qsv + 0.368410593050371 * dtR);
-            q2[idx] = nv;
-            break;
-          case 2:
-            nv = S(0.620101851488403 * double(v0[j]) + 0.379898148511597 * qsv + 0.251891774271694 * dtR);
-            q3[idx] = nv;
-            break;
-          default:
-            Rr[idx] = rhs;
-            nv = S(0.178079954393132 * double(v0[j]) + 0.821920045606868 * qsv + 0.544974750228521 * dtR);
-            q4[idx] = nv;
-            break;
+        for (int j = 0; j < CH; ++j) {
+          const int o = min(i0 + j, NpInt - 1) * E;
+          if (LAST || stage >= 1) v0[j] = q0[o];
+          if constexpr (LAST) {
+            v2[j] = q2[o];
+            v3[j] = q3[o];
+            vR[j] = Rr[o];
+          }
         }
-        sQ[r * P + e] = C(nv);
-        if (e < nreal && !(nv == nv)) bad = 1;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+          const int i = i0 + j;
+          if (i >= NpInt) continue;
+          const double rhs = double(acc[i]), qsv = double(q[i]), dtR = dte * rhs;
+          if constexpr (LAST) {
+            // R = -q0 + a q2 + b q3 + c q4 + d dt R3 + e dt RHS, q0 += R
+            const double dtR3 = dte * vR[j];
+            double Rn;
+            if constexpr (sizeof(S) == 4)
+              Rn = ssp_last_f32(te * NV + tn * NpInt + i >= (NpInt - 3) * kThreads, v0[j], double(v2[j]), double(v3[j]), qsv,
+                                dtR3, dtR);
+            else
+              Rn = -v0[j] + 0.517231671970585 * double(v2[j]) + 0.096059710526146 * double(v3[j]) +
+                   0.386708617503269 * qsv + 0.063692468666290 * dtR3 + 0.226007483236906 * dtR;
+            const double nv = v0[j] + Rn;
+            Rr[i * E] = Rn;
+            q0[i * E] = nv;
+            q[i] = C(nv);
+            if (real && !(nv == nv)) bad = 1;
+          } else {
+            const S nv = S(ssp_mid(stage, stage >= 1 ? v0[j] : 0.0, qsv, dtR));
+            if (stage == 3) Rr[i * E] = rhs;
+            qn[i * E] = nv;
+            q[i] = C(nv);
+            if (real && !(nv == nv)) bad = 1;
+          }
+        }
       }
     }
   }
@@ -1113,9 +1113,6 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     if constexpr (MF) {
       traces_mfma_regs<N, C>(qv, sT, lane, krow, me, TS);
     } else {
-      C q[NpInt];
-#pragma unroll
-      for (int i = 0; i < NpInt; ++i) q[i] = sQ[(tn * NpInt + i) * P + te];
 #pragma unroll 2
       for (int p = 0; p < NF; ++p) {
         C t = C(0);
@@ -1251,10 +1248,10 @@ __global__ void __launch_bounds__(kProThreads) k_prologue(StageArgs a) {
   double wl = 0.0;
   int bad = 0;
   if (on) {
-    const S *q = static_cast<const S *>(a.qs) + size_t(kk) * NV;
+    const S *q = static_cast<const S *>(a.qs) + state_at(kk, 0, NV);
     double u[NV];
 #pragma unroll
-    for (int i = 0; i < NV; ++i) u[i] = double(q[i]);
+    for (int i = 0; i < NV; ++i) u[i] = double(q[i * kTile]);
     for (int pp = 0; pp < NpEdge; ++pp) {
       const int p = f * NpEdge + pp;
       double tr[4];
@@ -1304,10 +1301,10 @@ __global__ void __launch_bounds__(256) k_halo_export(StageArgs a) {
   const int packed = a.g.xp_list[size_t(tile) * a.Xmax + w];
   const size_t dst = size_t(a.g.xp_dst[size_t(tile) * a.Xmax + w]);
   const int e = packed & 255, f = (packed >> 8) & 3;
-  const SIN *qn = static_cast<const SIN *>(a.qs) + size_t(tile * kTile + e) * NV + n * NpInt;
+  const SIN *qn = static_cast<const SIN *>(a.qs) + state_at(tile * kTile + e, n * NpInt, NV);
   C q[NpInt];
 #pragma unroll
-  for (int i = 0; i < NpInt; ++i) q[i] = C(qn[i]);
+  for (int i = 0; i < NpInt; ++i) q[i] = C(qn[i * kTile]);
   const C *Itp = Tabs<N, C>::ops() + Sh::NpFlux * NpInt;
   C *hout = static_cast<C *>(a.ht) + size_t(a.hpar) * a.ntiles * a.Fmax * NpEdge * 4;
 #pragma unroll
@@ -1347,10 +1344,10 @@ __global__ void __launch_bounds__(256) k_shock_sensor(StageArgs a) {
   if (kk >= a.Kp) return;
   // the element's density and size go out first, under the chain element ->
   // case -> control block of the skip check (kk < Kp keeps them in bounds)
-  const SIN *rho = static_cast<const SIN *>(a.qs) + size_t(kk) * NV;
+  const SIN *rho = static_cast<const SIN *>(a.qs) + state_at(kk, 0, NV);
   double r[NpInt];
 #pragma unroll
-  for (int i = 0; i < NpInt; ++i) r[i] = rho[i];
+  for (int i = 0; i < NpInt; ++i) r[i] = rho[i * kTile];
   const double hK = a.sh.hK[kk];
   // the element's case (a batch holds several, each with its own control)
   const int cs = a.tile_case[kk / kTile];
@@ -1453,11 +1450,11 @@ __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
   if (a.sh.filter_state) {
     ConstD *V = shock_ops_c(a.sh) + Sh::oV, *Vi = shock_ops_c(a.sh) + Sh::oVi, *mf = shock_ops_c(a.sh) + Sh::omf;
     const double fac = 1. - sin(0.5 * M_PI * sg);
-    SIN *q = static_cast<SIN *>(a.qs) + size_t(kk) * NV;
+    SIN *q = static_cast<SIN *>(a.qs) + state_at(kk, 0, NV);
     for (int n = 0; n < 4; ++n) {
       double u[NpInt], m[NpInt];
 #pragma unroll
-      for (int i = 0; i < NpInt; ++i) u[i] = q[n * NpInt + i];
+      for (int i = 0; i < NpInt; ++i) u[i] = q[(n * NpInt + i) * kTile];
 #pragma unroll
       for (int i = 0; i < NpInt; ++i) {
         double t = 0;
@@ -1470,7 +1467,7 @@ __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
         double t = 0;
 #pragma unroll
         for (int j = 0; j < NpInt; ++j) t += V[i * NpInt + j] * m[j];
-        q[n * NpInt + i] = SIN(t);
+        q[(n * NpInt + i) * kTile] = SIN(t);
       }
     }
   }
@@ -1478,16 +1475,13 @@ __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
 
 // Pass 2: the stage's owner-side wave speeds (|U|+c)/hK and viscous speeds
 // eps/hK^2 (StoreEdgeAggregates edges.go:246-289) from the own traces, one
-// tile of 64 elements x 4 variables per workgroup; the tile's state is
-// staged through LDS with coalesced loads.
+// tile of 64 elements x 4 variables per workgroup.
 template <int N, class SIN, class D>
 __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   using Sh = Shape<N>;
   constexpr int NpInt = Sh::NpInt, NpEdge = Sh::NpEdge, NpFlux = Sh::NpFlux, NF = Sh::NF, NV = Sh::NV,
-                E = kTile, P = kTile + 1;
-  // the tile state [NV][P], then (aliased) the traces [4][NF][E]
-  constexpr int LW = NV * P > 4 * NF * E ? NV * P : 4 * NF * E;
-  __shared__ D sbuf[LW];
+                E = kTile;
+  __shared__ D sTr[4 * NF * E];  // the traces [4][NF][E]
   __shared__ double red[2][kThreads / 64];
   const int tile = blockIdx.x, tid = threadIdx.x;
   const int te = tid % E, tn = tid / E, k0 = tile * E, Kp = a.Kp;
@@ -1497,16 +1491,9 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   // not depend on the control block (every tile lies inside the padded
   // range): their loads go out first, under the chain tile -> case ->
   // control block of the skip check.
-  constexpr int LPT = (E * NV + kThreads - 1) / kThreads;
-  SIN v[LPT];
-  {
-    const SIN *qt = Q + size_t(k0) * NV;
+  D u[NpInt];
 #pragma unroll
-    for (int j = 0; j < LPT; ++j) {
-      const int idx = tid + j * kThreads;
-      v[j] = idx < E * NV ? qt[idx] : SIN(0);
-    }
-  }
+  for (int i = 0; i < NpInt; ++i) u[i] = D(Q[size_t(k0) * NV + size_t(tn * NpInt + i) * E + te]);
   const int we = tid / 3, wf = tid - 3 * we;  // (element, face) of the wave-speed threads
   int wcode = 0;
   double woohK = 0.0;
@@ -1521,34 +1508,13 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   const CaseInfo &ci = a.cases[cs];
   Ctl *ctl = a.ctl + cs;
   if (a.stage < 0 || step_skipped(a, ctl, ci.ph.final_time)) return;
-  {
 #pragma unroll
-    for (int j = 0; j < LPT; ++j) {
-      const int idx = tid + j * kThreads;
-      if (idx < E * NV) {
-        const int e = idx / NV, r = idx - e * NV;
-        sbuf[r * P + e] = D(v[j]);
-      }
-    }
+  for (int p = 0; p < NF; ++p) {
+    D acc = 0;
+#pragma unroll
+    for (int j = 0; j < NpInt; ++j) acc += Itp[p * NpInt + j] * u[j];
+    sTr[(tn * NF + p) * E + te] = acc;
   }
-  __syncthreads();
-  D t[NF];
-  {
-    D u[NpInt];
-#pragma unroll
-    for (int i = 0; i < NpInt; ++i) u[i] = sbuf[(tn * NpInt + i) * P + te];
-#pragma unroll
-    for (int p = 0; p < NF; ++p) {
-      D acc = 0;
-#pragma unroll
-      for (int j = 0; j < NpInt; ++j) acc += Itp[p * NpInt + j] * u[j];
-      t[p] = acc;
-    }
-  }
-  __syncthreads();  // sbuf now holds the traces
-  D *sTr = sbuf;    // [4][NF][E]
-#pragma unroll
-  for (int p = 0; p < NF; ++p) sTr[(tn * NF + p) * E + te] = t[p];
   __syncthreads();
   // wave speeds of the owned faces: thread (element, face)
   double wl = 0.0, wv = 0.0;
@@ -1639,7 +1605,7 @@ __global__ void __launch_bounds__(256) k_shock_grad_act(StageArgs a) {
     const int kk = a.sh.act_list[it >> 3], tn = int(it >> 1) & 3, dir = int(it) & 1;
     D u[NpInt];
 #pragma unroll
-    for (int i = 0; i < NpInt; ++i) u[i] = D(Q[size_t(kk) * NV + tn * NpInt + i]);
+    for (int i = 0; i < NpInt; ++i) u[i] = D(Q[state_at(kk, tn * NpInt + i, NV)]);
     // edge values: the owner's trace at this face's points, in this face's
     // order. The three faces' neighbour entries, then the three source
     // states (the element's own where it owns the face, so every address is
@@ -1656,13 +1622,13 @@ __global__ void __launch_bounds__(256) k_shock_grad_act(StageArgs a) {
       nbf[f] = a.sh.nbr_face[fi];
       // unshared faces (boundary, padding) are always their own edge's owner
       own[f] = (code & FC_FLUX_OWNER) || (code & 15) != FK_Shared;
-      qsrc[f] = Q + size_t(own[f] ? kk : nb) * NV + tn * NpInt;
+      qsrc[f] = Q + state_at(own[f] ? kk : nb, tn * NpInt, NV);
     }
     D un[3][NpInt];
 #pragma unroll
     for (int f = 0; f < 3; ++f)
 #pragma unroll
-      for (int j = 0; j < NpInt; ++j) un[f][j] = D(qsrc[f][j]);
+      for (int j = 0; j < NpInt; ++j) un[f][j] = D(qsrc[f][j * kTile]);
     D ue[NF];
 #pragma unroll
     for (int f = 0; f < 3; ++f) {
@@ -1732,8 +1698,8 @@ __global__ void __launch_bounds__(256) k_shock_grad_act(StageArgs a) {
 // ---- launchers ----
 
 template <int N>
-size_t lds_bytes_n(size_t csize, int Hmax, int Fmax, int WXints, bool lts, bool mf) {
-  return lds_tile_bytes<N>(csize, Hmax, Fmax, WXints, mf) + (lts ? lds_lts_bytes : 0);
+size_t lds_bytes_n(size_t csize, int Hmax, int Fmax, int WXints, bool lts) {
+  return lds_tile_bytes<N>(csize, Hmax, Fmax, WXints) + (lts ? lds_lts_bytes : 0);
 }
 
 template <int N, class S, class SIN, class C, int FLUX, bool LAST, bool SHOCK, bool GEN>
@@ -1741,7 +1707,7 @@ hipError_t launch_stage_t(const StageArgs &a, hipStream_t s) {
   // one thread stages each list item into LDS
   if (a.Fmax > kThreads || (!SHOCK && (a.Wmax > kThreads || a.Xmax > kThreads))) return hipErrorInvalidValue;
   const size_t lds = lds_bytes_n<N>(sizeof(C), SHOCK ? a.Hmax : 0, a.Fmax, SHOCK ? 0 : a.Wmax + 2 * a.Xmax,
-                                    a.lts.on != 0, UseMfma<N, C, SHOCK>::value);
+                                    a.lts.on != 0);
   static size_t attr_bytes = 0;  // dynamic LDS the kernel is currently allowed
   if (lds > 64 * 1024 && lds > attr_bytes) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_stage<N, S, SIN, C, FLUX, LAST, SHOCK, GEN>),
@@ -1968,11 +1934,11 @@ static hipError_t launch_multi_k(const MultiArgs &m, hipStream_t s) {
     const size_t cs = sizeof(S) == 8 || G.N <= 1 ? sizeof(double) : sizeof(float);
     size_t b = 0;
     switch (G.N) {
-      case 0: b = lds_bytes_n<0>(cs, 0, G.Fmax, G.WXints, G.lts != 0, false); break;
-      case 1: b = lds_bytes_n<1>(cs, 0, G.Fmax, G.WXints, G.lts != 0, false); break;
-      case 2: b = lds_bytes_n<2>(cs, 0, G.Fmax, G.WXints, G.lts != 0, false); break;
-      case 3: b = lds_bytes_n<3>(cs, 0, G.Fmax, G.WXints, G.lts != 0, true); break;
-      default: b = lds_bytes_n<4>(cs, 0, G.Fmax, G.WXints, G.lts != 0, true); break;
+      case 0: b = lds_bytes_n<0>(cs, 0, G.Fmax, G.WXints, G.lts != 0); break;
+      case 1: b = lds_bytes_n<1>(cs, 0, G.Fmax, G.WXints, G.lts != 0); break;
+      case 2: b = lds_bytes_n<2>(cs, 0, G.Fmax, G.WXints, G.lts != 0); break;
+      case 3: b = lds_bytes_n<3>(cs, 0, G.Fmax, G.WXints, G.lts != 0); break;
+      default: b = lds_bytes_n<4>(cs, 0, G.Fmax, G.WXints, G.lts != 0); break;
     }
     lds = std::max(lds, b);
   }

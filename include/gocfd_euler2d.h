@@ -112,8 +112,8 @@ int gocfd_euler2d_rhs(gocfd_euler2d *h, const double *Q, double t, double *RHS);
  *      bit. Q and RHS are DEVICE pointers on the handle's device, in the
  *      reference layout [4][NpInt][K]. stream: a hipStream_t to enqueue on
  *      (the call then returns without waiting), or NULL for the handle's own
- *      stream (the call returns when the RHS is written). The element-major
- *      staging lives in a fixed 32 MiB device array per device: meshes with
+ *      stream (the call returns when the RHS is written). The staging in the
+ *      device's layout lives in a fixed 32 MiB device array per device: meshes with
  *      2 * Kp * 4 * NpInt * 8 bytes above that (Kp = K rounded up to the
  *      64-element tile; about K > 34,900 at N=4) get GOCFD_ERR_ARG. Every
  *      handle on a device shares that array: calls that overlap on one
