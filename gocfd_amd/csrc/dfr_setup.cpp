@@ -853,12 +853,14 @@ DeviceLayout build_device_layout(const Discretisation &d, int E, int TP) {
   }
   // Shared faces with Riemann work, per tile
   // (cross-tile faces first: item i of tile t receives its neighbour traces
-  // in halo-trace slot t * Fmax + i, written by the neighbour's tile)
+  // in halo-trace slot t * Fmax + i, written by the neighbour's tile; those
+  // this tile does not own lead, so that the lanes of a wave evaluate the same
+  // side)
   std::vector<int> item_of(size_t(3) * Kp, -1);  // flux-list item of each cross-tile face
   {
     std::vector<std::vector<int>> fl(L.ntiles);
     std::vector<std::vector<std::array<double, 4>>> fg(L.ntiles);
-    for (int pass = 0; pass < 2; ++pass)
+    for (int pass = 0; pass < 3; ++pass)
     for (int kk = 0; kk < K; ++kk)
       for (int f = 0; f < 3; ++f) {
         const size_t fi = size_t(f) * Kp + kk;
@@ -867,7 +869,7 @@ DeviceLayout build_device_layout(const Discretisation &d, int E, int TP) {
         const bool in_tile = !(uint32_t(L.nbr_slot[fi]) >> 31);
         const bool owner = code & FC_FLUX_OWNER;
         if (in_tile && !owner) continue;  // the in-tile owner fills this slot
-        if (in_tile != (pass == 1)) continue;
+        if (pass != (in_tile ? 2 : owner ? 1 : 0)) continue;
         if (!in_tile) item_of[fi] = int(fl[kk / E].size());
         const int base = int(uint32_t(L.nbr_slot[fi]) & 0x7fffffffu);
         if (base >= (1 << 18)) throw SetupError(GOCFD_ERR_MESH, "tile halo too large for the flux-list encoding");

@@ -50,16 +50,18 @@ __device__ __forceinline__ void flux_xy(C g, const C q[4], C Fx[4], C Fy[4]) {
   Fy[0] = q[2]; Fy[1] = q[2] * u; Fy[2] = q[2] * v + p; Fy[3] = v * (q[3] + p);
 }
 
-// One component n of the physical flux (n is wave-uniform in the kernels)
+// One component n of the physical flux (n is wave-uniform in the kernels).
+// The roundings are pinned: left to the compiler they follow the blocks around.
 template <class C>
 __device__ __forceinline__ void flux_component(int n, C g, C rho, C rhoU, C rhoV, C E, C &Fx, C &Fy) {
+#pragma clang fp contract(off)
   const C oorho = fdiv(C(1), rho);
-  const C u = rhoU * oorho, v = rhoV * oorho;
-  const C p = (g - C(1)) * (E - C(0.5) * rho * (u * u + v * v));
+  const C u = rhoU * oorho, v = rhoV * oorho, vv = v * v;
+  const C p = (g - C(1)) * fma(C(-0.5) * rho, fma(u, u, vv), E);
   switch (n) {
     case 0: Fx = rhoU; Fy = rhoV; break;
-    case 1: Fx = rhoU * u + p; Fy = rhoV * u; break;
-    case 2: Fx = rhoU * v; Fy = rhoV * v + p; break;
+    case 1: Fx = fma(rhoU, u, p); Fy = rhoV * u; break;
+    case 2: Fx = rhoU * v; Fy = fma(rhoV, v, p); break;
     default: Fx = u * (E + p); Fy = v * (E + p); break;
   }
 }

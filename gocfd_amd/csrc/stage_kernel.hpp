@@ -357,11 +357,11 @@ __device__ __forceinline__ bool step_skipped(const StageLaunch &l, const Ctl *ct
 // Riemann item) store nothing and reload garbage -- addresses among it. The
 // build's spill counts are checked by a test. GEN (a gamma other than 1.4)
 // needs the registers of pow, so it takes one wave per SIMD less; so does
-// Roe-ER at order 4 in FP64.
+// Roe-ER at order 4 in FP64. Up to order 1 the FP32 form computes in FP64.
 template <int N, class S, int FLUX, bool LAST, bool SHOCK, bool GEN>
 struct StageWaves {
   static constexpr int value = SHOCK            ? 1
-                               : sizeof(S) == 4 ? (LAST || GEN ? GOCFD_WAVES_F32_LAST : GOCFD_WAVES_F32)
+                               : sizeof(S) == 4 && N >= 2 ? (LAST || GEN ? GOCFD_WAVES_F32_LAST : GOCFD_WAVES_F32)
                                                 : (N == 4 && (GEN || FLUX == 3) ? 2 : GOCFD_WAVES_F64);
 };
 
@@ -390,16 +390,23 @@ __device__ __forceinline__ double ssp_last_f32(bool split, double q0, double q2,
   return fma(0.226007483236906, dtR, r);
 }
 
-// Stages 0..3 on the VALU path (euler.go:511-545), roundings pinned for the
-// same reason: c dt RHS + (a q0 + round(b q_s))
-__device__ __forceinline__ double ssp_mid(int stage, double q0, double qs, double dtR) {
-#pragma clang fp contract(off)
+// Stages 0..3 (euler.go:511-545): c dt RHS + (a q0 + round(b q_s)), roundings
+// pinned for the same reason. The coefficients are chosen once per stage: a
+// branch on the stage at every value cost as many instructions as the sum.
+struct SspCoef {
+  double a, b, c;
+};
+__device__ __forceinline__ SspCoef ssp_coef(int stage) {
   switch (stage) {
-    case 0: return fma(0.391752226571890, dtR, qs);
-    case 1: return fma(0.368410593050371, dtR, fma(0.444370493651235, q0, 0.555629506348765 * qs));
-    case 2: return fma(0.251891774271694, dtR, fma(0.620101851488403, q0, 0.379898148511597 * qs));
-    default: return fma(0.544974750228521, dtR, fma(0.178079954393132, q0, 0.821920045606868 * qs));
+    case 0: return {0.0, 1.0, 0.391752226571890};
+    case 1: return {0.444370493651235, 0.555629506348765, 0.368410593050371};
+    case 2: return {0.620101851488403, 0.379898148511597, 0.251891774271694};
+    default: return {0.178079954393132, 0.821920045606868, 0.544974750228521};
   }
+}
+__device__ __forceinline__ double ssp_mid(const SspCoef &k, double q0, double qs, double dtR) {
+#pragma clang fp contract(off)
+  return fma(k.c, dtR, fma(k.a, q0, k.b * qs));
 }
 
 // What bounds it and why this layout. With element-major tiles (an element's
@@ -411,6 +418,14 @@ __device__ __forceinline__ double ssp_mid(int stage, double q0, double qs, doubl
 // transfers, boundary lists included: order 2 FP64, 320,000 elements, 50 steps
 // 106 -> 33.7 ms; order 4, 80,000 elements, 100 steps in FP64 66.1 -> 32.9 ms,
 // in FP32 58.4 -> 25.6 ms.
+// What is left is latency and instructions: a tile's phases are chains of
+// loads and FP64 arithmetic with barriers between, 10 us for a tile alone.
+// Phase E's operands are therefore loaded under phase C, face points are taken
+// four at a time, the stage's coefficients are chosen once, and one Riemann
+// evaluation serves owners and others. Stage (FP64 unless said) before -> after
+// these: order 1, 3,034 elements 12.8 -> 12.0 us; order 2, 320,000 elements
+// 96.3 -> 90.6; order 4, 80,000 elements 55.3 -> 50.7, FP32 38.2 -> 37.3;
+// shock capturing at order 2, 249,386 elements 98.3 -> 85.4.
 // S: storage of the stage states q1..q4; SIN: storage of this stage's
 // input (q0 at stage 0 and for the RHS evaluation, else S). q0 and the
 // stage-3 RHS R, which accumulate the step, are always FP64.
@@ -492,6 +507,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   }
   // boundary faces: their loops run only if any
   const int bnd0 = a.g.bnd_ptr[tile], nbnd = a.g.bnd_ptr[tile + 1] - bnd0;
+  const int nbst = SHOCK ? 0 : a.g.bst_cnt[tile];
   int hk0 = -1, hf0 = 0;
   if (!HX && tid < a.Hmax * 4) {
     const int h = tid % a.Hmax;
@@ -507,10 +523,12 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   constexpr int KI = MF ? MS::KI : 1;
   const int lane = tid & 63, krow = lane >> 4;
   const int me = (tid >> 6) * 16 + (lane & 15);  // element of the lane (matrix-core path)
-  const int te = tid % E, tn = tid / E;  // (element, variable) of this thread (VALU path)
+  // (element, variable) of this thread (VALU path); a wave has one variable
+  const int te = tid % E, tn = __builtin_amdgcn_readfirstlane(tid / E);
   const size_t tb = size_t(k0) * NV;     // the tile's values
   const size_t vb = tb + size_t(tn * NpInt) * E + te;  // the thread's first (VALU path), the next E apart
   constexpr int VP = MF ? 1 : NpInt;
+  constexpr int UT = NpInt <= 6 ? 4 : 2;  // face points unrolled together (VALU path)
   C q[VP];      // VALU path: the thread's variable at its element's points
   C qv[4][KI];  // matrix-core path: the variables at points MS::point(krow, j)
   if constexpr (MF) {
@@ -601,10 +619,11 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   if constexpr (!MF) {
     const int kk = k0 + te;
     if constexpr (SHOCK) act = a.sh.active[kk] != 0;
+    constexpr int UJ = NpInt <= 3 ? NpInt : 2;
     const C Jdc = sJ[te], J0 = sJ[E + te], J1 = sJ[2 * E + te], J2 = sJ[3 * E + te], J3 = sJ[4 * E + te];
 #pragma unroll
     for (int i = 0; i < NpInt; ++i) acc[i] = C(0);
-#pragma unroll 1
+#pragma unroll UJ
     for (int j = 0; j < NpInt; ++j) {
       const C r0 = sQ[(0 * NpInt + j) * E + te], r1 = sQ[(1 * NpInt + j) * E + te];
       const C r2 = sQ[(2 * NpInt + j) * E + te], r3 = sQ[(3 * NpInt + j) * E + te];
@@ -619,10 +638,10 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
       }
       const C Fr = Jdc * dot2(J0, Fx, J1, Fy), Fs = Jdc * dot2(J2, Fx, J3, Fy);
 #pragma unroll
-      for (int i = 0; i < NpInt; ++i) acc[i] += DvT[j * NpInt + i] * Fr + DvT[(NpInt + j) * NpInt + i] * Fs;
+      for (int i = 0; i < NpInt; ++i) acc[i] += dot2(DvT[j * NpInt + i], Fr, DvT[(NpInt + j) * NpInt + i], Fs);
     }
     __syncthreads();  // every thread has read the state
-#pragma unroll 2
+#pragma unroll UT
     for (int p = 0; p < NF; ++p) {
       C t = C(0);
 #pragma unroll
@@ -695,9 +714,23 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
         for (int c = 0; c < 4; ++c) oth[c] = h[c];
       }
       const C nx = gq[0], ny = gq[1];
+      // The owner's trace is the left state. The tile's foreign items lead its
+      // list, so at most one wave holds both kinds. In FP64 one evaluation
+      // serves both (half the code); with FP32 stage states the two branches
+      // keep their roundings.
       const bool owner = packed & (1 << 12);
-      if (owner) numflux<C, !SHOCK>(FLUX, g, own, oth, nx, ny, F);
-      else numflux<C, !SHOCK>(FLUX, g, oth, own, nx, ny, F);
+      if constexpr (sizeof(S) == 8) {
+        C qL[4], qR[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          qL[c] = owner ? own[c] : oth[c];
+          qR[c] = owner ? oth[c] : own[c];
+        }
+        numflux<C, !SHOCK>(FLUX, g, qL, qR, nx, ny, F);
+      } else {
+        if (owner) numflux<C, !SHOCK>(FLUX, g, own, oth, nx, ny, F);
+        else numflux<C, !SHOCK>(FLUX, g, oth, own, nx, ny, F);
+      }
       if constexpr (SHOCK) {
         // Viscous edge flux at owner point jo (StoreEdgeViscousFlux,
         // edges.go:151-244): average of the two sides' eps*grad Q along
@@ -831,15 +864,48 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   }
   __syncthreads();
 
-  // FP32 matrix-core path, stages 1-3: phase E's q0 operand, loaded under
-  // phase C
-  constexpr bool PF = MF && !LAST && sizeof(C) == 4;
-  double q0p[PF ? 4 : 1][PF ? KI : 1];
-  if constexpr (PF) {
-    if (l.stage >= 1) {
-      const double *q0e = static_cast<const double *>(a.q0) + tb + me;
+  // phase E's operands, loaded under phase C: all of the thread's up to order
+  // 2, q0 of stages 1-3 on the matrix cores, whose last stage takes the four
+  // arrays a variable ahead (the first one here). Order 4 in FP64 has no
+  // registers left for them under C and loads them at E.
+  constexpr bool PV = !MF && NpInt <= 6, PQ = MF && !LAST, PL = MF && LAST, PC = !(N == 4 && sizeof(C) == 8);
+  constexpr int MD = PL && PC ? 2 : 1;
+  double v0[PV ? NpInt : 1], vR[PV && LAST ? NpInt : 1];
+  S v2[PV && LAST ? NpInt : 1], v3[PV && LAST ? NpInt : 1];
+  double m0[PQ ? 4 : MD][MF ? KI : 1], mR[MD][PL ? KI : 1];
+  S m2[MD][PL ? KI : 1], m3[MD][PL ? KI : 1];
+  if constexpr (PQ) {
 #pragma unroll
-      for (int c = 0; c < 4; ++c) lane_load<N, C>(q0e + c * NpInt * E, krow, q0p[c]);
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int j = 0; j < KI; ++j) m0[c][j] = 0.0;
+  }
+  const size_t eb = MF ? tb + me : vb;
+  double *q0 = static_cast<double *>(a.q0) + eb, *Rr = static_cast<double *>(a.R) + eb;
+  S *q1 = static_cast<S *>(a.q1) + eb, *q2 = static_cast<S *>(a.q2) + eb;
+  S *q3 = static_cast<S *>(a.q3) + eb, *q4 = static_cast<S *>(a.q4) + eb;
+  if constexpr (PV) {
+#pragma unroll
+    for (int i = 0; i < NpInt; ++i) {
+      v0[i] = 0.0;
+      if (LAST || l.stage >= 1) v0[i] = q0[i * E];
+      if constexpr (LAST) {
+        v2[i] = q2[i * E];
+        v3[i] = q3[i * E];
+        vR[i] = Rr[i * E];
+      }
+    }
+  }
+  if constexpr (PC) {
+    if constexpr (PQ) {
+      if (l.stage >= 1)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) lane_load<N, C>(q0 + c * NpInt * E, krow, m0[c]);
+    } else if constexpr (PL) {
+      lane_load<N, C>(q0, krow, m0[0]);
+      lane_load<N, C>(q2, krow, m2[0]);
+      lane_load<N, C>(q3, krow, m3[0]);
+      lane_load<N, C>(Rr, krow, mR[0]);
     }
   }
   // ---- C: interior flux + divergence ----
@@ -880,7 +946,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     for (int c = 0; c < 4; ++c) rq[c] = rq[c] * moojd;
   } else {
     // VALU: thread (element te, variable tn); the face fluxes
-#pragma unroll 2
+#pragma unroll UT
     for (int p = 0; p < NF; ++p) {
       const C Fe = sT[tn * TS + p * kTP + te];
 #pragma unroll
@@ -973,55 +1039,47 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   }
   int bad = 0;
   {
-    const size_t base = MF ? tb + me : vb;
-    double *q0 = static_cast<double *>(a.q0) + base;
-    S *q1 = static_cast<S *>(a.q1) + base;
-    S *q2 = static_cast<S *>(a.q2) + base;
-    S *q3 = static_cast<S *>(a.q3) + base;
-    S *q4 = static_cast<S *>(a.q4) + base;
-    double *Rr = static_cast<double *>(a.R) + base;
     if constexpr (MF) {
       // the lane's values: variable c at point MS::point(krow, j) of element
       // me; the divergence is rq, the stage input qv, which takes the new
       // state for phase F (a repeated point keeps its finite old value)
       const double dte = lts ? sDT[me] : dt;
+      if constexpr (!PC && PQ) {
+        if (stage >= 1)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) lane_load<N, C>(q0 + c * NpInt * E, krow, m0[c]);
+      }
       const bool real = me < nreal;
       if constexpr (LAST) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-          double v0[KI], vR[KI];
-          S v2[KI], v3[KI];
-          lane_load<N, C>(q0 + c * NpInt * E, krow, v0);
-          lane_load<N, C>(q2 + c * NpInt * E, krow, v2);
-          lane_load<N, C>(q3 + c * NpInt * E, krow, v3);
-          lane_load<N, C>(Rr + c * NpInt * E, krow, vR);
+          const int b = PC ? c & 1 : 0, cn = PC ? c + 1 : c;  // cn: the variable to load
+          if (cn < 4) {
+            lane_load<N, C>(q0 + cn * NpInt * E, krow, m0[PC ? b ^ 1 : 0]);
+            lane_load<N, C>(q2 + cn * NpInt * E, krow, m2[PC ? b ^ 1 : 0]);
+            lane_load<N, C>(q3 + cn * NpInt * E, krow, m3[PC ? b ^ 1 : 0]);
+            lane_load<N, C>(Rr + cn * NpInt * E, krow, mR[PC ? b ^ 1 : 0]);
+          }
+          double n0[KI], nR[KI];
 #pragma unroll
           for (int j = 0; j < KI; ++j) {
             const double dtR = dte * double(rq[c][j]);
-            const double Rn = -v0[j] + 0.517231671970585 * double(v2[j]) + 0.096059710526146 * double(v3[j]) +
-                              0.386708617503269 * double(qv[c][j]) + 0.063692468666290 * (dte * vR[j]) +
+            const double Rn = -m0[b][j] + 0.517231671970585 * double(m2[b][j]) + 0.096059710526146 * double(m3[b][j]) +
+                              0.386708617503269 * double(qv[c][j]) + 0.063692468666290 * (dte * mR[b][j]) +
                               0.226007483236906 * dtR;
-            vR[j] = Rn;
-            v0[j] += Rn;
+            nR[j] = Rn;
+            n0[j] = m0[b][j] + Rn;
             if (MS::point(krow, j) < NpInt) {
-              qv[c][j] = C(v0[j]);
-              if (real && !(v0[j] == v0[j])) bad = 1;
+              qv[c][j] = C(n0[j]);
+              if (real && !(n0[j] == n0[j])) bad = 1;
             }
           }
-          lane_store<N, C>(Rr + c * NpInt * E, krow, vR);
-          lane_store<N, C>(q0 + c * NpInt * E, krow, v0);
+          lane_store<N, C>(Rr + c * NpInt * E, krow, nR);
+          lane_store<N, C>(q0 + c * NpInt * E, krow, n0);
+          __builtin_amdgcn_sched_barrier(0);  // one variable ahead, not all: registers
         }
       } else {
-        double v0[4][KI];
-        if constexpr (PF) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-#pragma unroll
-            for (int j = 0; j < KI; ++j) v0[c][j] = q0p[c][j];  // loaded under phase C
-        } else if (stage >= 1) {
-#pragma unroll
-          for (int c = 0; c < 4; ++c) lane_load<N, C>(q0 + c * NpInt * E, krow, v0[c]);
-        }
+        const SspCoef k = ssp_coef(stage);
         S *qn = stage == 0 ? q1 : stage == 1 ? q2 : stage == 2 ? q3 : q4;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -1029,16 +1087,8 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
           double rh[KI];
 #pragma unroll
           for (int j = 0; j < KI; ++j) {
-            const double rhs = double(rq[c][j]);
-            const double qsv = double(qv[c][j]);
-            const double dtR = dte * rhs;
-            rh[j] = rhs;
-            switch (stage) {
-              case 0: nv[j] = S(qsv + 0.391752226571890 * dtR); break;
-              case 1: nv[j] = S(0.444370493651235 * v0[c][j] + 0.555629506348765 * qsv + 0.368410593050371 * dtR); break;
-              case 2: nv[j] = S(0.620101851488403 * v0[c][j] + 0.379898148511597 * qsv + 0.251891774271694 * dtR); break;
-              default: nv[j] = S(0.178079954393132 * v0[c][j] + 0.821920045606868 * qsv + 0.544974750228521 * dtR); break;
-            }
+            rh[j] = double(rq[c][j]);
+            nv[j] = S(ssp_mid(k, m0[c][j], double(qv[c][j]), dte * rh[j]));
             if (MS::point(krow, j) < NpInt) {
               qv[c][j] = C(nv[j]);
               if (real && !(nv[j] == nv[j])) bad = 1;
@@ -1049,25 +1099,36 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
         }
       }
     } else {
-      // the thread's values: variable tn at the points of element te; the
-      // operands in chunks of CH points (the last stage has four arrays of
-      // them), each loaded before it is combined and stored
+      // the thread's values: variable tn at the points of element te; beyond
+      // order 2 the operands come in chunks of CH points (the last stage has
+      // four arrays of them), each loaded before it is combined and stored
       const double dte = lts ? sDT[te] : dt;
       const bool real = te < nreal;
-      constexpr int CH = NpInt <= 6 ? NpInt : 5;
+      const SspCoef k = ssp_coef(stage);
+      constexpr int CH = PV ? NpInt : 5;
       S *qn = stage == 0 ? q1 : stage == 1 ? q2 : stage == 2 ? q3 : q4;
 #pragma unroll
       for (int i0 = 0; i0 < NpInt; i0 += CH) {
-        double v0[CH], vR[LAST ? CH : 1];
-        S v2[LAST ? CH : 1], v3[LAST ? CH : 1];
+        double c0[CH], cR[LAST ? CH : 1];
+        S c2[LAST ? CH : 1], c3[LAST ? CH : 1];
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
-          const int o = min(i0 + j, NpInt - 1) * E;
-          if (LAST || stage >= 1) v0[j] = q0[o];
-          if constexpr (LAST) {
-            v2[j] = q2[o];
-            v3[j] = q3[o];
-            vR[j] = Rr[o];
+          const int o = min(i0 + j, NpInt - 1);
+          if constexpr (PV) {
+            c0[j] = v0[j];
+            if constexpr (LAST) {
+              c2[j] = v2[j];
+              c3[j] = v3[j];
+              cR[j] = vR[j];
+            }
+          } else {
+            c0[j] = 0.0;
+            if (LAST || stage >= 1) c0[j] = q0[o * E];
+            if constexpr (LAST) {
+              c2[j] = q2[o * E];
+              c3[j] = q3[o * E];
+              cR[j] = Rr[o * E];
+            }
           }
         }
 #pragma unroll
@@ -1077,21 +1138,21 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
           const double rhs = double(acc[i]), qsv = double(q[i]), dtR = dte * rhs;
           if constexpr (LAST) {
             // R = -q0 + a q2 + b q3 + c q4 + d dt R3 + e dt RHS, q0 += R
-            const double dtR3 = dte * vR[j];
+            const double dtR3 = dte * cR[j];
             double Rn;
             if constexpr (sizeof(S) == 4)
-              Rn = ssp_last_f32(te * NV + tn * NpInt + i >= (NpInt - 3) * kThreads, v0[j], double(v2[j]), double(v3[j]), qsv,
+              Rn = ssp_last_f32(te * NV + tn * NpInt + i >= (NpInt - 3) * kThreads, c0[j], double(c2[j]), double(c3[j]), qsv,
                                 dtR3, dtR);
             else
-              Rn = -v0[j] + 0.517231671970585 * double(v2[j]) + 0.096059710526146 * double(v3[j]) +
+              Rn = -c0[j] + 0.517231671970585 * double(c2[j]) + 0.096059710526146 * double(c3[j]) +
                    0.386708617503269 * qsv + 0.063692468666290 * dtR3 + 0.226007483236906 * dtR;
-            const double nv = v0[j] + Rn;
+            const double nv = c0[j] + Rn;
             Rr[i * E] = Rn;
             q0[i * E] = nv;
             q[i] = C(nv);
             if (real && !(nv == nv)) bad = 1;
           } else {
-            const S nv = S(ssp_mid(stage, stage >= 1 ? v0[j] : 0.0, qsv, dtR));
+            const S nv = S(ssp_mid(k, c0[j], qsv, dtR));
             if (stage == 3) Rr[i * E] = rhs;
             qn[i * E] = nv;
             q[i] = C(nv);
@@ -1113,7 +1174,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     if constexpr (MF) {
       traces_mfma_regs<N, C>(qv, sT, lane, krow, me, TS);
     } else {
-#pragma unroll 2
+#pragma unroll UT
       for (int p = 0; p < NF; ++p) {
         C t = C(0);
 #pragma unroll
@@ -1145,7 +1206,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
       }
     }
     // the faces with a boundary state: the speed of that state
-    const int nbs = a.g.bst_cnt[tile] * NpEdge;
+    const int nbs = nbst * NpEdge;
 #pragma unroll 1
     for (int it = tid; it < nbs; it += kThreads) {
       const int w = it / NpEdge, pp = it - w * NpEdge;
@@ -1187,7 +1248,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
         const int e = packed & 255, f = packed >> 8;
         fw[size_t(f) * Kp + k0 + e] = from_bits(sWf[e * 3 + f]);
       }
-      for (int w = tid; w < a.g.bst_cnt[tile]; w += kThreads) {
+      for (int w = tid; w < nbst; w += kThreads) {
         const int packed = a.g.bnd_item[2 * size_t(bnd0 + w)];
         const int e = packed & 255, f = packed >> 8;
         fw[size_t(f) * Kp + k0 + e] = from_bits(sWf[e * 3 + f]);
