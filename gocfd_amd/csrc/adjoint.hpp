@@ -101,13 +101,14 @@ struct AdjBufs {
   void *out;            // next stage input (or the step's result)
   void *FE;             // face-point edge fluxes, scaled by ||n|| and side
   void *R;              // RHS output
-  void *SP;             // face-point wave speeds
+  void *SP;             // face-point wave speeds (local time stepping)
   void *dts;            // [5] stage time steps (double or dual)
   int *argmax;          // [5] face point of each stage's maximum wave speed
   double *Wv;           // [5] the maximum wave speeds
   double *time;         // step-start time (advanced by the last stage's dt)
   int *flag;            // set when a stage's dt would be clamped to FinalTime
   double *part_v;       // reduction partials (4 nparts)
+  void *part_t;         // largest wave speed of each workgroup of ADJ_FWD_FACE, and its point
   int *part_i;
   int nparts;
   // adjoint
@@ -152,8 +153,8 @@ struct AdjBufs {
 };
 
 enum AdjOp : int {
-  ADJ_FWD_FACE = 0,  // FE <- edge values of Us; SP <- owner-side wave speeds of Us
-  ADJ_ARGMAX,        // dts[stage], argmax[stage], Wv[stage] <- from SP; time, flag
+  ADJ_FWD_FACE = 0,  // FE <- edge values of Us; part_t, part_i (SP) <- owner-side wave speeds of Us
+  ADJ_ARGMAX,        // dts[stage], argmax[stage], Wv[stage] <- from the parts; time, flag
   ADJ_FWD_RHS,       // R <- RHS(Us, FE); out <- the stage's SSP54 combination
   ADJ_ADJ_SSP,       // cotangents through the SSP combination; lam_dt[stage]
   ADJ_ADJ_FACE,      // lamOwn, lamFarPts <- from lamR at Us

@@ -4,18 +4,14 @@
 #include <hip/hip_runtime.h>
 
 #include "adjoint.hpp"
-#include "dual.hpp"
+#include "adjoint_argmax.hpp"
 
 namespace gocfd {
 namespace dev {
 
 using ad::Dual;
 
-__device__ __forceinline__ double val_of(double a) { return a; }
-__device__ __forceinline__ double val_of(const Dual &a) { return a.v; }
-
-// Partial arg-max of the wave speeds: the largest value, ties to the
-// smallest index (a deterministic choice of the point the dt follows)
+// Partial arg-max of the viscous speeds
 template <class T>
 __global__ void __launch_bounds__(256) k_adj_argmax_part(const T *SP, size_t n, double *pv, int *pi) {
   __shared__ double sv[256];
@@ -46,28 +42,31 @@ __global__ void __launch_bounds__(256) k_adj_argmax_part(const T *SP, size_t n, 
   }
 }
 
-// The arg-max over the partials in one block (ties to the smallest index)
-__device__ int argmax_of_parts(const double *pv, const int *pi, int nparts, double *sv, int *si) {
+// The partial of the arg-max over the partials in one block (-1: none)
+constexpr int kFinalThreads = 1024;
+template <class V>
+__device__ int argmax_of_parts(const V *pv, const int *pi, int nparts, double *sv, int *si, int *sb) {
+  const int t = threadIdx.x;
   double bv = -2.;
-  int bi = -1;
-  for (int i = threadIdx.x; i < nparts; i += blockDim.x) {
-    if (pv[i] > bv || (pv[i] == bv && pi[i] >= 0 && (bi < 0 || pi[i] < bi))) { bv = pv[i]; bi = pi[i]; }
+  int bi = -1, bb = -1;
+  for (int i = t; i < nparts; i += kFinalThreads) {
+    const double v = val_of(pv[i]);
+    const int x = pi[i];
+    if (ranks_before(v, x, bv, bi)) { bv = v; bi = x; bb = i; }
   }
-  sv[threadIdx.x] = bv;
-  si[threadIdx.x] = bi;
+  sv[t] = bv;
+  si[t] = bi;
+  sb[t] = bb;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (int(threadIdx.x) < w) {
-      const double ov = sv[threadIdx.x + w];
-      const int oi = si[threadIdx.x + w];
-      if (ov > sv[threadIdx.x] || (ov == sv[threadIdx.x] && oi >= 0 && (si[threadIdx.x] < 0 || oi < si[threadIdx.x]))) {
-        sv[threadIdx.x] = ov;
-        si[threadIdx.x] = oi;
-      }
+  for (int w = kFinalThreads / 2; w > 0; w >>= 1) {
+    if (t < w && ranks_before(sv[t + w], si[t + w], sv[t], si[t])) {
+      sv[t] = sv[t + w];
+      si[t] = si[t + w];
+      sb[t] = sb[t + w];
     }
     __syncthreads();
   }
-  const int r = si[0];
+  const int r = sb[0];
   __syncthreads();
   return r;
 }
@@ -77,15 +76,17 @@ __device__ int argmax_of_parts(const double *pv, const int *pi, int nparts, doub
 // speed; calculateGlobalDT euler.go:945-971), the FinalTime check of the
 // solver's clamp, and the time advance after the last stage
 template <class T>
-__global__ void __launch_bounds__(256) k_adj_argmax_final(const T *SP, const double *pv, const int *pi, int nparts,
+__global__ void __launch_bounds__(kFinalThreads) k_adj_argmax_final(const T *pt, const int *pi, int nparts,
                                                           int stage, double cfl, double final_time, T *dts,
                                                           int *argmax, double *Wv, double *time, int *flag,
                                                           const T *SPV, const double *pv2, const int *pi2,
-                                                          double cdiff, int *argmaxv, double *Wvv, int *vbr) {
-  __shared__ double sv[256];
-  __shared__ int si[256];
-  const int idx = argmax_of_parts(pv, pi, nparts, sv, si);
-  const int idv = SPV ? argmax_of_parts(pv2, pi2, nparts, sv, si) : -1;
+                                                          int nparts2, double cdiff, int *argmaxv, double *Wvv, int *vbr) {
+  __shared__ double sv[kFinalThreads];
+  __shared__ int si[kFinalThreads], sb[kFinalThreads];
+  const int part = argmax_of_parts(pt, pi, nparts, sv, si, sb);
+  const int idx = part >= 0 ? pi[part] : -1;
+  const int part2 = SPV ? argmax_of_parts(pv2, pi2, nparts2, sv, si, sb) : -1;
+  const int idv = part2 >= 0 ? pi2[part2] : -1;
   if (threadIdx.x == 0) {
     argmax[stage] = idx;
     if (SPV) {
@@ -99,7 +100,7 @@ __global__ void __launch_bounds__(256) k_adj_argmax_final(const T *SP, const dou
       Wv[stage] = 0.;
       return;
     }
-    const T W = SP[idx];
+    const T W = pt[part];
     T dt = cfl / W;
     if (idv >= 0 && val_of(SPV[idv]) > 0.) {
       const T dtv = cdiff / SPV[idv];
@@ -241,29 +242,22 @@ hipError_t adj_launch_common(int op, const AdjArgs &a, const AdjBufs &b, hipStre
   switch (op) {
     case ADJ_ARGMAX: {
       const size_t nfp = size_t(3) * a.Kp * (a.N + 2);
+      const int np = int(blocks_of(nfp));  // ADJ_FWD_FACE's workgroups
+#define GOCFD_ARGMAX(TT)                                                                                         \
+  if (a.act)                                                                                                     \
+    hipLaunchKernelGGL((k_adj_argmax_part<TT>), dim3(b.nparts), dim3(256), 0, s, static_cast<const TT *>(b.SPV),   \
+                       nfp, b.part_v2, b.part_i2);                                                                \
+  hipLaunchKernelGGL((k_adj_argmax_final<TT>), dim3(1), dim3(kFinalThreads), 0, s,                                 \
+                     static_cast<const TT *>(b.part_t), b.part_i, np, b.stage, a.ph.cfl, a.ph.final_time,          \
+                     static_cast<TT *>(b.dts), b.argmax, b.Wv, b.time, b.flag,                                     \
+                     a.act ? static_cast<const TT *>(b.SPV) : nullptr, b.part_v2, b.part_i2, b.nparts, a.cdiff,     \
+                     b.argmaxv, b.Wvv, b.vbr);
       if (b.dual) {
-        hipLaunchKernelGGL((k_adj_argmax_part<Dual>), dim3(b.nparts), dim3(256), 0, s,
-                           static_cast<const Dual *>(b.SP), nfp, b.part_v, b.part_i);
-        if (a.act)
-          hipLaunchKernelGGL((k_adj_argmax_part<Dual>), dim3(b.nparts), dim3(256), 0, s,
-                             static_cast<const Dual *>(b.SPV), nfp, b.part_v2, b.part_i2);
-        hipLaunchKernelGGL((k_adj_argmax_final<Dual>), dim3(1), dim3(256), 0, s, static_cast<const Dual *>(b.SP),
-                           b.part_v, b.part_i, b.nparts, b.stage, a.ph.cfl, a.ph.final_time,
-                           static_cast<Dual *>(b.dts), b.argmax, b.Wv, b.time, b.flag,
-                           a.act ? static_cast<const Dual *>(b.SPV) : nullptr, b.part_v2, b.part_i2, a.cdiff,
-                           b.argmaxv, b.Wvv, b.vbr);
+        GOCFD_ARGMAX(Dual)
       } else {
-        hipLaunchKernelGGL((k_adj_argmax_part<double>), dim3(b.nparts), dim3(256), 0, s,
-                           static_cast<const double *>(b.SP), nfp, b.part_v, b.part_i);
-        if (a.act)
-          hipLaunchKernelGGL((k_adj_argmax_part<double>), dim3(b.nparts), dim3(256), 0, s,
-                             static_cast<const double *>(b.SPV), nfp, b.part_v2, b.part_i2);
-        hipLaunchKernelGGL((k_adj_argmax_final<double>), dim3(1), dim3(256), 0, s,
-                           static_cast<const double *>(b.SP), b.part_v, b.part_i, b.nparts, b.stage, a.ph.cfl,
-                           a.ph.final_time, static_cast<double *>(b.dts), b.argmax, b.Wv, b.time, b.flag,
-                           a.act ? static_cast<const double *>(b.SPV) : nullptr, b.part_v2, b.part_i2, a.cdiff,
-                           b.argmaxv, b.Wvv, b.vbr);
+        GOCFD_ARGMAX(double)
       }
+#undef GOCFD_ARGMAX
       break;
     }
     case ADJ_ADJ_SSP:
@@ -271,7 +265,8 @@ hipError_t adj_launch_common(int op, const AdjArgs &a, const AdjBufs &b, hipStre
       hipLaunchKernelGGL(k_adj_ssp, dim3(b.nparts), dim3(256), 0, s, b.stage, b.n, b.lam, b.lamU0, b.lamQ[1],
                          b.lamQ[2], b.lamQ[3], b.lamQ[4], b.lamR, b.lamR3, static_cast<const double *>(b.Rs),
                          static_cast<const double *>(b.R3), static_cast<const double *>(b.dts), b.part_v);
-      hipLaunchKernelGGL(k_adj_sum, dim3(1), dim3(256), 0, s, b.part_v, b.nparts, b.lam_dt, b.stage);
+      // (otherwise summed by the stage's dt term, k_adj_wave)
+      if (a.act) hipLaunchKernelGGL(k_adj_sum, dim3(1), dim3(256), 0, s, b.part_v, b.nparts, b.lam_dt, b.stage);
       break;
     case ADJ_FAR_SUM:
       // 4 partials per block; the result goes to b.target[0..3]

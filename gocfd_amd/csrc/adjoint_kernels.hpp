@@ -20,6 +20,7 @@
 #include <hip/hip_runtime.h>
 
 #include "adjoint.hpp"
+#include "adjoint_argmax.hpp"
 #include "dfr_setup.hpp"
 #include "dual.hpp"
 #include "kernels.hpp"
@@ -139,29 +140,59 @@ __device__ __forceinline__ void face_point(const AdjArgs &a, size_t t, int &f, i
 // A shared edge point's flux is evaluated once, by the owner's face point,
 // which writes both sides' edge values: w_own F* and -w_nbr F* at the
 // partner's reversed point (the value the reference stores once per edge
-// and reads from both sides). The same pass stores each face point's wave
+// and reads from both sides). The same pass takes each face point's wave
 // speed (|U| + c) / hK on its post-BC trace where the face bounds the time
-// step (the edge's owner side), -1 elsewhere.
+// step (the edge's owner side; -1 elsewhere): the workgroup's largest and its
+// point go to pt/pi (a pass over stored speeds took another 5 us at 20,000
+// elements, 2 us of them a launch), every one to SP with local time stepping.
 template <int N, class T, int FLUX>
-__global__ void __launch_bounds__(256) k_adj_fwd_face(AdjArgs a, const T *U, T *FE, T *SP) {
+__global__ void __launch_bounds__(256) k_adj_fwd_face(AdjArgs a, const T *U, T *FE, T *SP, T *pt, int *pi) {
   using Sh = AdjShape<N>;
   constexpr int NpEdge = Sh::NpEdge;
+  __shared__ double rv[4];
+  __shared__ int ri[4];
   const size_t t = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= size_t(3) * a.Kp * NpEdge) return;
-  int f, kk, pp;
-  size_t fi;
-  face_point<N>(a, t, f, kk, pp, fi);
-  if (kk >= a.K) {
+  const bool in = t < size_t(3) * a.Kp * NpEdge;
+  int f = 0, kk = a.K, pp = 0, code = 0;
+  size_t fi = 0;
+  if (in) face_point<N>(a, t, f, kk, pp, fi);
+  const bool real = in && kk < a.K;
+  T own[4], qfar[4], F[4], sp = T(-1.);
+  far_state(a, qfar);
+  if (real) {
+    code = a.code[fi];
+    trace_at<N>(a, U, kk, f * NpEdge + pp, own);
+    if (code & FC_WAVE) sp = wave_value(a, code, fi, a.oohK[kk], own, qfar);
+  }
+  if (in && a.lts) SP[t] = sp;
+  double mv = in ? val_of(sp) : -2.;
+  int mi = in ? int(t) : -1;
+  for (int d = 32; d > 0; d >>= 1) {
+    const double ov = __shfl_xor(mv, d, 64);
+    const int oi = __shfl_xor(mi, d, 64);
+    if (ranks_before(ov, oi, mv, mi)) {
+      mv = ov;
+      mi = oi;
+    }
+  }
+  if (threadIdx.x % 64 == 0) {
+    rv[threadIdx.x / 64] = mv;
+    ri[threadIdx.x / 64] = mi;
+  }
+  __syncthreads();
+  for (int w = 0; w < 4; ++w)
+    if (ranks_before(rv[w], ri[w], mv, mi)) {
+      mv = rv[w];
+      mi = ri[w];
+    }
+  if (threadIdx.x == 0) pi[blockIdx.x] = mi;
+  if (mi < 0 ? threadIdx.x == 0 : in && int(t) == mi) pt[blockIdx.x] = sp;  // the thread of the largest
+  if (!in) return;
+  if (!real) {
     for (int c = 0; c < 4; ++c) FE[4 * t + c] = T(0.);
-    SP[t] = T(-1.);
     return;
   }
-  const int code = a.code[fi], kind = code & 15;
-  T own[4], qfar[4], F[4];
-  trace_at<N>(a, U, kk, f * NpEdge + pp, own);
-  far_state(a, qfar);
-  SP[t] = (code & FC_WAVE) ? wave_value(a, code, fi, a.oohK[kk], own, qfar) : T(-1.);
-  if (kind == FK_Shared) {
+  if ((code & 15) == FK_Shared) {
     if (!(code & FC_FLUX_OWNER)) return;  // written by the owner
     const int nb = a.nbr_elem[fi], nf = a.nbr_face[fi], rp = NpEdge - 1 - pp;
     T oth[4];
@@ -895,12 +926,32 @@ __global__ void __launch_bounds__(256) k_adj_lts_wave(AdjArgs a, const double *U
 
 // The dt term of a stage: dt = CFL / W with W the wave speed at the stage's
 // arg-max face point; its cotangent goes to that point's trace (and the far
-// state for a far-field face). One thread.
+// state for a far-field face). One workgroup; lane (side, d) of the first
+// wave takes one input direction, then the lanes take the element's values.
+// (A single thread took 12 us, serial through eight dual evaluations.) part:
+// the partials of the dt cotangent, summed here in a fixed order (null: it is
+// in lam_dt already).
 template <int N>
-__global__ void k_adj_wave(AdjArgs a, int stage, const double *U, const int *argmax, const double *Wv,
-                           const double *lam_dt, double *target, double *lamFarW, const int *vbr) {
+__global__ void __launch_bounds__(256) k_adj_wave(AdjArgs a, int stage, const double *U, const int *argmax,
+                                                  const double *Wv, double *lam_dt, double *target, double *lamFarW,
+                                                  const int *vbr, const double *part, int nparts) {
   using Sh = AdjShape<N>;
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
+  __shared__ double red[256], lo[4];
+  double ldt = 0.;
+  if (part) {
+    double s = 0.;
+    for (int i = threadIdx.x; i < nparts; i += blockDim.x) s += part[i];
+    red[threadIdx.x] = s;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+      if (int(threadIdx.x) < w) red[threadIdx.x] += red[threadIdx.x + w];
+      __syncthreads();
+    }
+    ldt = red[0];
+    if (threadIdx.x == 0) lam_dt[stage] = ldt;
+  } else {
+    ldt = lam_dt[stage];
+  }
   if (vbr && vbr[stage]) return;  // the viscous dt bound this stage
   const int idx = argmax[stage];
   if (idx < 0) return;
@@ -908,32 +959,28 @@ __global__ void k_adj_wave(AdjArgs a, int stage, const double *U, const int *arg
   size_t fi;
   face_point<N>(a, size_t(idx), f, kk, pp, fi);
   const double W = Wv[stage];
-  const double lW = -(a.ph.cfl / (W * W)) * lam_dt[stage];
+  const double lW = -(a.ph.cfl / (W * W)) * ldt;
   const int code = a.code[fi];
-  double own[4], qfar[4];
-  trace_at<N>(a, U, kk, f * Sh::NpEdge + pp, own);
-  far_state(a, qfar);
   const bool far = (code & 15) == FK_Far && ((code >> 8) == 0 || a.io_tied);
-  double lo[4];
-  for (int d = 0; d < 4; ++d) {
+  const int side = int(threadIdx.x) >> 2, d = int(threadIdx.x) & 3;
+  if (side == 0 || (side == 1 && far)) {
+    double own[4], qfar[4];
+    trace_at<N>(a, U, kk, f * Sh::NpEdge + pp, own);
+    far_state(a, qfar);
     Dual o[4], q[4];
     for (int c = 0; c < 4; ++c) {
-      o[c] = Dual(own[c], c == d ? 1. : 0.);
-      q[c] = Dual(qfar[c]);
+      o[c] = Dual(own[c], side == 0 && c == d ? 1. : 0.);
+      q[c] = Dual(qfar[c], side == 1 && c == d ? 1. : 0.);
     }
-    lo[d] = lW * wave_value(a, code, fi, a.oohK[kk], o, q).d;
-    if (far) {
-      for (int c = 0; c < 4; ++c) {
-        o[c] = Dual(own[c]);
-        q[c] = Dual(qfar[c], c == d ? 1. : 0.);
-      }
-      lamFarW[d] += lW * wave_value(a, code, fi, a.oohK[kk], o, q).d;
-    }
+    const double v = lW * wave_value(a, code, fi, a.oohK[kk], o, q).d;
+    if (side == 0) lo[d] = v;
+    else lamFarW[d] += v;
   }
-  const double *row = a.Interp + (f * Sh::NpEdge + pp) * Sh::NpInt;
-  double *tg = target + size_t(kk) * Sh::NV;
-  for (int c = 0; c < 4; ++c)
-    for (int i = 0; i < Sh::NpInt; ++i) tg[c * Sh::NpInt + i] += row[i] * lo[c];
+  __syncthreads();
+  if (int(threadIdx.x) < Sh::NV) {
+    const int c = int(threadIdx.x) / Sh::NpInt, i = int(threadIdx.x) - c * Sh::NpInt;
+    target[size_t(kk) * Sh::NV + threadIdx.x] += a.Interp[(f * Sh::NpEdge + pp) * Sh::NpInt + i] * lo[c];
+  }
 }
 
 // ---- PerssonC0 with an active sensor ----
@@ -1520,14 +1567,16 @@ hipError_t adj_launch_n(int op, const AdjArgs &a, const AdjBufs &b, hipStream_t 
   const size_t nfp = size_t(3) * a.Kp * Sh::NpEdge;
   switch (op) {
     case ADJ_FWD_FACE:
-#define GOCFD_FWD_FACE(FL)                                                                                 \
-  if (b.dual)                                                                                              \
-    hipLaunchKernelGGL((k_adj_fwd_face<N, Dual, FL>), dim3(adj_blocks(nfp)), dim3(256), 0, s, a,           \
-                       static_cast<const Dual *>(b.Us), static_cast<Dual *>(b.FE), static_cast<Dual *>(b.SP)); \
-  else                                                                                                     \
-    hipLaunchKernelGGL((k_adj_fwd_face<N, double, FL>), dim3(adj_blocks(nfp)), dim3(256), 0, s, a,         \
-                       static_cast<const double *>(b.Us), static_cast<double *>(b.FE),                     \
-                       static_cast<double *>(b.SP));
+#define GOCFD_FWD_FACE_T(FL, TT)                                                                              \
+  hipLaunchKernelGGL((k_adj_fwd_face<N, TT, FL>), dim3(adj_blocks(nfp)), dim3(256), 0, s, a,                   \
+                     static_cast<const TT *>(b.Us), static_cast<TT *>(b.FE), static_cast<TT *>(b.SP),         \
+                     static_cast<TT *>(b.part_t), b.part_i);
+#define GOCFD_FWD_FACE(FL)       \
+  if (b.dual) {                  \
+    GOCFD_FWD_FACE_T(FL, Dual)   \
+  } else {                       \
+    GOCFD_FWD_FACE_T(FL, double) \
+  }
       switch (a.ph.flux) {
         case 0: GOCFD_FWD_FACE(0) break;
         case 1: GOCFD_FWD_FACE(1) break;
@@ -1535,6 +1584,7 @@ hipError_t adj_launch_n(int op, const AdjArgs &a, const AdjBufs &b, hipStream_t 
         default: GOCFD_FWD_FACE(3) break;
       }
 #undef GOCFD_FWD_FACE
+#undef GOCFD_FWD_FACE_T
       break;
     case ADJ_FWD_RHS: {
       const unsigned nb = unsigned((a.Kp + RhsElems<N>::value - 1) / RhsElems<N>::value);
@@ -1678,8 +1728,9 @@ hipError_t adj_launch_n(int op, const AdjArgs &a, const AdjBufs &b, hipStream_t 
                          b.lamEpsv, b.lamSigv, b.target);
       break;
     case ADJ_ADJ_WAVE:
-      hipLaunchKernelGGL((k_adj_wave<N>), dim3(1), dim3(64), 0, s, a, b.stage, static_cast<const double *>(b.Us),
-                         b.argmax, b.Wv, b.lam_dt, b.target, b.lamFarW, a.act ? b.vbr : nullptr);
+      hipLaunchKernelGGL((k_adj_wave<N>), dim3(1), dim3(256), 0, s, a, b.stage, static_cast<const double *>(b.Us),
+                         b.argmax, b.Wv, b.lam_dt, b.target, b.lamFarW, a.act ? b.vbr : nullptr,
+                         a.act ? nullptr : b.part_v, b.nparts);
       break;
     default:
       return hipErrorInvalidValue;

@@ -109,7 +109,7 @@ AdjointRunner::AdjointRunner(const Discretisation &d, const DeviceLayout &L, con
     R_[s].alloc(n_);
   }
   FE_.alloc(4 * nfp_);
-  SP_.alloc(nfp_);
+  if (lts) SP_.alloc(nfp_);
   tmp_.alloc(n_);
   dts_.alloc(5);
   argmax_.alloc(5);
@@ -117,7 +117,8 @@ AdjointRunner::AdjointRunner(const Discretisation &d, const DeviceLayout &L, con
   Wv_.alloc(5);
   time_.alloc(1);
   part_v_.alloc(4 * size_t(nparts_));
-  part_i_.alloc(size_t(nparts_));
+  part_t_.alloc((nfp_ + 255) / 256);
+  part_i_.alloc((nfp_ + 255) / 256);
   if (a_.act) {
     const size_t Kp = size_t(L.Kp), Nv = size_t(d.Nv), nr = size_t(NR_) * Kp;
     sig_.alloc(Kp);
@@ -233,6 +234,7 @@ void AdjointRunner::forward_step(bool dual, const void *Ustart, void *Uend, doub
   b.time = time;
   b.flag = flag_.p;
   b.part_v = part_v_.p;
+  b.part_t = part_t_.p;
   b.part_i = part_i_.p;
   b.n = n_;
   for (int s = 0; s < 5; ++s) {
@@ -453,7 +455,6 @@ void AdjointRunner::vjp(const double *q0, double t0, int nsteps, int every, cons
   dev::AdjBufs b{};
   b.dual = 0;
   b.part_v = part_v_.p;
-  b.part_i = part_i_.p;
   b.n = n_;
   b.lamU0 = lamU0.p;
   for (int s = 1; s < 5; ++s) b.lamQ[s] = lamQ[s].p;

@@ -101,7 +101,7 @@ class AdjointRunner {
   // stage record (sized for dual values; the double sweeps use the front half)
   DevBuf<dev::ad_storage> U_[5], R_[5];
   DevBuf<dev::ad_storage> FE_, SP_, tmp_;
-  DevBuf<dev::ad_storage> dts_;
+  DevBuf<dev::ad_storage> dts_, part_t_;
   DevBuf<int> argmax_, flag_, part_i_;
   DevBuf<double> Wv_, time_, part_v_;
   int nparts_ = 1024;
