@@ -386,51 +386,62 @@ void AdjointRunner::vjp(const double *q0, double t0, int nsteps, int every, cons
   every_ = std::min(every_, nsteps);
   const int nblocks = (nsteps + every_ - 1) / every_;
   const size_t bytes = n_ * sizeof(double);
-  // pooled states: checkpoints [0, nblocks), block starts, the result
+  // The states a step's transposed stages need (its start, four stage inputs
+  // and five right-hand sides: 10) are kept from the forward sweep for the last
+  // blocks, which are then not swept again: as many blocks as fit in a quarter
+  // of the free device memory, but one where the caller chose the spacing (that
+  // bounds the memory). The blocks before them are recomputed from their
+  // checkpoints into the first kept block's states, whose own steps are then
+  // done with; if not even one block fits, each step's record is recomputed
+  // from its start just before its transposed stages.
+  const size_t per_block = 10 * size_t(every_), have = states_.size();
+  size_t free_b = 0, total_b = 0;
+  HIPCHECK(hipMemGetInfo(&free_b, &total_b));
+  const size_t room = have + (free_b / 4) / bytes, fixed = size_t(nblocks + 1 + every_);
+  int kept = room > fixed ? int(std::min<size_t>(size_t(every > 0 ? 1 : nblocks), (room - fixed) / per_block)) : 0;
+  // GOCFD_ADJOINT_KEEP_RECORDS=0 forces the per-step recomputation
+  if (const char *e = std::getenv("GOCFD_ADJOINT_KEEP_RECORDS"))
+    if (e[0] == '0') kept = 0;
+  // the active sensor path keeps one step's record (its fields per stage)
+  if (a_.act) kept = 0;
+  stored_records_ = kept > 0;
+  // Pooled states: checkpoints [0, nblocks), the result, a block's starts where
+  // no record holds them, then 10 states per step of a kept block
+  const size_t rec0 = size_t(nblocks + 1 + (stored_records_ ? 0 : every_));
+  const int first_kept = nblocks - kept;
   std::vector<double *> ck(nblocks), S(every_, nullptr);
   for (int i = 0; i < nblocks; ++i) ck[i] = state(size_t(i));
-  for (int i = 1; i < every_; ++i) S[i] = state(size_t(nblocks + i));
-  double *const end = state(size_t(nblocks + every_));
-  const size_t rec0 = size_t(nblocks + every_ + 1);  // first stage-record state
+  double *const end = state(size_t(nblocks));
+  for (int i = 1; i < every_; ++i) S[i] = state(stored_records_ ? rec0 + 10 * size_t(i) : size_t(nblocks + i));
+  // step i of kept block q (0: the first kept): its start and its record
+  std::vector<StageRecord> recs(size_t(kept) * every_);
+  std::vector<double *> kept_start(recs.size());
+  for (size_t i = 0; i < recs.size(); ++i) {
+    StageRecord &r = recs[i];
+    const size_t s0 = rec0 + 10 * i;
+    kept_start[i] = i % every_ == 0 ? nullptr : state(s0);  // a block's first step starts at its checkpoint
+    r.U[0] = nullptr;
+    for (int s = 1; s < 5; ++s) r.U[s] = state(s0 + size_t(s));
+    for (int s = 0; s < 5; ++s) r.R[s] = state(s0 + 5 + size_t(s));
+    fill_small(r, small(i));
+  }
   HIPCHECK(hipMemsetAsync(flag_.p, 0, sizeof(int), s_));
   HIPCHECK(hipMemcpyAsync(time_.p, &t0, sizeof(double), hipMemcpyHostToDevice, s_));
   HIPCHECK(hipMemcpyAsync(ck[0], q0, bytes, hipMemcpyDeviceToDevice, s_));
-  // The stage records of a whole block are kept when the states they still
-  // need fit in a quarter of the free device memory; otherwise each step's
-  // record is recomputed from its start just before its transposed stages.
-  size_t free_b = 0, total_b = 0;
-  HIPCHECK(hipMemGetInfo(&free_b, &total_b));
-  const size_t want = rec0 + 9 * size_t(every_), have = states_.size();
-  stored_records_ = (want > have ? (want - have) * bytes : 0) <= free_b / 4;
-  // GOCFD_ADJOINT_KEEP_RECORDS=0 forces the per-step recomputation
-  if (const char *e = std::getenv("GOCFD_ADJOINT_KEEP_RECORDS")) stored_records_ = stored_records_ && e[0] != '0';
-  // the active sensor path keeps one step's record (its fields per stage)
-  if (a_.act) stored_records_ = false;
-  // With one block and its records kept, the record sweep is the forward
-  // sweep (with the FinalTime check); otherwise a forward sweep first stores
-  // the checkpoints at the block starts.
-  const bool one_sweep = nblocks == 1 && stored_records_;
+  // forward sweep: the checkpoints, the kept records, the FinalTime check
   const StageRecord scratch = scratch_record();
-  if (!one_sweep) {
-    for (int bk = 0; bk < nblocks; ++bk) {
-      const int j0 = bk * every_, cnt = std::min(every_, nsteps - j0);
-      const double *src = ck[bk];
-      for (int i = 0; i < cnt; ++i) {
-        double *dst = i + 1 < cnt ? S[i + 1] : (bk + 1 < nblocks ? ck[bk + 1] : end);
-        forward_step(false, src, dst, time_.p, scratch);
-        src = dst;
-      }
+  for (int bk = 0; bk < nblocks; ++bk) {
+    const int j0 = bk * every_, cnt = std::min(every_, nsteps - j0);
+    const size_t r0 = size_t(bk - first_kept) * every_;
+    const double *src = ck[bk];
+    for (int i = 0; i < cnt; ++i) {
+      double *dst = i + 1 == cnt ? (bk + 1 < nblocks ? ck[bk + 1] : end)
+                    : bk < first_kept ? S[i + 1] : kept_start[r0 + size_t(i) + 1];
+      forward_step(false, src, dst, time_.p, bk < first_kept ? scratch : recs[r0 + size_t(i)]);
+      src = dst;
     }
-    check_flag();
   }
-  std::vector<StageRecord> recs(stored_records_ ? size_t(every_) : 0);
-  for (size_t i = 0; i < recs.size(); ++i) {
-    StageRecord &r = recs[i];
-    r.U[0] = nullptr;
-    for (int s = 1; s < 5; ++s) r.U[s] = state(rec0 + 9 * i + size_t(s - 1));
-    for (int s = 0; s < 5; ++s) r.R[s] = state(rec0 + 9 * i + 4 + size_t(s));
-    fill_small(r, small(i));
-  }
+  check_flag();
   // reverse sweep
   if (!lamU0_.p) {
     lamU0_.alloc(n_);
@@ -475,18 +486,18 @@ void AdjointRunner::vjp(const double *q0, double t0, int nsteps, int every, cons
   b.lamEpsv = lamEpsv_.p;
   for (int bk = nblocks - 1; bk >= 0; --bk) {
     const int j0 = bk * every_, cnt = std::min(every_, nsteps - j0);
+    // the block's states: its own, or those of the first kept block
+    const size_t r0 = bk > first_kept ? size_t(bk - first_kept) * every_ : 0;
     std::vector<const double *> starts(cnt);
     starts[0] = ck[bk];
-    for (int i = 0; i < cnt; ++i) {
-      void *next = i + 1 < cnt ? static_cast<void *>(S[i + 1]) : static_cast<void *>(tmp_.p);
-      if (stored_records_) forward_step(false, starts[i], next, one_sweep ? time_.p : nullptr, recs[i]);
-      else if (i + 1 < cnt) forward_step(false, starts[i], next, nullptr, scratch);
-      if (i + 1 < cnt) starts[i + 1] = S[i + 1];
-    }
-    if (one_sweep) check_flag();
+    for (int i = 1; i < cnt; ++i) starts[i] = stored_records_ ? kept_start[r0 + size_t(i)] : S[i];
+    if (bk < first_kept)
+      for (int i = 0; i < (stored_records_ ? cnt : cnt - 1); ++i)
+        forward_step(false, starts[i], i + 1 < cnt ? const_cast<double *>(starts[i + 1]) : static_cast<void *>(tmp_.p),
+                     nullptr, stored_records_ ? recs[r0 + size_t(i)] : scratch);
     for (int i = cnt - 1; i >= 0; --i) {
       if (stored_records_) {
-        adjoint_step(starts[i], recs[i], b);
+        adjoint_step(starts[i], recs[r0 + size_t(i)], b);
       } else {
         forward_step(false, starts[i], tmp_.p, nullptr, scratch);
         adjoint_step(starts[i], scratch, b);

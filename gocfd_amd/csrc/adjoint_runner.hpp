@@ -1,10 +1,12 @@
 // Host driver of the tangent-linear and discrete-adjoint step (kernels in
 // adjoint_kernels.hpp / adjoint_common.hip, scope in adjoint.hpp).
 //
-// vjp: one forward sweep stores the state every `every` steps; the reverse
-// sweep recomputes each block of steps from its checkpoint, then each step's
-// five stage inputs, right-hand sides, dts and arg-max points, and applies
-// the transposed stages from the last to the first.
+// vjp: one forward sweep stores the state every `every` steps and, for the last
+// blocks that fit, each step's five stage inputs, right-hand sides, dts and
+// arg-max points; the reverse sweep recomputes these for the other blocks from
+// their checkpoints and applies the transposed stages from the last to the
+// first. (Recomputing every block took 44.5 ms for 20 steps at order 3, 100,000
+// elements, with all four blocks kept 33.4.)
 // jvp: the forward sweep in dual arithmetic.
 #pragma once
 

@@ -202,9 +202,10 @@ int gocfd_euler2d_get_element_dt(gocfd_euler2d *h, double *DT);
 /* Vector-Jacobian product over nsteps steps: dQ0 = (dQn/dQ)^T dQn_bar and
  * dQinf = (dQn/dQinf)^T dQn_bar (dQinf may be NULL). The reverse sweep
  * recomputes the steps from a checkpoint every checkpoint_every steps (0:
- * ceil(sqrt(nsteps))) and each step's stages from its start; with
- * checkpoint_every >= nsteps (one block) whose stage records fit in device
- * memory, the one recording sweep is also the forward sweep. */
+ * ceil(sqrt(nsteps))) and each step's stages from its start, except those of
+ * the last blocks whose stage records (10 states per step) the forward sweep
+ * kept: as many blocks as fit in a quarter of the free device memory with
+ * checkpoint_every = 0, at most one otherwise. */
 int gocfd_euler2d_vjp(gocfd_euler2d *h, int32_t nsteps, int32_t checkpoint_every, const double *dQn_bar,
                       double *dQ0, double *dQinf);
 /* Jacobian-vector product over nsteps steps (tangent-linear step in dual
