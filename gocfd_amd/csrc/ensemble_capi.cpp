@@ -277,7 +277,8 @@ struct gocfd_ensemble {
         if (g->shock) {
           a.sh.vbuf = int(gstage & 1);
           a.sh.filter_state = s == 2 ? 1 : 0;
-          for (int pass = 0; pass < dev::kShockPasses; ++pass) HIPCHECK(dev::launch_shock(g->N, prec, pass, a, st));
+          for (int pass = 0; pass < dev::kShockPasses; ++pass)
+            if (dev::shock_pass_runs(pass, s, gstage)) HIPCHECK(dev::launch_shock(g->N, prec, pass, a, st));
         }
         HIPCHECK(dev::launch_stage(g->N, prec, g->shock ? 1 : 0, a, st));
       }

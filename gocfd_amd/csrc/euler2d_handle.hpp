@@ -190,7 +190,7 @@ struct gocfd_euler2d {
       HIPCHECK(dev::launch_fill_u64(epsV.p, epsV.n, 0ull, stream));
     }
     if (lts) HIPCHECK(dev::launch_fill_f64(DTv.p, DTv.n, 0.0, stream));
-    if (!shock) {  // with shock capturing each stage's gradient pass measures its wave speeds
+    if (!shock) {  // with shock capturing a pass of the first stage measures its wave speeds
       dev::StageArgs a = args();
       a.qs = q[0];
       a.ring = 0;
@@ -227,7 +227,8 @@ struct gocfd_euler2d {
     if (shock) {
       a.sh.vbuf = int(gstage & 1);
       a.sh.filter_state = a.stage == 2 ? 1 : 0;
-      for (int pass = 0; pass < dev::kShockPasses; ++pass) HIPCHECK(dev::launch_shock(N, prec, pass, a, s));
+      for (int pass = 0; pass < dev::kShockPasses; ++pass)
+        if (dev::shock_pass_runs(pass, a.stage, gstage)) HIPCHECK(dev::launch_shock(N, prec, pass, a, s));
     }
     HIPCHECK(dev::launch_stage(N, prec, shock ? 1 : 0, a, s));
   }

@@ -164,9 +164,14 @@ hipError_t launch_prologue(int N, int prec, const StageArgs &a, hipStream_t s);
 // the step sequence; stage launches write them for their new state)
 hipError_t launch_halo_export(int N, int prec, const StageArgs &a, hipStream_t s);
 // Shock-capturing passes of one stage: 0 sensor + vertex max, 1 element
-// fields (+ stage-state filter, active-element list), 2 wave speeds,
-// 3 eps * gradient of the active elements.
+// fields (+ stage-state filter, active-element list, viscous speeds), 2 wave
+// speeds (of a stage input that no stage kernel measured), 3 eps * gradient of
+// the active elements.
 constexpr int kShockPasses = 4;
+// gstage: stages since the restart
+inline bool shock_pass_runs(int pass, int stage, long long gstage) {
+  return pass != 2 || stage == 2 || (stage >= 0 && gstage == 0);
+}
 hipError_t launch_shock(int N, int prec, int pass, const StageArgs &a, hipStream_t s);
 hipError_t launch_ctl_init(Ctl *ctl, double time, hipStream_t s, int ncases = 1);
 hipError_t launch_fill_u64(unsigned long long *p, size_t n, unsigned long long v, hipStream_t s);

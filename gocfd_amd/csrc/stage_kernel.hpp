@@ -299,10 +299,10 @@ __device__ __forceinline__ double point_speed(double g, const double q[4], doubl
 // NpEdge Hmax] (rows of kTP elements; rounded to 32 bytes; before the traces
 // it holds the tile state of the VALU path for the interior flux), the Riemann
 // items' geometry [Fmax][4] and the elements' metric terms [6][kTile];
-// without shock capturing, phase G's lists: the elements' 1/hK [kTile]
-// (FP64), the owned faces [Wmax] and the export items with their
-// destinations [2][Xmax] (ints; WXints = Wmax + 2 Xmax); local time stepping adds the
-// element dt and face-speed buffers.
+// phase G's lists: the elements' 1/hK [kTile] (FP64), the owned faces [Wmax]
+// and without shock capturing the export items with their destinations
+// [2][Xmax] (ints; WXints = Wmax + 2 Xmax, or Wmax); local time stepping adds
+// the element dt and face-speed buffers.
 template <int N>
 __host__ __device__ constexpr size_t lds_trace_bytes(size_t csize, int Hmax) {
   static_assert(4 * Shape<N>::NF * kTP >= Shape<N>::NV * kTile, "the state fits the trace buffer");
@@ -453,14 +453,14 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   // the Riemann items' geometry and the metric terms (Jdet, Jinv[4], -1/Jdet)
   V4 *sFG = reinterpret_cast<V4 *>(smem_raw + lds_trace_bytes<N>(sizeof(C), HX ? 0 : a.Hmax));  // [Fmax]
   C *sJ = reinterpret_cast<C *>(sFG + a.Fmax);                                                 // [6][E]
-  // phase G's lists (without shock capturing)
+  // phase G's lists (the export items without shock capturing)
   double *sOK = reinterpret_cast<double *>(sJ + 6 * E);  // [E] 1/hK
   int *sWP = reinterpret_cast<int *>(sOK + E);           // [Wmax] owned faces e | f << 8
   int *sXP = sWP + a.Wmax, *sXD = sXP + a.Xmax;          // [Xmax] export items, destinations
   // local time stepping only: element dt and per-face speed maxima, after
   // the tile buffers (the launch adds their bytes only when LTS is on)
   double *sDT = reinterpret_cast<double *>(
-      smem_raw + lds_tile_bytes<N>(sizeof(C), HX ? 0 : a.Hmax, a.Fmax, HX ? a.Wmax + 2 * a.Xmax : 0));
+      smem_raw + lds_tile_bytes<N>(sizeof(C), HX ? 0 : a.Hmax, a.Fmax, HX ? a.Wmax + 2 * a.Xmax : a.Wmax));
   unsigned long long *sWf = reinterpret_cast<unsigned long long *>(sDT + kTile);
   __shared__ double red[kThreads / 64];
 
@@ -494,20 +494,20 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     if (c == 0) jm1 = a.g.Jinv[3 * size_t(Kp) + k0 + e];
   }
   // phase G's lists (owned faces, 1/hK; export items)
-  const int nwc = HX ? a.g.wave_cnt[tile] : 0, nxc = HX ? a.g.xp_cnt[tile] : 0;
+  const int nwc = a.g.wave_cnt[tile], nxc = HX ? a.g.xp_cnt[tile] : 0;
   int gw = 0, gx = 0, gd = 0;
   double gok = 0.;
+  if (tid < a.Wmax) gw = a.g.wave_list[size_t(tile) * a.Wmax + tid];
+  if (tid < E) gok = a.g.oohK[k0 + tid];
   if constexpr (HX) {
-    if (tid < a.Wmax) gw = a.g.wave_list[size_t(tile) * a.Wmax + tid];
     if (tid < a.Xmax) {
       gx = a.g.xp_list[size_t(tile) * a.Xmax + tid];
       gd = a.g.xp_dst[size_t(tile) * a.Xmax + tid];
     }
-    if (tid < E) gok = a.g.oohK[k0 + tid];
   }
   // boundary faces: their loops run only if any
   const int bnd0 = a.g.bnd_ptr[tile], nbnd = a.g.bnd_ptr[tile + 1] - bnd0;
-  const int nbst = SHOCK ? 0 : a.g.bst_cnt[tile];
+  const int nbst = a.g.bst_cnt[tile];
   int hk0 = -1, hf0 = 0;
   if (!HX && tid < a.Hmax * 4) {
     const int h = tid % a.Hmax;
@@ -584,13 +584,13 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     for (int i = 0; i < NpInt; ++i) sQ[(tn * NpInt + i) * E + te] = q[i];
   }
   if (tid < a.Fmax) sFG[tid] = fgv;
+  if (tid < a.Wmax) sWP[tid] = gw;
+  if (tid < E) sOK[tid] = gok;
   if constexpr (HX) {
-    if (tid < a.Wmax) sWP[tid] = gw;
     if (tid < a.Xmax) {
       sXP[tid] = gx;
       sXD[tid] = gd;
     }
-    if (tid < E) sOK[tid] = gok;
   }
   {
     const int c = tid / E, e = tid - c * E;
@@ -1164,9 +1164,12 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
   }
   const double tnext = LAST ? time + dt : time;
   double wl = 0.0;
-  if constexpr (!SHOCK) {
-    // With shock capturing the next stage state may be filtered before its
-    // traces are taken, so its wave speeds come from the gradient pass.
+  // With shock capturing the input of stage 2 is filtered before its traces are
+  // taken, so its wave speeds come from a pass after the filter. (Every stage's
+  // came from that pass: 26 us of a stage's 150 at order 2, 249,386 elements;
+  // here they add 12.)
+  const bool waves = !SHOCK || stage != 1;
+  if (waves) {
     if (lts && tid < 3 * E) sWf[tid] = 0ull;
     __syncthreads();
 
@@ -1223,6 +1226,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
       wl = fmax(wl, wsp);
       if (lts) atomicMax(&sWf[e * 3 + f], bits(wsp));
     }
+    if constexpr (HX) {
     V4 *hout = static_cast<V4 *>(a.ht) + size_t(l.hpar ^ 1) * a.ntiles * a.Fmax * NpEdge;
 #pragma unroll
     for (int j = 0; j < ITG; ++j) {
@@ -1235,11 +1239,12 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
             V4{sT[p * kTP + e], sT[TS + p * kTP + e], sT[2 * TS + p * kTP + e], sT[3 * TS + p * kTP + e]};
       }
     }
+    }
   }
   wl = wave_max(wl);
   if ((tid & 63) == 0) red[tid >> 6] = wl;
   bad = __syncthreads_or(bad);
-  if constexpr (!SHOCK) {
+  if (waves) {
     if (lts) {
       double *fw = a.lts.fw + size_t(l.par2 ^ 1) * 3 * Kp;
       const int *wlist = a.g.wave_list + size_t(tile) * a.Wmax;
@@ -1256,7 +1261,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     }
   }
   if (tid == 0) {
-    if constexpr (!SHOCK) {
+    if (waves) {
       double m = red[0];
       for (int w = 1; w < kThreads / 64; ++w) m = fmax(m, red[w]);
       atomic_max_bits(&ctl->wmax[(l.ring + 1) % 3], m);
@@ -1454,12 +1459,13 @@ __global__ void __launch_bounds__(256) k_shock_sensor(StageArgs a) {
 // Pass 1: sigma = mean of the vertex maxima (MergeVertexScalarToElement),
 // eps at the RT points by barycentric interpolation of the vertex maxima
 // (InterpolateEpsilonSigma dissipation.go:219-242), the modal filter of the
-// stage state at rkStep 2 (euler.go:603-608), and clearing of the other
+// stage state at rkStep 2 (euler.go:603-608), the owned faces' viscous speeds
+// eps/hK^2 (StoreEdgeAggregates edges.go:246-289), and clearing of the other
 // vertex buffer for the next stage. One thread per element (padded range).
 template <int N, class SIN>
 __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
   using Sh = Shape<N>;
-  constexpr int NpInt = Sh::NpInt, NV = Sh::NV, NR = Sh::NR;
+  constexpr int NpInt = Sh::NpInt, NpEdge = Sh::NpEdge, NV = Sh::NV, NR = Sh::NR;
   const int gid = blockIdx.x * blockDim.x + threadIdx.x;
   {
     unsigned long long *so = a.sh.sigV + size_t(a.sh.vbuf ^ 1) * a.sh.Nv;
@@ -1474,21 +1480,19 @@ __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
   // the element's vertices go out first, under the chain element -> case ->
   // control block of the skip check (kk < Kp keeps them in bounds)
   const int v0 = a.sh.evert[kk], v1 = a.sh.evert[size_t(a.Kp) + kk], v2 = a.sh.evert[2 * size_t(a.Kp) + kk];
+  const int code[3] = {a.g.code[kk], a.g.code[size_t(a.Kp) + kk], a.g.code[2 * size_t(a.Kp) + kk]};
+  const double oohK = a.g.oohK[kk];
   const int cs = a.tile_case[kk / kTile];
   const CaseInfo &ci = a.cases[cs];
   if (step_skipped(a, a.ctl + cs, ci.ph.final_time)) return;
   double *epsF = a.sh.epsF + kk;  // [NR][Kp]
-  if (kk >= ci.k_end) {  // padding
-    a.sh.sigma[kk] = 0.;
-    a.sh.active[kk] = 0;
-    return;
-  }
+  const bool real = kk < ci.k_end;  // else padding
   const unsigned long long *sv = a.sh.sigV + size_t(a.sh.vbuf) * a.sh.Nv;
   const unsigned long long *ev = a.sh.epsV + size_t(a.sh.vbuf) * a.sh.Nv;
-  const double sg = ((from_bits(sv[v0]) + from_bits(sv[v1])) + from_bits(sv[v2])) / 3.;
+  const double sg = real ? ((from_bits(sv[v0]) + from_bits(sv[v1])) + from_bits(sv[v2])) / 3. : 0.;
   a.sh.sigma[kk] = sg;
   const double e0 = from_bits(ev[v0]), e1 = from_bits(ev[v1]), e2 = from_bits(ev[v2]);
-  const bool act = e0 > 0. || e1 > 0. || e2 > 0.;
+  const bool act = real && (e0 > 0. || e1 > 0. || e2 > 0.);
   a.sh.active[kk] = act ? 1 : 0;
   {
     // append to the active-element list: one atomic per wave
@@ -1503,12 +1507,30 @@ __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
   }
   // an inactive element's eps is zero at every RT point; readers check the
   // flag instead of reading epsF
+  double fv[3] = {0., 0., 0.};  // the faces' largest eps
   if (act) {
     ConstD *B = shock_ops_c(a.sh) + Sh::oBary;
 #pragma unroll
-    for (int r = 0; r < NR; ++r) epsF[size_t(r) * a.Kp] = B[3 * r] * e0 + B[3 * r + 1] * e1 + B[3 * r + 2] * e2;
+    for (int r = 0; r < NR; ++r) {
+      const double e = B[3 * r] * e0 + B[3 * r + 1] * e1 + B[3 * r + 2] * e2;
+      epsF[size_t(r) * a.Kp] = e;
+      if (r >= NpInt) fv[(r - NpInt) / NpEdge] = fmax(fv[(r - NpInt) / NpEdge], e);
+    }
   }
-  if (a.sh.filter_state) {
+  if (a.stage >= 0 && (__ballot(act) || a.lts.on)) {
+    double wv = 0.;
+#pragma unroll
+    for (int f = 0; f < 3; ++f) {
+      if (real && (code[f] & FC_WAVE)) {
+        const double v = oohK * oohK * fv[f];
+        if (a.lts.on) a.lts.fwv[(size_t(a.par2) * 3 + f) * a.Kp + kk] = v;
+        wv = fmax(wv, v);
+      }
+    }
+    wv = wave_max(wv);  // a wave's elements belong to one tile, so to one case
+    if ((threadIdx.x & 63) == 0 && wv > 0.) atomic_max_bits(&a.ctl[cs].wmaxv[a.ring], wv);
+  }
+  if (a.sh.filter_state && real) {
     ConstD *V = shock_ops_c(a.sh) + Sh::oV, *Vi = shock_ops_c(a.sh) + Sh::oVi, *mf = shock_ops_c(a.sh) + Sh::omf;
     const double fac = 1. - sin(0.5 * M_PI * sg);
     SIN *q = static_cast<SIN *>(a.qs) + state_at(kk, 0, NV);
@@ -1534,8 +1556,9 @@ __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
   }
 }
 
-// Pass 2: the stage's owner-side wave speeds (|U|+c)/hK and viscous speeds
-// eps/hK^2 (StoreEdgeAggregates edges.go:246-289) from the own traces, one
+// Pass 2: the owner-side wave speeds (|U|+c)/hK (StoreEdgeAggregates
+// edges.go:246-289) of a stage input that no stage kernel measured: the
+// filtered one of stage 2, and a restart's first. From the own traces, one
 // tile of 64 elements x 4 variables per workgroup.
 template <int N, class SIN, class D>
 __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
@@ -1543,13 +1566,12 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   constexpr int NpInt = Sh::NpInt, NpEdge = Sh::NpEdge, NpFlux = Sh::NpFlux, NF = Sh::NF, NV = Sh::NV,
                 E = kTile;
   __shared__ D sTr[4 * NF * E];  // the traces [4][NF][E]
-  __shared__ double red[2][kThreads / 64];
+  __shared__ double red[kThreads / 64];
   const int tile = blockIdx.x, tid = threadIdx.x;
   const int te = tid % E, tn = tid / E, k0 = tile * E, Kp = a.Kp;
   const SIN *Q = static_cast<const SIN *>(a.qs);
   const D *Itp = Tabs<N, D>::ops() + NpFlux * NpInt;
-  // The tile's state and the owned faces' codes, 1/hK and active flags do
-  // not depend on the control block (every tile lies inside the padded
+  // The tile's state and the owned faces' codes and 1/hK do not depend on the control block (every tile lies inside the padded
   // range): their loads go out first, under the chain tile -> case ->
   // control block of the skip check.
   D u[NpInt];
@@ -1558,11 +1580,9 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   const int we = tid / 3, wf = tid - 3 * we;  // (element, face) of the wave-speed threads
   int wcode = 0;
   double woohK = 0.0;
-  bool wact = false;
   if (tid < 3 * E) {
     wcode = a.g.code[size_t(wf) * Kp + k0 + we];
     woohK = a.g.oohK[k0 + we];
-    wact = a.sh.active[k0 + we] != 0;
   }
   // the tile's case (a batch holds several, each with its own control)
   const int cs = a.tile_case[tile];
@@ -1578,7 +1598,7 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   }
   __syncthreads();
   // wave speeds of the owned faces: thread (element, face)
-  double wl = 0.0, wv = 0.0;
+  double wl = 0.0;
   int bad = 0;
   const double time = ctl->time[a.step_index & 1];
   if (tid < 3 * E) {
@@ -1588,9 +1608,7 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
     if (k < ci.k_end && (code & FC_WAVE)) {
       const int kind = code & 15;
       const double oohK = woohK;
-      const bool actk = wact;  // else eps = 0 on the face
-      const double *ef = a.sh.epsF + size_t(NpInt + f * NpEdge) * Kp + k;
-      double fwl = 0.0, fwv = 0.0;
+      double fwl = 0.0;
       for (int pp = 0; pp < NpEdge; ++pp) {
         const int p = f * NpEdge + pp;
         double q[4] = {double(sTr[(0 * NF + p) * E + e]), double(sTr[(1 * NF + p) * E + e]),
@@ -1602,31 +1620,18 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
         const double sp = point_speed(ci.ph.gamma, q, oohK);
         if (!(sp == sp)) bad = 1;
         fwl = fmax(fwl, sp);
-        if (actk) fwv = fmax(fwv, oohK * oohK * ef[size_t(pp) * Kp]);
       }
-      if (a.lts.on) {
-        a.lts.fw[size_t(a.par2) * 3 * Kp + fi] = fwl;
-        a.lts.fwv[size_t(a.par2) * 3 * Kp + fi] = fwv;
-      }
+      if (a.lts.on) a.lts.fw[size_t(a.par2) * 3 * Kp + fi] = fwl;
       wl = fwl;
-      wv = fwv;
     }
   }
   wl = wave_max(wl);
-  wv = wave_max(wv);
-  if ((tid & 63) == 0) {
-    red[0][tid >> 6] = wl;
-    red[1][tid >> 6] = wv;
-  }
+  if ((tid & 63) == 0) red[tid >> 6] = wl;
   bad = __syncthreads_or(bad);
   if (tid == 0) {
-    double m = red[0][0], mv = red[1][0];
-    for (int w = 1; w < kThreads / 64; ++w) {
-      m = fmax(m, red[0][w]);
-      mv = fmax(mv, red[1][w]);
-    }
+    double m = red[0];
+    for (int w = 1; w < kThreads / 64; ++w) m = fmax(m, red[w]);
     atomic_max_bits(&ctl->wmax[a.ring], m);
-    atomic_max_bits(&ctl->wmaxv[a.ring], mv);
     if (bad) atomicOr(&ctl->nan, 1);
   }
 }
@@ -1766,8 +1771,8 @@ size_t lds_bytes_n(size_t csize, int Hmax, int Fmax, int WXints, bool lts) {
 template <int N, class S, class SIN, class C, int FLUX, bool LAST, bool SHOCK, bool GEN>
 hipError_t launch_stage_t(const StageArgs &a, hipStream_t s) {
   // one thread stages each list item into LDS
-  if (a.Fmax > kThreads || (!SHOCK && (a.Wmax > kThreads || a.Xmax > kThreads))) return hipErrorInvalidValue;
-  const size_t lds = lds_bytes_n<N>(sizeof(C), SHOCK ? a.Hmax : 0, a.Fmax, SHOCK ? 0 : a.Wmax + 2 * a.Xmax,
+  if (a.Fmax > kThreads || a.Wmax > kThreads || (!SHOCK && a.Xmax > kThreads)) return hipErrorInvalidValue;
+  const size_t lds = lds_bytes_n<N>(sizeof(C), SHOCK ? a.Hmax : 0, a.Fmax, SHOCK ? a.Wmax : a.Wmax + 2 * a.Xmax,
                                     a.lts.on != 0);
   static size_t attr_bytes = 0;  // dynamic LDS the kernel is currently allowed
   if (lds > 64 * 1024 && lds > attr_bytes) {
