@@ -276,7 +276,6 @@ struct gocfd_ensemble {
         hipStream_t st = branches ? g->stream : stream;
         if (g->shock) {
           a.sh.vbuf = int(gstage & 1);
-          a.sh.filter_state = s == 2 ? 1 : 0;
           for (int pass = 0; pass < dev::kShockPasses; ++pass)
             if (dev::shock_pass_runs(pass, s, gstage)) HIPCHECK(dev::launch_shock(g->N, prec, pass, a, st));
         }

@@ -226,7 +226,6 @@ struct gocfd_euler2d {
     if (!s) s = stream;
     if (shock) {
       a.sh.vbuf = int(gstage & 1);
-      a.sh.filter_state = a.stage == 2 ? 1 : 0;
       for (int pass = 0; pass < dev::kShockPasses; ++pass)
         if (dev::shock_pass_runs(pass, a.stage, gstage)) HIPCHECK(dev::launch_shock(N, prec, pass, a, s));
     }

@@ -122,7 +122,6 @@ struct ShockArgs {
   const double *Nxo, *Nyo;           // [3][Kp] own outward normals
   const double *vooL;                // [3][Kp] 1 / owner edge length (shared faces)
   double kappa, eps0, cdiff, omega;
-  int filter_state;                  // filter the stage state (rkStep == 2)
 };
 
 struct StageArgs {
@@ -164,9 +163,9 @@ hipError_t launch_prologue(int N, int prec, const StageArgs &a, hipStream_t s);
 // the step sequence; stage launches write them for their new state)
 hipError_t launch_halo_export(int N, int prec, const StageArgs &a, hipStream_t s);
 // Shock-capturing passes of one stage: 0 sensor + vertex max, 1 element
-// fields (+ stage-state filter, active-element list, viscous speeds), 2 wave
-// speeds (of a stage input that no stage kernel measured), 3 eps * gradient of
-// the active elements.
+// fields (+ active-element list, viscous speeds), 2 wave speeds (of a stage
+// input that no stage kernel measured; stage 2's state filter first), 3 eps *
+// gradient of the active elements.
 constexpr int kShockPasses = 4;
 // gstage: stages since the restart
 inline bool shock_pass_runs(int pass, int stage, long long gstage) {

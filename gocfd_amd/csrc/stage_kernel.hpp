@@ -1458,8 +1458,7 @@ __global__ void __launch_bounds__(256) k_shock_sensor(StageArgs a) {
 
 // Pass 1: sigma = mean of the vertex maxima (MergeVertexScalarToElement),
 // eps at the RT points by barycentric interpolation of the vertex maxima
-// (InterpolateEpsilonSigma dissipation.go:219-242), the modal filter of the
-// stage state at rkStep 2 (euler.go:603-608), the owned faces' viscous speeds
+// (InterpolateEpsilonSigma dissipation.go:219-242), the owned faces' viscous speeds
 // eps/hK^2 (StoreEdgeAggregates edges.go:246-289), and clearing of the other
 // vertex buffer for the next stage. One thread per element (padded range).
 template <int N, class SIN>
@@ -1530,36 +1529,18 @@ __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
     wv = wave_max(wv);  // a wave's elements belong to one tile, so to one case
     if ((threadIdx.x & 63) == 0 && wv > 0.) atomic_max_bits(&a.ctl[cs].wmaxv[a.ring], wv);
   }
-  if (a.sh.filter_state && real) {
-    ConstD *V = shock_ops_c(a.sh) + Sh::oV, *Vi = shock_ops_c(a.sh) + Sh::oVi, *mf = shock_ops_c(a.sh) + Sh::omf;
-    const double fac = 1. - sin(0.5 * M_PI * sg);
-    SIN *q = static_cast<SIN *>(a.qs) + state_at(kk, 0, NV);
-    for (int n = 0; n < 4; ++n) {
-      double u[NpInt], m[NpInt];
-#pragma unroll
-      for (int i = 0; i < NpInt; ++i) u[i] = q[(n * NpInt + i) * kTile];
-#pragma unroll
-      for (int i = 0; i < NpInt; ++i) {
-        double t = 0;
-#pragma unroll
-        for (int j = 0; j < NpInt; ++j) t += Vi[i * NpInt + j] * u[j];
-        m[i] = i == 0 ? t : t * (mf[i] * fac);
-      }
-#pragma unroll
-      for (int i = 0; i < NpInt; ++i) {
-        double t = 0;
-#pragma unroll
-        for (int j = 0; j < NpInt; ++j) t += V[i * NpInt + j] * m[j];
-        q[(n * NpInt + i) * kTile] = SIN(t);
-      }
-    }
-  }
 }
 
 // Pass 2: the owner-side wave speeds (|U|+c)/hK (StoreEdgeAggregates
 // edges.go:246-289) of a stage input that no stage kernel measured: the
-// filtered one of stage 2, and a restart's first. From the own traces, one
-// tile of 64 elements x 4 variables per workgroup.
+// filtered one of stage 2, whose modal filter (rkStep 2, euler.go:603-608)
+// runs here first, and a restart's first. From the own traces, one tile of 64
+// elements x 4 variables per workgroup. (In pass 1 the filter ran the four
+// variables one after another in a thread per element, and its matrices'
+// scalar registers, 400 spilled at order 3, slowed the pass at every stage:
+// pass 1 12.1 -> 7.2 us of every stage at order 3 in FP32, 40,000 elements, and
+// 11.1 -> 8.7 at order 2 in FP64, 249,386; this pass 9.6 -> 12.6 and 23.6 ->
+// 32.0 of stage 2.)
 template <int N, class SIN, class D>
 __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   using Sh = Shape<N>;
@@ -1569,14 +1550,16 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   __shared__ double red[kThreads / 64];
   const int tile = blockIdx.x, tid = threadIdx.x;
   const int te = tid % E, tn = tid / E, k0 = tile * E, Kp = a.Kp;
-  const SIN *Q = static_cast<const SIN *>(a.qs);
+  SIN *Q = static_cast<SIN *>(a.qs) + size_t(k0) * NV + size_t(tn * NpInt) * E + te;  // the thread's values, E apart
   const D *Itp = Tabs<N, D>::ops() + NpFlux * NpInt;
   // The tile's state and the owned faces' codes and 1/hK do not depend on the control block (every tile lies inside the padded
   // range): their loads go out first, under the chain tile -> case ->
   // control block of the skip check.
+  SIN v[NpInt];
   D u[NpInt];
 #pragma unroll
-  for (int i = 0; i < NpInt; ++i) u[i] = D(Q[size_t(k0) * NV + size_t(tn * NpInt + i) * E + te]);
+  for (int i = 0; i < NpInt; ++i) v[i] = Q[i * E];
+  const double sg = a.sh.sigma[k0 + te];
   const int we = tid / 3, wf = tid - 3 * we;  // (element, face) of the wave-speed threads
   int wcode = 0;
   double woohK = 0.0;
@@ -1589,6 +1572,28 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   const CaseInfo &ci = a.cases[cs];
   Ctl *ctl = a.ctl + cs;
   if (a.stage < 0 || step_skipped(a, ctl, ci.ph.final_time)) return;
+  if (a.stage == 2 && k0 + te < ci.k_end) {
+    ConstD *V = shock_ops_c(a.sh) + Sh::oV, *Vi = shock_ops_c(a.sh) + Sh::oVi, *mf = shock_ops_c(a.sh) + Sh::omf;
+    const double fac = 1. - sin(0.5 * M_PI * sg);
+    double m[NpInt];
+#pragma unroll
+    for (int i = 0; i < NpInt; ++i) {
+      double t = 0;
+#pragma unroll
+      for (int j = 0; j < NpInt; ++j) t += Vi[i * NpInt + j] * double(v[j]);
+      m[i] = i == 0 ? t : t * (mf[i] * fac);
+    }
+#pragma unroll
+    for (int i = 0; i < NpInt; ++i) {
+      double t = 0;
+#pragma unroll
+      for (int j = 0; j < NpInt; ++j) t += V[i * NpInt + j] * m[j];
+      v[i] = SIN(t);
+      Q[i * E] = v[i];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NpInt; ++i) u[i] = D(v[i]);
 #pragma unroll
   for (int p = 0; p < NF; ++p) {
     D acc = 0;
