@@ -204,18 +204,22 @@ struct gocfd_euler2d {
 
   // Arguments of an RHS evaluation of the FP64 state qs (tile layout) into
   // out, with its halo traces in the buffer the next stage does not read
-  // (the one the last stage read); on stream s
-  dev::StageArgs rhs_args(const void *qs, double t, double *out, hipStream_t s) {
+  // (the one the last stage read); on stream s. With Q (reference layout,
+  // device memory) qs is filled from it first.
+  dev::StageArgs rhs_args(void *qs, double t, double *out, hipStream_t s, const double *Q = nullptr) {
     dev::StageArgs a = args();
     a.stage = -1;
     a.t_rhs = t;
-    a.qs = const_cast<void *>(qs);
+    a.qs = qs;
     a.rhs_out = out;
     a.ring = int(gstage % 3);
     a.par2 = int(gstage & 1);
     a.hpar = a.par2 ^ 1;
     a.step_index = step_index;
-    if (!shock) HIPCHECK(dev::launch_halo_export(prm.polynomial_order, prec, a, s));
+    double *qd = static_cast<double *>(qs);
+    if (Q && shock) HIPCHECK(dev::launch_gather_state(Q, perm.p, L.K, L.Kp, d.ops.NpInt, true, true, qd, s));
+    else if (Q) HIPCHECK(dev::launch_gather_export(prm.polynomial_order, prec, a, Q, perm.p, L.K, qd, s));
+    else if (!shock) HIPCHECK(dev::launch_halo_export(prm.polynomial_order, prec, a, s));
     return a;
   }
 

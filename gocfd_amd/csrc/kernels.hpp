@@ -26,6 +26,16 @@ __host__ __device__ constexpr size_t state_at(int kk, int r, int NV) {
   return (size_t(kk / kTile) * NV + r) * kTile + kk % kTile;
 }
 
+// Value r of an element from the reference layout [4][NpInt][K]; k = -1: a
+// padding element's, the inert state {1, 0, 0, 2.5} or zero
+__device__ __forceinline__ double gathered(const double *Q, int k, int r, int K, int NpInt, bool inert) {
+  if (k >= 0) return Q[size_t(r) * K + k];
+  return !inert ? 0.0 : r < NpInt ? 1.0 : r >= 3 * NpInt ? 2.5 : 0.0;
+}
+
+// Workgroups of 256 for n values of a state
+inline int state_grid(size_t n) { return n > 8192 * size_t(256) ? 8192 : int((n + 255) / 256); }
+
 // Device control block. Time is double-buffered by step parity and the wave
 // speed maxima live in rings of three slots indexed by the global stage
 // counter, so that no kernel writes a value another block of the same launch
@@ -162,6 +172,10 @@ hipError_t launch_prologue(int N, int prec, const StageArgs &a, hipStream_t s);
 // Halo traces of the FP64 state a.qs into buffer a.hpar (a state set outside
 // the step sequence; stage launches write them for their new state)
 hipError_t launch_halo_export(int N, int prec, const StageArgs &a, hipStream_t s);
+// launch_gather_state (tile layout, inert padding) and launch_halo_export of
+// the result, in one launch; a.qs is not read
+hipError_t launch_gather_export(int N, int prec, const StageArgs &a, const double *Q, const int *perm, int K,
+                                double *out, hipStream_t s);
 // Shock-capturing passes of one stage: 0 sensor + vertex max, 1 element
 // fields (+ active-element list, viscous speeds), 2 wave speeds (of a stage
 // input that no stage kernel measured; stage 2's state filter first), 3 eps *
@@ -220,6 +234,8 @@ hipError_t upload_operators_multi(int flux, int N, const double *divT, const dou
 template <int N> hipError_t launch_stage_n(int prec, int shock, const StageArgs &a, hipStream_t s);
 template <int N> hipError_t launch_prologue_n(int prec, const StageArgs &a, hipStream_t s);
 template <int N> hipError_t launch_halo_export_n(int prec, const StageArgs &a, hipStream_t s);
+template <int N> hipError_t launch_gather_export_n(int prec, const StageArgs &a, const double *Q, const int *perm,
+                                                   int K, double *out, hipStream_t s);
 template <int N> hipError_t launch_shock_n(int prec, int pass, const StageArgs &a, hipStream_t s);
 template <int N> hipError_t upload_operators_n(const double *divT, const double *interp);
 // Per-flux entry points of the multi-order kernels (one translation unit per flux)

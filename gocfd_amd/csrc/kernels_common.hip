@@ -36,6 +36,13 @@ hipError_t launch_halo_export(int N, int prec, const StageArgs &a, hipStream_t s
 #undef CALL
 }
 
+hipError_t launch_gather_export(int N, int prec, const StageArgs &a, const double *Q, const int *perm, int K,
+                                double *out, hipStream_t s) {
+#define CALL(n) launch_gather_export_n<n>(prec, a, Q, perm, K, out, s)
+  GOCFD_DISPATCH_ORDER(N, CALL)
+#undef CALL
+}
+
 hipError_t launch_shock(int N, int prec, int pass, const StageArgs &a, hipStream_t s) {
 #define CALL(n) launch_shock_n<n>(prec, pass, a, s)
   GOCFD_DISPATCH_ORDER(N, CALL)
@@ -126,11 +133,7 @@ __global__ void __launch_bounds__(256) k_gather_state(const double *__restrict__
   for (size_t idx = size_t(blockIdx.x) * blockDim.x + threadIdx.x; idx < n; idx += size_t(gridDim.x) * blockDim.x) {
     int kk, r;
     state_of(idx, NV, tiled, kk, r);
-    const int k = perm[kk];
-    double v = 0.0;
-    if (k >= 0) v = Q[size_t(r) * K + k];
-    else if (inert) v = r < NpInt ? 1.0 : r >= 3 * NpInt ? 2.5 : 0.0;
-    out[idx] = v;
+    out[idx] = gathered(Q, perm[kk], r, K, NpInt, inert);
   }
 }
 
@@ -154,8 +157,6 @@ __global__ void __launch_bounds__(256) k_element_major(const double *__restrict_
     out[idx] = in[state_at(kk, r, NV)];
   }
 }
-
-static int state_grid(size_t n) { return int(std::min<size_t>((n + 255) / 256, 8192)); }
 
 hipError_t launch_gather_state(const double *Q, const int *perm, int K, int Kp, int NpInt, bool tiled, bool inert,
                                double *out, hipStream_t s) {

@@ -64,8 +64,7 @@ extern "C" int gocfd_euler2d_rhs_noalloc(gocfd_euler2d *h, const double *Q, doub
   double *in = g_scratch[h->device], *out = in + vals;
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : h->stream;
   const int NpInt = h->d.ops.NpInt;
-  HIPCHECK(dev::launch_gather_state(Q, h->perm.p, h->L.K, h->L.Kp, NpInt, true, true, in, s));
-  dev::StageArgs a = h->rhs_args(in, t, out, s);
+  dev::StageArgs a = h->rhs_args(in, t, out, s, Q);
   h->launch_one_stage(a, s);
   if (h->shock) {  // the vertex buffers this evaluation used must be clear for the next stage
     HIPCHECK(dev::launch_fill_u64(h->sigV.p, h->sigV.n, 0ull, s));
