@@ -222,11 +222,21 @@ __device__ __forceinline__ bool gamma_is_14(double g) {
   return x > 2.5 - 1e-13 && x < 2.5 + 1e-13;
 }
 
+// How the powers of a boundary state are taken. Ref: as the reference writes
+// them, for solvers with FP32 stage states, where a last bit of the FP64 state
+// (or of a boundary wave speed, through dt) can move the next rounding to FP32,
+// and one moved value reaches an element further at each stage: with the other
+// forms a vortex of 12,168 elements at order 4 ended 24 steps 7e-7 away. (They
+// were faster: 100 steps of 80,000 elements at order 4 24.6 ms, 25.8 with Ref, 24
+// cases of 2,000 to 20,000 elements 11.6 and 12.3.) Pow and G14 serve FP64
+// solvers: one power, or for gamma = 1.4 (the caller has checked) none; they
+// differ from Ref by roundings.
+enum class BcForm { Ref, Pow, G14 };
+
 // RiemannBC (model_problems/Euler2D/bcs.go:70-133), in FP64 (T = double) or
 // in FP64 dual arithmetic for the tangent-linear and adjoint kernels.
 // pinf/cinf come from the freestream even for the analytic vortex state.
-// GEN: any gamma; without it gamma is 1.4 (the caller has checked).
-template <class T, class P, bool GEN = true>
+template <class T, class P, BcForm FORM = BcForm::Pow>
 __device__ __forceinline__ void riemann_bc(double g, double minf, P pinf, P cinf, const T qi[4],
                                            const T qinf[4], double nx, double ny, T qb[4]) {
   const T rhoI = qi[0], uI = qi[1] / qi[0], vI = qi[2] / qi[0];
@@ -242,26 +252,35 @@ __device__ __forceinline__ void riemann_bc(double g, double minf, P pinf, P cinf
     const T Rint = VnI + 2. * cI * OOGM1;
     const T Vn = 0.5 * (Rint + Rinf);
     const T c = 0.25 * GM1 * (Rint - Rinf);
-    // The boundary density and pressure from c and the entropy of the
-    // upwind side, p0 / rho0^g (far state on inflow, interior on outflow):
-    // rho = (c^2 / (g beta))^(1/(g-1)) with beta = p0 / rho0^g is
-    // rho0 (c^2 rho0 / (g p0))^(1/(g-1)), and beta rho^g = rho c^2 / g, so one
-    // power is left of the formula's three, and none for g = 1.4, where
-    // x^2.5 = x^2 sqrt(x).
-    T Vt, rho0, p0;
-    if (VnI < 0) { Vt = tx * uF + ty * vF; rho0 = rhoF; p0 = pinf; }
-    else { Vt = tx * uI + ty * vI; rho0 = rhoI; p0 = pI; }
-    const T u = Vn * nx + Vt * tx, v = Vn * ny + Vt * ty;
-    const T X = c * c * rho0 / (g * p0);
-    T Xp;
-    if constexpr (GEN) {
-      if (gamma_is_14(g)) Xp = X * X * sqrt(X);
-      else Xp = pow(X, OOGM1);
+    T Vt, rho, p;
+    if constexpr (FORM == BcForm::Ref) {
+      T beta;
+      if (VnI < 0) { Vt = tx * uF + ty * vF; beta = pinf / pow(rhoF, g); }
+      else { Vt = tx * uI + ty * vI; beta = pI / pow(rhoI, g); }
+      rho = pow(c * c / (g * beta), OOGM1);
+      p = beta * pow(rho, g);
     } else {
-      Xp = X * X * sqrt(X);
+      // The boundary density and pressure from c and the entropy of the
+      // upwind side, p0 / rho0^g (far state on inflow, interior on outflow):
+      // rho = (c^2 / (g beta))^(1/(g-1)) with beta = p0 / rho0^g is
+      // rho0 (c^2 rho0 / (g p0))^(1/(g-1)), and beta rho^g = rho c^2 / g, so one
+      // power is left of the formula's three, and none for g = 1.4, where
+      // x^2.5 = x^2 sqrt(x).
+      T rho0, p0;
+      if (VnI < 0) { Vt = tx * uF + ty * vF; rho0 = rhoF; p0 = pinf; }
+      else { Vt = tx * uI + ty * vI; rho0 = rhoI; p0 = pI; }
+      const T X = c * c * rho0 / (g * p0);
+      T Xp;
+      if constexpr (FORM == BcForm::Pow) {
+        if (gamma_is_14(g)) Xp = X * X * sqrt(X);
+        else Xp = pow(X, OOGM1);
+      } else {
+        Xp = X * X * sqrt(X);
+      }
+      rho = rho0 * Xp;
+      p = rho * c * c * (1. / g);
     }
-    const T rho = rho0 * Xp;
-    const T p = rho * c * c * (1. / g);
+    const T u = Vn * nx + Vt * tx, v = Vn * ny + Vt * ty;
     qb[0] = rho; qb[1] = rho * u; qb[2] = rho * v; qb[3] = p * OOGM1 + 0.5 * rho * (u * u + v * v);
   } else if (VnI < 0) {
     for (int c = 0; c < 4; ++c) qb[c] = qinf[c];
@@ -272,6 +291,7 @@ __device__ __forceinline__ void riemann_bc(double g, double minf, P pinf, P cinf
 
 // IVortex.GetStateC with beta=5, centre (5,0), gamma=1.4, Ufs=1
 // (isentropic_vortex/analytic_vortex.go:31-82, initialization.go:61-71)
+template <BcForm FORM>
 __device__ __forceinline__ void ivortex_state(double t, double x, double y, double q[4]) {
   const double beta = 5., X0 = 5., Y0 = 0., G = 1.4;
   const double oo2pi = 0.5 * (1. / M_PI), GM1 = G - 1;
@@ -280,12 +300,22 @@ __device__ __forceinline__ void ivortex_state(double t, double x, double y, doub
   const double xm = x - u * t, ym = y - v * t;
   const double r2 = (xm - X0) * (xm - X0) + (ym - Y0) * (ym - Y0);
   const double ex1r = exp(1 - r2);
-  // rho = t^(1/(G-1)) = t^2.5 and p = rho^G = rho t
-  const double tv1 = 1.0 - (GM1 * beta * beta * (ex1r * ex1r) / fac);
-  u -= beta * ex1r * (ym - Y0) * oo2pi;
-  v += beta * ex1r * (xm - X0) * oo2pi;
-  const double rho = tv1 * tv1 * sqrt(tv1);
-  const double p = rho * tv1;
+  double rho, p;
+  if constexpr (FORM == BcForm::Ref) {
+    const double OOGM1 = 1. / GM1;
+    const double tv1 = 1.0 - (GM1 * beta * beta * exp(2.0 * (1.0 - r2)) / fac);
+    u -= beta * ex1r * (ym - Y0) * oo2pi;
+    v += beta * ex1r * (xm - X0) * oo2pi;
+    rho = pow(tv1, OOGM1);
+    p = pow(rho, G);
+  } else {
+    // rho = t^(1/(G-1)) = t^2.5 and p = rho^G = rho t
+    const double tv1 = 1.0 - (GM1 * beta * beta * (ex1r * ex1r) / fac);
+    u -= beta * ex1r * (ym - Y0) * oo2pi;
+    v += beta * ex1r * (xm - X0) * oo2pi;
+    rho = tv1 * tv1 * sqrt(tv1);
+    p = rho * tv1;
+  }
   q[0] = rho; q[1] = rho * u; q[2] = rho * v;
   q[3] = p * (1. / (G - 1.)) + 0.5 * rho * (u * u + v * v);
 }

@@ -265,7 +265,7 @@ __device__ __forceinline__ void atomic_max_bits(unsigned long long *p, double v)
   if (b > *reinterpret_cast<volatile unsigned long long *>(p)) atomicMax(p, b);
 }
 
-template <bool GEN, class C>
+template <BcForm FORM, class C>
 __device__ __forceinline__ void boundary_state(int kind, const Phys &ph, const double *bxy, int bidx,
                                                int NpEdge, int pp, double t, const C own[4],
                                                double nx, double ny, double qb[4]) {
@@ -282,10 +282,15 @@ __device__ __forceinline__ void boundary_state(int kind, const Phys &ph, const d
     qf[0] = qs[0]; qf[1] = qs[1]; qf[2] = qs[2]; qf[3] = qs[3];
   } else {
     const double *xy = bxy + 2 * (size_t(bidx) * NpEdge + pp);
-    ivortex_state(t, xy[0], xy[1], qf);
+    ivortex_state<FORM>(t, xy[0], xy[1], qf);
   }
-  riemann_bc<double, double, GEN>(gam, minf, pinf, cinf, qi, qf, nx, ny, qb);
+  riemann_bc<double, double, FORM>(gam, minf, pinf, cinf, qi, qf, nx, ny, qb);
 }
+
+// The form of a solver's boundary states: S its stage-state storage, GEN a
+// gamma other than 1.4
+template <class S, bool GEN>
+constexpr BcForm kBcForm = sizeof(S) == 4 ? BcForm::Ref : GEN ? BcForm::Pow : BcForm::G14;
 
 // Wave speed (|U| + c) / hK of a face point (StoreEdgeAggregates, edges.go:264-272)
 __device__ __forceinline__ double point_speed(double g, const double q[4], double oohK) {
@@ -339,7 +344,7 @@ __device__ __forceinline__ bool step_skipped(const StageLaunch &l, const Ctl *ct
 // FP64 tile needs about 45 KB of LDS at N=4 (three workgroups per CU) and
 // fits 168 VGPRs; the FP32 stages fit 128 VGPRs without spilling. On the VALU
 // path the tile's state stays in its threads' registers: the order-2 FP64
-// stage fits 128 VGPRs and 27 KB of LDS, four workgroups per CU (with a state
+// stage fits 128 VGPRs and 34 KB of LDS, four workgroups per CU (with a state
 // buffer in LDS: 40 KB, three).
 #ifndef GOCFD_WAVES_F32
 #define GOCFD_WAVES_F32 4
@@ -355,13 +360,14 @@ __device__ __forceinline__ bool step_skipped(const StageLaunch &l, const Ctl *ct
 // vector spill stores among the lane writes at the head of the block, before
 // the exec mask is restored, so the lanes that were off (those without a
 // Riemann item) store nothing and reload garbage -- addresses among it. The
-// build's spill counts are checked by a test. GEN (a gamma other than 1.4)
-// needs the registers of pow, so it takes one wave per SIMD less; so does
-// Roe-ER at order 4 in FP64. Up to order 1 the FP32 form computes in FP64.
+// build's spill counts are checked by a test. GEN (FP64, a gamma other than
+// 1.4) needs the registers of pow, so at order 4 it takes one wave per SIMD
+// less; so does Roe-ER there. FP32 stage states always take pow (kBcForm), which
+// fits. Up to order 1 the FP32 form computes in FP64.
 template <int N, class S, int FLUX, bool LAST, bool SHOCK, bool GEN>
 struct StageWaves {
   static constexpr int value = SHOCK            ? 1
-                               : sizeof(S) == 4 && N >= 2 ? (LAST || GEN ? GOCFD_WAVES_F32_LAST : GOCFD_WAVES_F32)
+                               : sizeof(S) == 4 && N >= 2 ? (LAST ? GOCFD_WAVES_F32_LAST : GOCFD_WAVES_F32)
                                                 : (N == 4 && (GEN || FLUX == 3) ? 2 : GOCFD_WAVES_F64);
 };
 
@@ -820,7 +826,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
     C F[4] = {C(0), C(0), C(0), C(0)};
     if (kind == FK_Far || kind == FK_IVortex) {
       double qb[4];
-      boundary_state<GEN>(kind, ph, a.g.bxy, code >> 8, NpEdge, pp, time, own, nxd, nyd, qb);
+      boundary_state<kBcForm<S, GEN>>(kind, ph, a.g.bxy, code >> 8, NpEdge, pp, time, own, nxd, nyd, qb);
       const C q[4] = {C(qb[0]), C(qb[1]), C(qb[2]), C(qb[3])};
       C Fx[4], Fy[4];
       flux_xy(g, q, Fx, Fy);
@@ -1220,7 +1226,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
 #pragma unroll
       for (int c = 0; c < 4; ++c) own[c] = sT[c * TS + p * kTP + e];
       double q[4];
-      boundary_state<GEN>(code & 15, ph, a.g.bxy, code >> 8, NpEdge, pp, tnext, own, geo[0], geo[1], q);
+      boundary_state<kBcForm<S, GEN>>(code & 15, ph, a.g.bxy, code >> 8, NpEdge, pp, tnext, own, geo[0], geo[1], q);
       const double wsp = point_speed(ph.gamma, q, geo[3]);
       if (!(wsp == wsp)) bad = 1;
       wl = fmax(wl, wsp);
@@ -1298,7 +1304,7 @@ k_stage(StageArgs) {
 // address: 110 to 330 us at 80,000 to 320,000 triangles), and each face's to
 // the per-face speed buffer of local time stepping.
 constexpr int kProThreads = 3 * kTile;
-template <int N, class S>
+template <int N, BcForm FORM>
 __global__ void __launch_bounds__(kProThreads) k_prologue(StageArgs a) {
   using Sh = Shape<N>;
   constexpr int NpInt = Sh::NpInt, NpEdge = Sh::NpEdge, NV = Sh::NV;
@@ -1314,7 +1320,7 @@ __global__ void __launch_bounds__(kProThreads) k_prologue(StageArgs a) {
   double wl = 0.0;
   int bad = 0;
   if (on) {
-    const S *q = static_cast<const S *>(a.qs) + state_at(kk, 0, NV);
+    const double *q = static_cast<const double *>(a.qs) + state_at(kk, 0, NV);
     double u[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) u[i] = double(q[i * kTile]);
@@ -1331,7 +1337,7 @@ __global__ void __launch_bounds__(kProThreads) k_prologue(StageArgs a) {
       const int kind = code & 15;
       if (kind == FK_Far || kind == FK_IVortex) {
         const double own[4] = {tr[0], tr[1], tr[2], tr[3]};
-        boundary_state<true>(kind, ci.ph, a.g.bxy, code >> 8, NpEdge, pp, ctl->time[a.step_index & 1], own,
+        boundary_state<FORM>(kind, ci.ph, a.g.bxy, code >> 8, NpEdge, pp, ctl->time[a.step_index & 1], own,
                        a.g.Nx[fi], a.g.Ny[fi], tr);
       }
       const double w = point_speed(ci.ph.gamma, tr, a.g.oohK[kk]);
@@ -1570,7 +1576,7 @@ __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
 // pass 1 12.1 -> 7.2 us of every stage at order 3 in FP32, 40,000 elements, and
 // 11.1 -> 8.7 at order 2 in FP64, 249,386; this pass 9.6 -> 12.6 and 23.6 ->
 // 32.0 of stage 2.)
-template <int N, class SIN, class D>
+template <int N, class SIN, class D, BcForm FORM>
 __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
   using Sh = Shape<N>;
   constexpr int NpInt = Sh::NpInt, NpEdge = Sh::NpEdge, NpFlux = Sh::NpFlux, NF = Sh::NF, NV = Sh::NV,
@@ -1649,7 +1655,7 @@ __global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
                        double(sTr[(2 * NF + p) * E + e]), double(sTr[(3 * NF + p) * E + e])};
         if (kind == FK_Far || kind == FK_IVortex) {
           const double own[4] = {q[0], q[1], q[2], q[3]};
-          boundary_state<true>(kind, ci.ph, a.g.bxy, code >> 8, NpEdge, pp, time, own, a.g.Nx[fi], a.g.Ny[fi], q);
+          boundary_state<FORM>(kind, ci.ph, a.g.bxy, code >> 8, NpEdge, pp, time, own, a.g.Nx[fi], a.g.Ny[fi], q);
         }
         const double sp = point_speed(ci.ph.gamma, q, oohK);
         if (!(sp == sp)) bad = 1;
@@ -1829,7 +1835,9 @@ hipError_t launch_stage_l(const StageArgs &a, hipStream_t s) {
 
 template <int N, class S, class C, int FLUX, bool SHOCK>
 hipError_t launch_stage_g(const StageArgs &a, hipStream_t s) {
-  if (a.gen) return launch_stage_l<N, S, C, FLUX, SHOCK, true>(a, s);
+  // (FP32 stage states take one form of the boundary state for every gamma)
+  if constexpr (sizeof(S) == 8)
+    if (a.gen) return launch_stage_l<N, S, C, FLUX, SHOCK, true>(a, s);
   return launch_stage_l<N, S, C, FLUX, SHOCK, false>(a, s);
 }
 
@@ -1863,8 +1871,9 @@ hipError_t launch_stage_n(int prec, int shock, const StageArgs &a, hipStream_t s
 
 template <int N>
 hipError_t launch_prologue_n(int prec, const StageArgs &a, hipStream_t s) {
-  (void)prec;  // the prologue reads q0, which is FP64 in every precision
-  hipLaunchKernelGGL((k_prologue<N, double>), dim3(a.ntiles), dim3(kProThreads), 0, s, a);
+  // it reads q0, which is FP64 in every precision
+  if (prec == 0) hipLaunchKernelGGL((k_prologue<N, BcForm::Pow>), dim3(a.ntiles), dim3(kProThreads), 0, s, a);
+  else hipLaunchKernelGGL((k_prologue<N, BcForm::Ref>), dim3(a.ntiles), dim3(kProThreads), 0, s, a);
   return hipGetLastError();
 }
 
@@ -1890,7 +1899,7 @@ hipError_t launch_gather_export_n(int prec, const StageArgs &a, const double *Q,
   return hipGetLastError();
 }
 
-template <int N, class SIN, class D>
+template <int N, class SIN, class D, BcForm FORM>
 hipError_t launch_shock_t(int pass, const StageArgs &a, hipStream_t s) {
   switch (pass) {
     case 0:
@@ -1900,7 +1909,7 @@ hipError_t launch_shock_t(int pass, const StageArgs &a, hipStream_t s) {
       hipLaunchKernelGGL((k_shock_prep<N, SIN>), dim3((a.Kp + 255) / 256), dim3(256), 0, s, a);
       break;
     case 2:
-      hipLaunchKernelGGL((k_shock_grad<N, SIN, D>), dim3(a.ntiles), dim3(kThreads), 0, s, a);
+      hipLaunchKernelGGL((k_shock_grad<N, SIN, D, FORM>), dim3(a.ntiles), dim3(kThreads), 0, s, a);
       break;
     case 3:
       hipLaunchKernelGGL((k_shock_grad_act<N, SIN, D>),
@@ -1917,9 +1926,9 @@ hipError_t launch_shock_t(int pass, const StageArgs &a, hipStream_t s) {
 // evaluation, else the stage state in the precision's storage.
 template <int N>
 hipError_t launch_shock_n(int prec, int pass, const StageArgs &a, hipStream_t s) {
-  if (prec == 0) return launch_shock_t<N, double, double>(pass, a, s);
-  if (a.stage <= 0) return launch_shock_t<N, double, BulkC<N>>(pass, a, s);
-  return launch_shock_t<N, float, BulkC<N>>(pass, a, s);
+  if (prec == 0) return launch_shock_t<N, double, double, BcForm::Pow>(pass, a, s);
+  if (a.stage <= 0) return launch_shock_t<N, double, BulkC<N>, BcForm::Ref>(pass, a, s);
+  return launch_shock_t<N, float, BulkC<N>, BcForm::Ref>(pass, a, s);
 }
 
 // The order-N tables of the including translation unit (internal linkage:

@@ -1,0 +1,81 @@
+"""FP32-bulk results keep their bits from build to build: with FP32 stage
+states a last bit of an FP64 intermediate (a boundary state, the time step, a
+sum of the stage combination) can move the next rounding to FP32, and one moved
+value reaches an element further at every stage, so the roundings of these
+intermediates are part of the result. The digests were taken before
+the stage kernels were split by gamma; a case is skipped where the host's
+mathematics library gives other setup bits (operators, geometry, start)."""
+import hashlib
+
+import numpy as np
+import pytest
+
+from gocfd_amd import Euler, InputParameters2D, Mesh, meshgen
+
+pytestmark = pytest.mark.gpu
+
+
+def _quads(*size, boundary="far"):
+    def mesh(tmp):
+        VX, VY, E, tags = meshgen.jittered_quads(*size)
+        return Mesh.from_arrays(VX, VY, E, {boundary if k == "far" else k: v for k, v in tags.items()})
+    return mesh
+
+
+def _file(make, *size):
+    def mesh(tmp):
+        path = str(tmp / "m.su2")
+        make(path, *size)
+        return Mesh.read(path)
+    return mesh
+
+
+FOIL = dict(InitType="Freestream", Minf=0.5, Alpha=2.0)
+# name: (mesh, parameters, steps, relative perturbation of the start, setup digest, result digest)
+CASES = {
+    "vortex_p1_roe_er": (_quads(14, 11), dict(PolynomialOrder=1, FluxType="Roe-ER", InitType="IVortex"), 16, 0.0,
+                         "4d7500c63fc4036e", "e9746817212c8f6a"),
+    "vortex_boundary_p0": (_quads(9, 13, boundary="wall"),  # the vortex's own boundary state
+                           dict(PolynomialOrder=0, FluxType="Roe", InitType="IVortex"), 12, 0.0,
+                           "933a72f7b3a8d516", "143acdcf646faded"),
+    "airfoil_p1": (_file(meshgen.airfoil_mesh, 60, 20), dict(PolynomialOrder=1, FluxType="Lax", **FOIL), 40, 1e-3,
+                   "174f80e1167985c4", "cf84e703d26532fa"),
+    "airfoil_gamma13_p1": (_file(meshgen.airfoil_mesh, 60, 20), dict(PolynomialOrder=1, FluxType="Roe", Gamma=1.3, **FOIL), 40,
+                           1e-3, "8bf4f13b1cbe5841", "e884a4574aebf129"),
+    "airfoil_lts_p3": (_file(meshgen.airfoil_mesh, 60, 20), dict(PolynomialOrder=3, FluxType="Roe", LocalTimeStepping=True,
+                                                                **FOIL), 40, 1e-3, "73c51fbcfce60215", "52e9cb3152163d19"),
+    "airfoil_shock_p1": (_file(meshgen.airfoil_mesh, 60, 20), dict(PolynomialOrder=1, FluxType="Roe", InitType="Freestream",
+                                                                  Minf=0.8, Alpha=1.0, Limiter="PerssonC0", Kappa=3.0), 40, 0.0,
+                         "d80ef4be69d18bd1", "c167d75e114cadd9"),
+}
+
+
+def _digest(*arrays):
+    h = hashlib.sha256()
+    for a in arrays:
+        h.update(np.ascontiguousarray(a, dtype=np.float64).tobytes())
+    return h.hexdigest()[:16]
+
+
+def run_case(name, tmp):
+    """(setup digest, result digest): the state, the time and, with local time stepping, the element time steps."""
+    mesh, kw, steps, noise = CASES[name][:4]
+    e = Euler(InputParameters2D(CFL=0.5, FinalTime=1e9, **kw), mesh(tmp), precision="fp32")
+    q = e.Q
+    o, g = e.operators(), e.geometry()
+    setup = _digest(q, *[o[k] for k in sorted(o)], *[g[k] for k in sorted(g)])
+    if noise:
+        e.Q = q * (1.0 + noise * np.random.default_rng(5).standard_normal(q.shape))
+    e.step(steps)
+    out = [e.Q, np.array([e.time_info()[0]])]
+    if kw.get("LocalTimeStepping"):
+        out.append(e.element_dt())
+    return setup, _digest(*out)
+
+
+@pytest.mark.parametrize("name", CASES)
+def test_fp32_results_keep_their_bits(tmp_path, name):
+    setup, result = run_case(name, tmp_path)
+    if setup != CASES[name][4]:
+        pytest.skip("the host's mathematics library rounds the setup differently")
+    assert result == CASES[name][5]
