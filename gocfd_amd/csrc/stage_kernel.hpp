@@ -396,9 +396,12 @@ __device__ __forceinline__ double ssp_last_f32(bool split, double q0, double q2,
   return fma(0.226007483236906, dtR, r);
 }
 
-// Stages 0..3 (euler.go:511-545): c dt RHS + (a q0 + round(b q_s)), roundings
-// pinned for the same reason. The coefficients are chosen once per stage: a
-// branch on the stage at every value cost as many instructions as the sum.
+// Stages 0..3 (euler.go:511-545): a q0 + b q_s + c dt RHS, roundings pinned for
+// the same reason: c dt RHS is added last, fused; of the other two products the
+// VALU path rounds b q_s, the matrix-core path a q0. (With b q_s rounded there
+// too, one case of 24 in an FP32 ensemble ended 24 steps 5e-8 away.) The
+// coefficients are chosen once per stage: a branch on the stage at every value
+// cost as many instructions as the sum.
 struct SspCoef {
   double a, b, c;
 };
@@ -410,9 +413,10 @@ __device__ __forceinline__ SspCoef ssp_coef(int stage) {
     default: return {0.178079954393132, 0.821920045606868, 0.544974750228521};
   }
 }
+template <bool MF>
 __device__ __forceinline__ double ssp_mid(const SspCoef &k, double q0, double qs, double dtR) {
 #pragma clang fp contract(off)
-  return fma(k.c, dtR, fma(k.a, q0, k.b * qs));
+  return fma(k.c, dtR, MF ? fma(k.b, qs, k.a * q0) : fma(k.a, q0, k.b * qs));
 }
 
 // What bounds it and why this layout. With element-major tiles (an element's
@@ -1094,7 +1098,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
 #pragma unroll
           for (int j = 0; j < KI; ++j) {
             rh[j] = double(rq[c][j]);
-            nv[j] = S(ssp_mid(k, m0[c][j], double(qv[c][j]), dte * rh[j]));
+            nv[j] = S(ssp_mid<MF>(k, m0[c][j], double(qv[c][j]), dte * rh[j]));
             if (MS::point(krow, j) < NpInt) {
               qv[c][j] = C(nv[j]);
               if (real && !(nv[j] == nv[j])) bad = 1;
@@ -1158,7 +1162,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
             q[i] = C(nv);
             if (real && !(nv == nv)) bad = 1;
           } else {
-            const S nv = S(ssp_mid(k, c0[j], qsv, dtR));
+            const S nv = S(ssp_mid<MF>(k, c0[j], qsv, dtR));
             if (stage == 3) Rr[i * E] = rhs;
             qn[i * E] = nv;
             q[i] = C(nv);
