@@ -1,5 +1,6 @@
 // Host driver of the tangent-linear and discrete-adjoint step.
 #include "adjoint_runner.hpp"
+#include "adjoint_budget.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -394,11 +395,10 @@ void AdjointRunner::vjp(const double *q0, double t0, int nsteps, int every, cons
   // checkpoints into the first kept block's states, whose own steps are then
   // done with; if not even one block fits, each step's record is recomputed
   // from its start just before its transposed stages.
-  const size_t per_block = 10 * size_t(every_), have = states_.size();
   size_t free_b = 0, total_b = 0;
   HIPCHECK(hipMemGetInfo(&free_b, &total_b));
-  const size_t room = have + (free_b / 4) / bytes, fixed = size_t(nblocks + 1 + every_);
-  int kept = room > fixed ? int(std::min<size_t>(size_t(every > 0 ? 1 : nblocks), (room - fixed) / per_block)) : 0;
+  int kept = kept_blocks(free_b, states_.size() * bytes, size_t(nblocks + 1 + every_) * bytes, 10 * size_t(every_) * bytes,
+                         every > 0 ? 1 : nblocks);
   // GOCFD_ADJOINT_KEEP_RECORDS=0 forces the per-step recomputation
   if (const char *e = std::getenv("GOCFD_ADJOINT_KEEP_RECORDS"))
     if (e[0] == '0') kept = 0;
