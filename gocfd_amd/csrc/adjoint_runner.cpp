@@ -112,10 +112,10 @@ AdjointRunner::AdjointRunner(const Discretisation &d, const DeviceLayout &L, con
   FE_.alloc(4 * nfp_);
   if (lts) SP_.alloc(nfp_);
   tmp_.alloc(n_);
-  dts_.alloc(5);
-  argmax_.alloc(5);
+  scratch_small_.dts.alloc(5);
+  scratch_small_.argmax.alloc(5);
+  scratch_small_.Wv.alloc(5);
   flag_.alloc(1);
-  Wv_.alloc(5);
   time_.alloc(1);
   part_v_.alloc(4 * size_t(nparts_));
   part_t_.alloc((nfp_ + 255) / 256);
@@ -156,39 +156,29 @@ AdjointRunner::AdjointRunner(const Discretisation &d, const DeviceLayout &L, con
   }
 }
 
-double *AdjointRunner::state(size_t i) {
-  while (states_.size() <= i) {
-    states_.push_back(std::make_unique<DevBuf<double>>());
-    states_.back()->alloc(n_);
-  }
-  return states_[i]->p;
+// Buffers for `kept` blocks of records and the checkpoints; false when the
+// device has no room for them (what fitted stays for a smaller try)
+bool AdjointRunner::reserve(size_t nstates, size_t nsteps) {
+  const size_t Kp = size_t(a_.Kp), lts = a_.lts ? 5 * Kp : 0;
+  // GOCFD_TEST_RECORD_STEPS: records of more steps are refused as if the
+  // device had no memory for them
+  if (const char *e = std::getenv("GOCFD_TEST_RECORD_STEPS"))
+    if (long(nsteps) > std::atol(e)) return false;
+  return grow(ckpt_, nstates * n_) && grow(rec_, 10 * nsteps * n_) && grow(small_.dts, 5 * nsteps) &&
+         grow(small_.argmax, 5 * nsteps) && grow(small_.Wv, 5 * nsteps) && grow(small_.dtk, lts * nsteps) &&
+         grow(small_.srck, lts * nsteps) && grow(small_.wk, lts * nsteps);
 }
 
-AdjointRunner::SmallRecord &AdjointRunner::small(size_t i) {
-  while (smalls_.size() <= i) {
-    smalls_.push_back(std::make_unique<SmallRecord>());
-    SmallRecord &sm = *smalls_.back();
-    sm.dts.alloc(5);
-    sm.argmax.alloc(5);
-    sm.Wv.alloc(5);
-    if (a_.lts) {
-      sm.dtk.alloc(5 * size_t(a_.Kp));
-      sm.srck.alloc(5 * size_t(a_.Kp));
-      sm.wk.alloc(5 * size_t(a_.Kp));
-    }
-  }
-  return *smalls_[i];
-}
-
-void AdjointRunner::fill_small(StageRecord &r, SmallRecord &sm) {
-  r.dts = sm.dts.p;
-  r.argmax = sm.argmax.p;
-  r.Wv = sm.Wv.p;
+// step: the record's place in the arrays
+void AdjointRunner::fill_small(StageRecord &r, SmallRecord &sm, size_t step) {
+  r.dts = sm.dts.p + 5 * step;
+  r.argmax = sm.argmax.p + 5 * step;
+  r.Wv = sm.Wv.p + 5 * step;
   for (int s = 0; s < 5; ++s) {
-    const size_t o = size_t(s) * a_.Kp;
-    r.dtk[s] = sm.dtk.p ? static_cast<void *>(sm.dtk.p + o) : nullptr;
-    r.srck[s] = sm.srck.p ? sm.srck.p + o : nullptr;
-    r.wk[s] = sm.wk.p ? sm.wk.p + o : nullptr;
+    const size_t o = (5 * step + size_t(s)) * size_t(a_.Kp);
+    r.dtk[s] = a_.lts ? static_cast<void *>(sm.dtk.p + o) : nullptr;
+    r.srck[s] = a_.lts ? sm.srck.p + o : nullptr;
+    r.wk[s] = a_.lts ? sm.wk.p + o : nullptr;
   }
 }
 
@@ -203,10 +193,7 @@ AdjointRunner::StageRecord AdjointRunner::scratch_record() {
     r.U[s] = U_[s].p;
     r.R[s] = R_[s].p;
   }
-  fill_small(r, scratch_small_);
-  r.dts = dts_.p;
-  r.argmax = argmax_.p;
-  r.Wv = Wv_.p;
+  fill_small(r, scratch_small_, 0);
   if (a_.act) {
     const size_t Kp = size_t(a_.Kp), Nv = size_t(a_.Nv), nr = size_t(NR_) * Kp;
     for (int s = 0; s < 5; ++s) {
@@ -389,41 +376,49 @@ void AdjointRunner::vjp(const double *q0, double t0, int nsteps, int every, cons
   const size_t bytes = n_ * sizeof(double);
   // The states a step's transposed stages need (its start, four stage inputs
   // and five right-hand sides: 10) are kept from the forward sweep for the last
-  // blocks, which are then not swept again: as many blocks as fit in a quarter
-  // of the free device memory, but one where the caller chose the spacing (that
-  // bounds the memory). The blocks before them are recomputed from their
-  // checkpoints into the first kept block's states, whose own steps are then
-  // done with; if not even one block fits, each step's record is recomputed
-  // from its start just before its transposed stages.
+  // blocks, which are then not swept again: as many blocks as kept_blocks
+  // allows, but one where the caller chose the spacing (that bounds the
+  // memory). The blocks before them are recomputed from their checkpoints into
+  // the first kept block's states, whose own steps are then done with; if not
+  // even one block fits, each step's record is recomputed from its start just
+  // before its transposed stages.
+  // All records are one allocation, and the checkpoints another: an allocation
+  // for every state took 33 us each, 0.4 ms a step of a first call.
   size_t free_b = 0, total_b = 0;
   HIPCHECK(hipMemGetInfo(&free_b, &total_b));
-  int kept = kept_blocks(free_b, states_.size() * bytes, size_t(nblocks + 1 + every_) * bytes, 10 * size_t(every_) * bytes,
-                         every > 0 ? 1 : nblocks);
+  const size_t step_b = 10 * bytes + (a_.lts ? 5 * size_t(a_.Kp) * (sizeof(dev::ad_storage) + sizeof(int) + sizeof(double)) : 0);
+  int kept = kept_blocks(free_b, ckpt_.n * sizeof(double) + rec_.n / (10 * n_) * step_b, size_t(nblocks + 1 + every_) * bytes,
+                         size_t(every_) * step_b, every > 0 ? 1 : nblocks);
   // GOCFD_ADJOINT_KEEP_RECORDS=0 forces the per-step recomputation
   if (const char *e = std::getenv("GOCFD_ADJOINT_KEEP_RECORDS"))
     if (e[0] == '0') kept = 0;
   // the active sensor path keeps one step's record (its fields per stage)
   if (a_.act) kept = 0;
+  // Checkpoints, the result, and a block's starts where no record holds them;
+  // fewer blocks where the memory has gone since it was counted
+  while (!reserve(size_t(nblocks) + 1 + (kept ? 0 : every_), size_t(kept) * every_)) {
+    if (kept == 0) throw SetupError(GOCFD_ERR_DEVICE, "no device memory for the checkpoints of " + std::to_string(nsteps) + " steps");
+    rec_.free();
+    kept /= 2;
+  }
   stored_records_ = kept > 0;
-  // Pooled states: checkpoints [0, nblocks), the result, a block's starts where
-  // no record holds them, then 10 states per step of a kept block
-  const size_t rec0 = size_t(nblocks + 1 + (stored_records_ ? 0 : every_));
   const int first_kept = nblocks - kept;
+  auto ckpt = [&](int i) { return ckpt_.p + size_t(i) * n_; };
+  auto rec = [&](size_t i) { return rec_.p + i * n_; };
   std::vector<double *> ck(nblocks), S(every_, nullptr);
-  for (int i = 0; i < nblocks; ++i) ck[i] = state(size_t(i));
-  double *const end = state(size_t(nblocks));
-  for (int i = 1; i < every_; ++i) S[i] = state(stored_records_ ? rec0 + 10 * size_t(i) : size_t(nblocks + i));
+  for (int i = 0; i < nblocks; ++i) ck[i] = ckpt(i);
+  double *const end = ckpt(nblocks);
+  for (int i = 1; i < every_; ++i) S[i] = stored_records_ ? rec(10 * size_t(i)) : ckpt(nblocks + i);
   // step i of kept block q (0: the first kept): its start and its record
   std::vector<StageRecord> recs(size_t(kept) * every_);
   std::vector<double *> kept_start(recs.size());
   for (size_t i = 0; i < recs.size(); ++i) {
     StageRecord &r = recs[i];
-    const size_t s0 = rec0 + 10 * i;
-    kept_start[i] = i % every_ == 0 ? nullptr : state(s0);  // a block's first step starts at its checkpoint
+    kept_start[i] = i % every_ == 0 ? nullptr : rec(10 * i);  // a block's first step starts at its checkpoint
     r.U[0] = nullptr;
-    for (int s = 1; s < 5; ++s) r.U[s] = state(s0 + size_t(s));
-    for (int s = 0; s < 5; ++s) r.R[s] = state(s0 + 5 + size_t(s));
-    fill_small(r, small(i));
+    for (int s = 1; s < 5; ++s) r.U[s] = rec(10 * i + size_t(s));
+    for (int s = 0; s < 5; ++s) r.R[s] = rec(10 * i + 5 + size_t(s));
+    fill_small(r, small_, i);
   }
   HIPCHECK(hipMemsetAsync(flag_.p, 0, sizeof(int), s_));
   HIPCHECK(hipMemcpyAsync(time_.p, &t0, sizeof(double), hipMemcpyHostToDevice, s_));
@@ -443,7 +438,7 @@ void AdjointRunner::vjp(const double *q0, double t0, int nsteps, int every, cons
   }
   check_flag();
   // reverse sweep
-  if (!lamU0_.p) {
+  if (!far_d_.p) {  // the last one: a failed call leaves none half made
     lamU0_.alloc(n_);
     for (int s = 1; s < 5; ++s) lamQ_[s].alloc(n_);
     lamR_.alloc(n_);
@@ -515,7 +510,7 @@ void AdjointRunner::jvp(const double *q0, const double *dq0, const double dfar[4
                         double *qn, double *dqn) {
   if (nsteps < 1) throw SetupError(GOCFD_ERR_ARG, "nsteps must be positive");
   for (int c = 0; c < 4; ++c) a_.dfar[c] = dfar ? dfar[c] : 0.;
-  if (!dualA_.p) {
+  if (!dualB_.p) {
     dualA_.alloc(n_);
     dualB_.alloc(n_);
   }

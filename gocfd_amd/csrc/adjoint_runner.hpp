@@ -75,18 +75,17 @@ class AdjointRunner {
   StageRecord scratch_record();
   void check_flag();
   // Buffers kept from call to call (grown on demand, freed with the solver):
-  // element-array states (checkpoints, block starts, stage records) and the
-  // small per-step record arrays
-  double *state(size_t i);
+  // element-array states (checkpoints and block starts; ten per step of the
+  // stage records) and the records' small arrays
   struct SmallRecord {
-    DevBuf<dev::ad_storage> dts, dtk;  // dtk, srck, wk: [5][Kp] with local time stepping
+    DevBuf<dev::ad_storage> dts, dtk;  // per step [5]; dtk, srck, wk: [5][Kp] with local time stepping
     DevBuf<int> argmax, srck;
     DevBuf<double> Wv, wk;
   };
-  void fill_small(StageRecord &r, SmallRecord &sm);
-  SmallRecord &small(size_t i);
-  std::vector<std::unique_ptr<DevBuf<double>>> states_;
-  std::vector<std::unique_ptr<SmallRecord>> smalls_;
+  void fill_small(StageRecord &r, SmallRecord &sm, size_t step);
+  bool reserve(size_t nstates, size_t nsteps);
+  DevBuf<double> ckpt_, rec_;
+  SmallRecord small_;
   DevBuf<double> lamU0_, lamQ_[5], lamR_, lamR3_, lamOwn_, lamFarPts_, lamFarW_, lam_dt_, far_d_;
   DevBuf<dev::ad_storage> dualA_, dualB_;
   SmallRecord scratch_small_;
@@ -103,9 +102,9 @@ class AdjointRunner {
   // stage record (sized for dual values; the double sweeps use the front half)
   DevBuf<dev::ad_storage> U_[5], R_[5];
   DevBuf<dev::ad_storage> FE_, SP_, tmp_;
-  DevBuf<dev::ad_storage> dts_, part_t_;
-  DevBuf<int> argmax_, flag_, part_i_;
-  DevBuf<double> Wv_, time_, part_v_;
+  DevBuf<dev::ad_storage> part_t_;
+  DevBuf<int> flag_, part_i_;
+  DevBuf<double> time_, part_v_;
   int nparts_ = 1024;
   // active PerssonC0 (global time stepping)
   DevBuf<double> shops_, hK_, Nxo_, Nyo_, vooL_;

@@ -20,11 +20,15 @@ namespace capi {
 int fail(int code, const std::string &msg);
 const char *last_error();
 
+// (an error is taken off the runtime's record: the next call's launch checks
+// would report it again)
 #define HIPCHECK(expr)                                                                     \
   do {                                                                                     \
     hipError_t e_ = (expr);                                                                \
-    if (e_ != hipSuccess)                                                                  \
+    if (e_ != hipSuccess) {                                                                \
+      (void)hipGetLastError();                                                             \
       throw ::gocfd::SetupError(GOCFD_ERR_DEVICE, std::string(#expr) + ": " + hipGetErrorString(e_)); \
+    }                                                                                      \
   } while (0)
 
 #define GUARD_BEGIN try {
@@ -57,6 +61,23 @@ struct DevBuf {
   }
   ~DevBuf() { free(); }
 };
+
+// At least count values; false when the device has no memory for them (the
+// buffer is then empty, and the error is taken off the runtime's record)
+template <class T>
+bool grow(DevBuf<T> &b, size_t count) {
+  if (b.n >= count) return true;
+  b.free();
+  const hipError_t e = hipMalloc(&b.p, count * sizeof(T));
+  if (e == hipErrorOutOfMemory) {
+    b.p = nullptr;
+    (void)hipGetLastError();
+    return false;
+  }
+  HIPCHECK(e);
+  b.n = count;
+  return true;
+}
 
 // A host array of doubles on the device in the stage kernel's arithmetic
 // type: FP32 for the FP32-bulk precision from N=2 on, else FP64

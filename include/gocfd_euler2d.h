@@ -204,8 +204,10 @@ int gocfd_euler2d_get_element_dt(gocfd_euler2d *h, double *DT);
  * recomputes the steps from a checkpoint every checkpoint_every steps (0:
  * ceil(sqrt(nsteps))) and each step's stages from its start, except those of
  * the last blocks whose stage records (10 states per step) the forward sweep
- * kept: as many blocks as fit in a quarter of the free device memory with
- * checkpoint_every = 0, at most one otherwise. */
+ * kept: with checkpoint_every = 0 as many blocks as fit, with the checkpoints,
+ * in a quarter of the device memory that is free or that the handle already
+ * holds for them, at most one otherwise; fewer where that memory is gone by
+ * then. The handle holds the memory until it is destroyed. */
 int gocfd_euler2d_vjp(gocfd_euler2d *h, int32_t nsteps, int32_t checkpoint_every, const double *dQn_bar,
                       double *dQ0, double *dQinf);
 /* Jacobian-vector product over nsteps steps (tangent-linear step in dual
