@@ -91,19 +91,35 @@ struct StageTypeBuf {
   const void *ptr() const { return f.p ? static_cast<const void *>(f.p) : static_cast<const void *>(d.p); }
 };
 
+// The stage states q1..q4 of a solver or group, one allocation
+struct StageStates {
+  DevBuf<unsigned char> mem;
+  // nval values of ssize bytes each (4 or 8) per state
+  void alloc(size_t nval, size_t ssize, void *q[5]) {
+    mem.alloc(4 * nval * ssize);
+    for (int s = 1; s < 5; ++s) q[s] = mem.p + size_t(s - 1) * nval * ssize;
+  }
+  // Between calls nothing lives in them (a step's first stage writes q1 before
+  // anything reads it), so state transfers use them: 16 nval bytes or more for
+  // a state's 8 nval
+  double *staging() const { return reinterpret_cast<double *>(mem.p); }
+};
+
 // Host states in the reference layout [4][NpInt][K] to and from the device's
 // tile layout (or element-major, tiled = false). The re-layout runs on the device: the host only
-// copies, through a device staging array of the reference layout's size and,
+// copies, through device memory of the caller's (stage, the state's size) and,
 // for states up to kPin bytes, one pinned host buffer. (On the host the
 // strided re-layout took 14 ms into and 18 ms out of the device at 80,000
 // triangles, order 4, 38 MB; the copies alone take 1.3 and 3.7 ms. A
 // pageable copy of 256 KB took 115 us where the pinned one and its host copy
-// take 14; from 4 MB on the pageable copy is as fast.) One transfer at a time:
-// calls on one handle are not re-entrant, and every entry point waits for its
-// stream before it returns.
+// take 14; from 4 MB on the pageable copy is as fast.) The pinned buffer is
+// allocated at the first transfer, once, for the largest state that the owner
+// will move through it (fit): grown state by state it took nine allocations in
+// the first read of 24 cases, 10 ms. One transfer at a time: calls on one
+// handle are not re-entrant, and every entry point waits for its stream before
+// it returns.
 struct HostIo {
   static constexpr size_t kPin = size_t(4) << 20;
-  DevBuf<double> stage;
   double *pin = nullptr;
   size_t npin = 0;
   dev::Ctl *ctl = nullptr;  // behind the buffer, in the same pinned allocation
@@ -111,40 +127,39 @@ struct HostIo {
   HostIo(const HostIo &) = delete;
   HostIo &operator=(const HostIo &) = delete;
   ~HostIo() { if (pin) (void)hipHostFree(pin); }
-  void reserve(size_t vals) {
-    if (stage.n < vals) stage.alloc(vals);
-    const size_t bytes = vals * sizeof(double), want = bytes <= kPin ? bytes : 0;
-    if (!pin || npin < want) {
-      if (pin) (void)hipHostFree(pin);
-      pin = nullptr;
-      ctl = nullptr;
-      npin = 0;
-      HIPCHECK(hipHostMalloc(reinterpret_cast<void **>(&pin), want + sizeof(dev::Ctl), hipHostMallocDefault));
-      npin = want;
-      ctl = reinterpret_cast<dev::Ctl *>(reinterpret_cast<char *>(pin) + want);
-    }
+  static size_t bytes_of(int K, int NpInt) { return size_t(K) * 4 * NpInt * sizeof(double); }
+  // States of K elements will be moved (all owners call it before the first transfer)
+  void fit(int K, int NpInt) {
+    const size_t bytes = bytes_of(K, NpInt);
+    if (bytes <= kPin) npin = std::max(npin, bytes);
+  }
+  void reserve() {
+    if (pin) return;
+    HIPCHECK(hipHostMalloc(reinterpret_cast<void **>(&pin), npin + sizeof(dev::Ctl), hipHostMallocDefault));
+    ctl = reinterpret_cast<dev::Ctl *>(reinterpret_cast<char *>(pin) + npin);
   }
   // Q is free again on return; the re-layout may still run on the stream
-  void put(const double *Q, const int *perm, int K, int Kp, int NpInt, bool tiled, bool inert, double *dst, hipStream_t s) {
-    const size_t vals = size_t(K) * 4 * NpInt, bytes = vals * sizeof(double);
-    reserve(vals);
-    if (bytes <= kPin) {
+  void put(const double *Q, const int *perm, int K, int Kp, int NpInt, bool tiled, bool inert, double *stage, double *dst,
+           hipStream_t s) {
+    const size_t bytes = bytes_of(K, NpInt);
+    reserve();
+    if (bytes <= npin) {
       std::memcpy(pin, Q, bytes);
-      HIPCHECK(hipMemcpyAsync(stage.p, pin, bytes, hipMemcpyHostToDevice, s));
+      HIPCHECK(hipMemcpyAsync(stage, pin, bytes, hipMemcpyHostToDevice, s));
     } else {
-      HIPCHECK(hipMemcpyAsync(stage.p, Q, bytes, hipMemcpyHostToDevice, s));
+      HIPCHECK(hipMemcpyAsync(stage, Q, bytes, hipMemcpyHostToDevice, s));
       HIPCHECK(hipStreamSynchronize(s));
     }
-    HIPCHECK(dev::launch_gather_state(stage.p, perm, K, Kp, NpInt, tiled, inert, dst, s));
+    HIPCHECK(dev::launch_gather_state(stage, perm, K, Kp, NpInt, tiled, inert, dst, s));
   }
   // Returns when Q is written
-  void get(const double *src, const int *perm, int K, int NpInt, bool tiled, double *Q, hipStream_t s) {
-    const size_t vals = size_t(K) * 4 * NpInt, bytes = vals * sizeof(double);
-    reserve(vals);
-    HIPCHECK(dev::launch_scatter_state(src, perm, K, NpInt, tiled, stage.p, s));
-    HIPCHECK(hipMemcpyAsync(bytes <= kPin ? pin : Q, stage.p, bytes, hipMemcpyDeviceToHost, s));
+  void get(const double *src, const int *perm, int K, int NpInt, bool tiled, double *stage, double *Q, hipStream_t s) {
+    const size_t bytes = bytes_of(K, NpInt);
+    reserve();
+    HIPCHECK(dev::launch_scatter_state(src, perm, K, NpInt, tiled, stage, s));
+    HIPCHECK(hipMemcpyAsync(bytes <= npin ? pin : Q, stage, bytes, hipMemcpyDeviceToHost, s));
     HIPCHECK(hipStreamSynchronize(s));
-    if (bytes <= kPin) std::memcpy(Q, pin, bytes);
+    if (bytes <= npin) std::memcpy(Q, pin, bytes);
   }
 };
 

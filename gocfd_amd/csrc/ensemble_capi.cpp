@@ -113,6 +113,7 @@ struct EnsGroup {
   DevBuf<double> ht;
   StageTypeBuf flux_geo;
   void *q[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  StageStates qstage;                  // q[1..4]
   void *R = nullptr;
   std::vector<double> q0_init;         // initial state, tile layout (tuning restores it)
   // local time stepping
@@ -127,7 +128,7 @@ struct EnsGroup {
   hipStream_t stream = nullptr;        // the group's branch of a parallel graph
   hipEvent_t done = nullptr;
   ~EnsGroup() {
-    for (auto &p : q) if (p) (void)hipFree(p);
+    if (q[0]) (void)hipFree(q[0]);
     if (R) (void)hipFree(R);
     if (done) (void)hipEventDestroy(done);
     if (stream) (void)hipStreamDestroy(stream);
@@ -610,10 +611,8 @@ void build_group(gocfd_ensemble &h, EnsGroup &g) {
   }
   HIPCHECK(hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking));
   HIPCHECK(hipEventCreateWithFlags(&g.done, hipEventDisableTiming));
-  for (int s = 1; s < 5; ++s) {
-    HIPCHECK(hipMalloc(&g.q[s], nval * h.ssize));
-    HIPCHECK(hipMemset(g.q[s], 0, nval * h.ssize));
-  }
+  g.qstage.alloc(nval, h.ssize, g.q);  // every stage writes the whole of its output before the next one reads it
+  for (int ci : g.cases) h.io.fit(h.cases[ci]->L.K, NpInt);
   HIPCHECK(hipMalloc(&g.R, nval * sizeof(double)));
   HIPCHECK(hipMemset(g.R, 0, nval * sizeof(double)));
 }
@@ -731,8 +730,8 @@ int gocfd_ensemble_get_state(gocfd_ensemble *h, int32_t c, double *Q) {
   HIPCHECK(hipSetDevice(h->device));
   const EnsCase &cs = *h->cases[c];
   const EnsGroup &g = *h->groups[cs.group];
-  h->io.get(static_cast<const double *>(g.q[0]) + size_t(cs.off) * g.NV, g.perm.p + cs.off, cs.L.K, cs.d.ops.NpInt, true, Q,
-            h->stream);
+  h->io.get(static_cast<const double *>(g.q[0]) + size_t(cs.off) * g.NV, g.perm.p + cs.off, cs.L.K, cs.d.ops.NpInt, true,
+            g.qstage.staging(), Q, h->stream);
   return GOCFD_OK;
   GUARD_END
 }

@@ -101,7 +101,8 @@ int gocfd_euler2d_create(const gocfd_mesh *mesh, const gocfd_params *p, gocfd_eu
   const size_t nval = size_t(h->L.Kp) * h->NV;
   HIPCHECK(hipMalloc(&h->q[0], nval * sizeof(double)));
   // every stage writes the whole of its output before the next one reads it
-  for (int s = 1; s < 5; ++s) HIPCHECK(hipMalloc(&h->q[s], nval * h->ssize));
+  h->qstage.alloc(nval, h->ssize, h->q);
+  h->io.fit(h->L.K, h->d.ops.NpInt);
   HIPCHECK(hipMalloc(&h->R, nval * sizeof(double)));
   HIPCHECK(hipMemset(h->R, 0, nval * sizeof(double)));
   HIPCHECK(hipMalloc(&h->ctl, sizeof(dev::Ctl)));

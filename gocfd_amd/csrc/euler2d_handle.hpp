@@ -34,6 +34,7 @@ struct gocfd_euler2d {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   // state (tile layout, dev::state_at: Kp * NV values of the storage type)
   void *q[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};
+  StageStates qstage;  // q[1..4]
   void *R = nullptr;
   void *scratch_in = nullptr;
   DevBuf<double> rhs_out;
@@ -73,7 +74,7 @@ struct gocfd_euler2d {
 
   ~gocfd_euler2d() {
     if (stream) (void)hipStreamSynchronize(stream);
-    for (auto &p : q) if (p) (void)hipFree(p);
+    if (q[0]) (void)hipFree(q[0]);
     if (R) (void)hipFree(R);
     if (scratch_in) (void)hipFree(scratch_in);
     if (ctl) (void)hipFree(ctl);
@@ -125,18 +126,20 @@ struct gocfd_euler2d {
   // reference layout [4][NpInt][K] (double) <-> FP64 device buffer in the
   // tile layout (q0 and the RHS-evaluation input) on the handle's stream
   void to_device(const double *Q, void *dst) {
-    io.put(Q, perm.p, L.K, L.Kp, d.ops.NpInt, true, true, static_cast<double *>(dst), stream);
+    io.put(Q, perm.p, L.K, L.Kp, d.ops.NpInt, true, true, qstage.staging(), static_cast<double *>(dst), stream);
   }
   // returns when Q is written
   void from_device(const void *src, double *Q) {
-    io.get(static_cast<const double *>(src), perm.p, L.K, d.ops.NpInt, true, Q, stream);
+    io.get(static_cast<const double *>(src), perm.p, L.K, d.ops.NpInt, true, qstage.staging(), Q, stream);
   }
   // The derivative kernels' element-major buffers: a cotangent or tangent,
   // zero on the padding elements; the way back; and the current state
   void to_device_deriv(const double *Q, double *dst) {
-    io.put(Q, perm.p, L.K, L.Kp, d.ops.NpInt, false, false, dst, stream);
+    io.put(Q, perm.p, L.K, L.Kp, d.ops.NpInt, false, false, qstage.staging(), dst, stream);
   }
-  void from_device_deriv(const double *src, double *Q) { io.get(src, perm.p, L.K, d.ops.NpInt, false, Q, stream); }
+  void from_device_deriv(const double *src, double *Q) {
+    io.get(src, perm.p, L.K, d.ops.NpInt, false, qstage.staging(), Q, stream);
+  }
   const double *state_deriv() {
     if (q0_deriv.n < size_t(L.Kp) * NV) q0_deriv.alloc(size_t(L.Kp) * NV);
     HIPCHECK(dev::launch_element_major(static_cast<const double *>(q[0]), L.Kp, d.ops.NpInt, q0_deriv.p, stream));
