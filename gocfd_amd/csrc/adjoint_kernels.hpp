@@ -165,8 +165,11 @@ __global__ void __launch_bounds__(256) k_adj_fwd_face(AdjArgs a, const T *U, T *
     if (code & FC_WAVE) sp = wave_value(a, code, fi, a.oohK[kk], own, qfar);
   }
   if (in && a.lts) SP[t] = sp;
-  double mv = in ? val_of(sp) : -2.;
-  int mi = in ? int(t) : -1;
+  // a NaN speed does not take part (it ranks before none, and none before it,
+  // so the threads would not agree on the largest)
+  const bool cand = in && val_of(sp) == val_of(sp);
+  double mv = cand ? val_of(sp) : -2.;
+  int mi = cand ? int(t) : -1;
   for (int d = 32; d > 0; d >>= 1) {
     const double ov = __shfl_xor(mv, d, 64);
     const int oi = __shfl_xor(mi, d, 64);
