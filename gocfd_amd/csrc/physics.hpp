@@ -226,17 +226,17 @@ __device__ __forceinline__ bool gamma_is_14(double g) {
 // them, for solvers with FP32 stage states, where a last bit of the FP64 state
 // (or of a boundary wave speed, through dt) can move the next rounding to FP32,
 // and one moved value reaches an element further at each stage: with the other
-// forms a vortex of 12,168 elements at order 4 ended 24 steps 7e-7 away. (They
-// were faster: 100 steps of 80,000 elements at order 4 24.6 ms, 25.8 with Ref, 24
-// cases of 2,000 to 20,000 elements 11.6 and 12.3.) Pow and G14 serve FP64
-// solvers: one power, or for gamma = 1.4 (the caller has checked) none; they
-// differ from Ref by roundings.
-enum class BcForm { Ref, Pow, G14 };
+// form a vortex of 12,168 elements at order 4 ended 24 steps 7e-7 away. (It
+// was faster: 100 steps of 80,000 elements at order 4 24.6 ms, 25.8 with Ref, 24
+// cases of 2,000 to 20,000 elements 11.6 and 12.3.) Also for every gamma but
+// 1.4. G14: gamma = 1.4 (the caller has checked), without a power, for FP64; it
+// differs from Ref by roundings. Any: looks at gamma.
+enum class BcForm { Ref, G14, Any };
 
 // RiemannBC (model_problems/Euler2D/bcs.go:70-133), in FP64 (T = double) or
 // in FP64 dual arithmetic for the tangent-linear and adjoint kernels.
 // pinf/cinf come from the freestream even for the analytic vortex state.
-template <class T, class P, BcForm FORM = BcForm::Pow>
+template <class T, class P, BcForm FORM = BcForm::Any>
 __device__ __forceinline__ void riemann_bc(double g, double minf, P pinf, P cinf, const T qi[4],
                                            const T qinf[4], double nx, double ny, T qb[4]) {
   const T rhoI = qi[0], uI = qi[1] / qi[0], vI = qi[2] / qi[0];
@@ -253,32 +253,24 @@ __device__ __forceinline__ void riemann_bc(double g, double minf, P pinf, P cinf
     const T Vn = 0.5 * (Rint + Rinf);
     const T c = 0.25 * GM1 * (Rint - Rinf);
     T Vt, rho, p;
-    if constexpr (FORM == BcForm::Ref) {
+    if (FORM == BcForm::G14 || (FORM == BcForm::Any && gamma_is_14(g))) {
+      // The boundary density and pressure from c and the entropy of the
+      // upwind side, beta = p0 / rho0^g (far state on inflow, interior on
+      // outflow): rho = (c^2 / (g beta))^(1/(g-1)) is rho0 (c^2 rho0 / (g p0))^2.5
+      // and beta rho^g is rho c^2 / g. A negative density has no power rho0^g,
+      // also where a negative pressure makes the quotient positive.
+      T rho0, p0;
+      if (VnI < 0) { Vt = tx * uF + ty * vF; rho0 = rhoF; p0 = pinf; }
+      else { Vt = tx * uI + ty * vI; rho0 = rhoI; p0 = pI; }
+      const T X = rho0 < 0 ? T(NAN) : c * c * rho0 / (g * p0);
+      rho = rho0 * (X * X * sqrt(X));
+      p = rho * c * c * (1. / g);
+    } else {
       T beta;
       if (VnI < 0) { Vt = tx * uF + ty * vF; beta = pinf / pow(rhoF, g); }
       else { Vt = tx * uI + ty * vI; beta = pI / pow(rhoI, g); }
       rho = pow(c * c / (g * beta), OOGM1);
       p = beta * pow(rho, g);
-    } else {
-      // The boundary density and pressure from c and the entropy of the
-      // upwind side, p0 / rho0^g (far state on inflow, interior on outflow):
-      // rho = (c^2 / (g beta))^(1/(g-1)) with beta = p0 / rho0^g is
-      // rho0 (c^2 rho0 / (g p0))^(1/(g-1)), and beta rho^g = rho c^2 / g, so one
-      // power is left of the formula's three, and none for g = 1.4, where
-      // x^2.5 = x^2 sqrt(x).
-      T rho0, p0;
-      if (VnI < 0) { Vt = tx * uF + ty * vF; rho0 = rhoF; p0 = pinf; }
-      else { Vt = tx * uI + ty * vI; rho0 = rhoI; p0 = pI; }
-      const T X = c * c * rho0 / (g * p0);
-      T Xp;
-      if constexpr (FORM == BcForm::Pow) {
-        if (gamma_is_14(g)) Xp = X * X * sqrt(X);
-        else Xp = pow(X, OOGM1);
-      } else {
-        Xp = X * X * sqrt(X);
-      }
-      rho = rho0 * Xp;
-      p = rho * c * c * (1. / g);
     }
     const T u = Vn * nx + Vt * tx, v = Vn * ny + Vt * ty;
     qb[0] = rho; qb[1] = rho * u; qb[2] = rho * v; qb[3] = p * OOGM1 + 0.5 * rho * (u * u + v * v);

@@ -290,7 +290,7 @@ __device__ __forceinline__ void boundary_state(int kind, const Phys &ph, const d
 // The form of a solver's boundary states: S its stage-state storage, GEN a
 // gamma other than 1.4
 template <class S, bool GEN>
-constexpr BcForm kBcForm = sizeof(S) == 4 ? BcForm::Ref : GEN ? BcForm::Pow : BcForm::G14;
+constexpr BcForm kBcForm = sizeof(S) == 4 || GEN ? BcForm::Ref : BcForm::G14;
 
 // Wave speed (|U| + c) / hK of a face point (StoreEdgeAggregates, edges.go:264-272)
 __device__ __forceinline__ double point_speed(double g, const double q[4], double oohK) {
@@ -1876,7 +1876,7 @@ hipError_t launch_stage_n(int prec, int shock, const StageArgs &a, hipStream_t s
 template <int N>
 hipError_t launch_prologue_n(int prec, const StageArgs &a, hipStream_t s) {
   // it reads q0, which is FP64 in every precision
-  if (prec == 0) hipLaunchKernelGGL((k_prologue<N, BcForm::Pow>), dim3(a.ntiles), dim3(kProThreads), 0, s, a);
+  if (prec == 0) hipLaunchKernelGGL((k_prologue<N, BcForm::Any>), dim3(a.ntiles), dim3(kProThreads), 0, s, a);
   else hipLaunchKernelGGL((k_prologue<N, BcForm::Ref>), dim3(a.ntiles), dim3(kProThreads), 0, s, a);
   return hipGetLastError();
 }
@@ -1930,7 +1930,7 @@ hipError_t launch_shock_t(int pass, const StageArgs &a, hipStream_t s) {
 // evaluation, else the stage state in the precision's storage.
 template <int N>
 hipError_t launch_shock_n(int prec, int pass, const StageArgs &a, hipStream_t s) {
-  if (prec == 0) return launch_shock_t<N, double, double, BcForm::Pow>(pass, a, s);
+  if (prec == 0) return launch_shock_t<N, double, double, BcForm::Any>(pass, a, s);
   if (a.stage <= 0) return launch_shock_t<N, double, BulkC<N>, BcForm::Ref>(pass, a, s);
   return launch_shock_t<N, float, BulkC<N>, BcForm::Ref>(pass, a, s);
 }
