@@ -101,6 +101,7 @@ struct EnsCase {
 struct EnsGroup {
   int N = 0, Kp = 0, ntiles = 0, Hmax = 1, Wmax = 1, Fmax = 1, Xmax = 1, NV = 0;
   bool shock = false, lts = false;  // PerssonC0 limiter, LocalTimeStepping (the same for the group)
+  bool gen = false;                 // FP64 and a gamma other than 1.4: the kernels that take powers
   double kappa = 0;
   int Nv = 0;                       // vertices of the group's cases
   std::vector<int> cases;
@@ -201,8 +202,7 @@ struct gocfd_ensemble {
     a.Interp64 = g.Interp64.p;
     const EnsCase &c0 = *cases[g.cases[0]];
     a.ph = phys_of(c0.fs, c0.prm);
-    for (int ci : g.cases)
-      if (general_gamma(phys_of(cases[ci]->fs, cases[ci]->prm))) a.gen = 1;
+    a.gen = g.gen ? 1 : 0;
     a.lts.on = g.lts ? 1 : 0;
     a.lts.fw = g.fw.p; a.lts.fwv = g.fwv.p; a.lts.wsrc = g.wsrc.p; a.lts.DTk = g.DTk.p; a.lts.DTv = g.DTv.p;
     if (g.shock) {
@@ -250,20 +250,19 @@ struct gocfd_ensemble {
   void enqueue_step(bool branches) {
     const bool multi = parallel == 2 && multi_ok;
     for (int s = 0; s < 5; ++s) {
-      if (multi) {
+      // (one launch for the groups of each kind of gamma)
+      for (int gen = 0; multi && gen < 2; ++gen) {
         dev::MultiArgs m{};
-        m.ngroups = int(mgroups.size());
         m.xcd_tiles = xcd_tiles;
-        for (int gi : mgroups) m.gen |= args(*groups[size_t(gi)]).gen;
+        m.gen = gen;
         m.l = dev::MultiLaunch{s, step_index, int(gstage % 3), int(gstage & 1), int(gstage & 1)};
-        int t0 = 0;
         for (size_t i = 0; i < mgroups.size(); ++i) {
           const EnsGroup &g = *groups[size_t(mgroups[i])];
-          m.g[i] = dev::MultiGroup{margs.p + i, t0, g.N, g.Fmax, g.Wmax + 2 * g.Xmax, g.lts ? 1 : 0};
-          t0 += g.ntiles;
+          if (int(g.gen) != gen) continue;
+          m.g[m.ngroups++] = dev::MultiGroup{margs.p + i, m.ntiles, g.N, g.Fmax, g.Wmax + 2 * g.Xmax, g.lts ? 1 : 0};
+          m.ntiles += g.ntiles;
         }
-        m.ntiles = t0;
-        HIPCHECK(dev::launch_stage_multi(prec, flux, m, stream));
+        if (m.ngroups) HIPCHECK(dev::launch_stage_multi(prec, flux, m, stream));
       }
       for (auto &g : groups) {
         if (multi && !g->shock) continue;
@@ -645,14 +644,16 @@ int gocfd_ensemble_create(int32_t ncases, const gocfd_mesh *const *meshes, const
     c->L = build_device_layout(c->d, dev::kTile, dev::kTP);
     h->cases.push_back(std::move(c));
   }
-  // one group per order, limiter (with its Kappa) and time-stepping mode:
-  // a group shares one kernel variant and one set of shock constants
-  std::map<std::tuple<int, int, int, double>, std::vector<int>> by_kind;
+  // one group per order, limiter (with its Kappa), time-stepping mode and (in
+  // FP64) kind of gamma: a group shares one kernel variant, that of its cases
+  // alone, and one set of shock constants
+  std::map<std::tuple<int, int, int, double, int>, std::vector<int>> by_kind;
   for (int i = 0; i < ncases; ++i) {
     const gocfd_params &p = h->cases[i]->prm;
     const bool shock = p.limiter == 1 && p.polynomial_order != 0;
     const double kappa = shock ? (p.kappa != 0. ? p.kappa : 5.) : 0.;
-    by_kind[std::make_tuple(p.polynomial_order, shock ? 1 : 0, p.local_time_stepping ? 1 : 0, kappa)].push_back(i);
+    const int gen = h->prec == 0 && general_gamma(phys_of(h->cases[i]->fs, p)) ? 1 : 0;
+    by_kind[std::make_tuple(p.polynomial_order, shock ? 1 : 0, p.local_time_stepping ? 1 : 0, kappa, gen)].push_back(i);
   }
   size_t lds = 0;
   for (auto &kv : by_kind) {
@@ -661,6 +662,7 @@ int gocfd_ensemble_create(int32_t ncases, const gocfd_mesh *const *meshes, const
     g->shock = std::get<1>(kv.first) != 0;
     g->lts = std::get<2>(kv.first) != 0;
     g->kappa = std::get<3>(kv.first);
+    g->gen = std::get<4>(kv.first) != 0;
     g->cases = kv.second;
     for (int ci : g->cases) {
       h->cases[ci]->group = int(h->groups.size());
@@ -687,16 +689,18 @@ int gocfd_ensemble_create(int32_t ncases, const gocfd_mesh *const *meshes, const
     // the groups without shock capturing, for the multi-order launch
     std::vector<dev::StageArgs> ma;
     bool ok = true;
+    size_t kind[2] = {0, 0};  // groups of a launch
     for (size_t i = 0; i < h->groups.size(); ++i) {
       const EnsGroup &g = *h->groups[i];
       if (g.shock) continue;
       ok = ok && g.Fmax <= dev::kThreads && g.Wmax <= dev::kThreads && g.Xmax <= dev::kThreads;
       h->mgroups.push_back(int(i));
+      ++kind[g.gen ? 1 : 0];
       ma.push_back(h->args(g));
     }
     // FP64 only: the FP32 multi-order kernel faulted the GPU in its first
     // run and stays off until that is explained
-    h->multi_ok = ok && h->prec == 0 && !ma.empty() && ma.size() <= size_t(dev::kMultiMax);
+    h->multi_ok = ok && h->prec == 0 && !ma.empty() && std::max(kind[0], kind[1]) <= size_t(dev::kMultiMax);
     if (h->multi_ok) h->margs.upload(ma);
   }
   h->restart();

@@ -141,7 +141,7 @@ struct StageArgs {
   int step_index;      // steps since the state was set (selects time parity)
   int ring;            // global stage counter mod 3
   int par2;            // global stage counter mod 2
-  int gen;             // 1: a case's gamma is not 1.4 (in FP64 the boundary state then needs a power)
+  int gen;             // 1: the cases' gamma is not 1.4 (in FP64 their boundary states need powers)
   int hpar;            // halo-trace buffer holding this stage's input traces
   // Halo-trace buffers [2][ntiles Fmax][NpEdge][4] in the stage arithmetic
   // type (without shock capturing): by tile and flux-list item, the traces
@@ -222,7 +222,7 @@ struct MultiLaunch {
 };
 struct MultiArgs {
   int ngroups, ntiles, xcd_tiles;
-  int gen;  // a group's gen
+  int gen;  // the groups' gen
   MultiLaunch l;
   MultiGroup g[kMultiMax];
 };
