@@ -232,8 +232,7 @@ struct gocfd_ensemble {
         HIPCHECK(dev::launch_fill_u64(g->epsV.p, g->epsV.n, 0ull, stream));
       }
       if (g->lts) HIPCHECK(dev::launch_fill_f64(g->DTv.p, g->DTv.n, 0.0, stream));
-      // with shock capturing each stage's gradient pass measures its wave speeds
-      if (g->shock) continue;
+      if (g->shock) continue;  // a pass of the first stage measures its wave speeds
       dev::StageArgs a = args(*g);
       a.qs = g->q[0];
       a.ring = 0;
@@ -698,8 +697,8 @@ int gocfd_ensemble_create(int32_t ncases, const gocfd_mesh *const *meshes, const
       ++kind[g.gen ? 1 : 0];
       ma.push_back(h->args(g));
     }
-    // FP64 only: the FP32 multi-order kernel faulted the GPU in its first
-    // run and stays off until that is explained
+    // FP64 only: no FP32 multi-order kernel is built (it spilled vector
+    // registers, which the compiler can place wrongly)
     h->multi_ok = ok && h->prec == 0 && !ma.empty() && std::max(kind[0], kind[1]) <= size_t(dev::kMultiMax);
     if (h->multi_ok) h->margs.upload(ma);
   }

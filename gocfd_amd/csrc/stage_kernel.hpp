@@ -32,9 +32,10 @@
 // From N=3 on without shock capturing, the FluxEdgeInterp (A, F) and DivInt
 // (C) contractions run on the matrix cores as 16x16x4 FP32 or FP64 MFMA
 // tiles, with the element state held in the MFMA result-row layout.
-// With shock capturing three passes precede each stage launch: the sensor
-// with the vertex max-merge, the element viscosity fields (and the stage-2
-// state filter), and the RT gradient with the stage's wave speeds.
+// With shock capturing passes precede each stage launch: the sensor with the
+// vertex max-merge, the element viscosity fields with the viscous speeds, at
+// stage 2 and after a restart the wave speeds (stage 2's state filter first),
+// and eps * gradient of the active elements.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -383,9 +384,12 @@ __device__ __forceinline__ C dot2(C a, C x, C b, C y) {
 // Stage 4 of SSP54 (euler.go:555-565): R = -q0 + a q2 + b q3 + c q4 + d dt R3 +
 // e dt RHS, on the VALU path with FP32 stage states. A last bit of q0 can
 // move the next rounding to an FP32 stage state by 6e-8, so the roundings of
-// the sum are pinned: the products with q2 and q3 are rounded for the last
-// three of every NpInt values of the tile in element order (split), fused for
-// the others.
+// the sum are pinned to those that FP32 results have had: the products with q2
+// and q3 are rounded for the last 3 kThreads of a tile's 64 4 NpInt values in
+// element order (split; a thread's second chunk of loads, when the combination
+// went over the tile in that order), fused for the others. Neither is the more
+// accurate one; one order for all would move FP32 results of order 2 and of
+// shock capturing.
 __device__ __forceinline__ double ssp_last_f32(bool split, double q0, double q2, double q3, double q4, double dtR3,
                                                double dtR) {
 #pragma clang fp contract(off)
@@ -1237,18 +1241,18 @@ __device__ __forceinline__ void stage_tile(const StageArgs &a, const StageLaunch
       if (lts) atomicMax(&sWf[e * 3 + f], bits(wsp));
     }
     if constexpr (HX) {
-    V4 *hout = static_cast<V4 *>(a.ht) + size_t(l.hpar ^ 1) * a.ntiles * a.Fmax * NpEdge;
+      V4 *hout = static_cast<V4 *>(a.ht) + size_t(l.hpar ^ 1) * a.ntiles * a.Fmax * NpEdge;
 #pragma unroll
-    for (int j = 0; j < ITG; ++j) {
-      const int it = tid + j * kThreads;
-      if (it < nxp) {
-        const int w = it / NpEdge, pp = it - w * NpEdge;
-        const int xk = sXP[w];
-        const int e = xk & 255, f = (xk >> 8) & 3, p = f * NpEdge + pp;
-        hout[size_t(sXD[w]) * NpEdge + (NpEdge - 1 - pp)] =
-            V4{sT[p * kTP + e], sT[TS + p * kTP + e], sT[2 * TS + p * kTP + e], sT[3 * TS + p * kTP + e]};
+      for (int j = 0; j < ITG; ++j) {
+        const int it = tid + j * kThreads;
+        if (it < nxp) {
+          const int w = it / NpEdge, pp = it - w * NpEdge;
+          const int xk = sXP[w];
+          const int e = xk & 255, f = (xk >> 8) & 3, p = f * NpEdge + pp;
+          hout[size_t(sXD[w]) * NpEdge + (NpEdge - 1 - pp)] =
+              V4{sT[p * kTP + e], sT[TS + p * kTP + e], sT[2 * TS + p * kTP + e], sT[3 * TS + p * kTP + e]};
+        }
       }
-    }
     }
   }
   wl = wave_max(wl);
@@ -1581,7 +1585,7 @@ __global__ void __launch_bounds__(256) k_shock_prep(StageArgs a) {
 // 11.1 -> 8.7 at order 2 in FP64, 249,386; this pass 9.6 -> 12.6 and 23.6 ->
 // 32.0 of stage 2.)
 template <int N, class SIN, class D, BcForm FORM>
-__global__ void __launch_bounds__(kThreads) k_shock_grad(StageArgs a) {
+__global__ void __launch_bounds__(kThreads) k_shock_speed(StageArgs a) {
   using Sh = Shape<N>;
   constexpr int NpInt = Sh::NpInt, NpEdge = Sh::NpEdge, NpFlux = Sh::NpFlux, NF = Sh::NF, NV = Sh::NV,
                 E = kTile;
@@ -1913,7 +1917,7 @@ hipError_t launch_shock_t(int pass, const StageArgs &a, hipStream_t s) {
       hipLaunchKernelGGL((k_shock_prep<N, SIN>), dim3((a.Kp + 255) / 256), dim3(256), 0, s, a);
       break;
     case 2:
-      hipLaunchKernelGGL((k_shock_grad<N, SIN, D, FORM>), dim3(a.ntiles), dim3(kThreads), 0, s, a);
+      hipLaunchKernelGGL((k_shock_speed<N, SIN, D, FORM>), dim3(a.ntiles), dim3(kThreads), 0, s, a);
       break;
     case 3:
       hipLaunchKernelGGL((k_shock_grad_act<N, SIN, D>),
@@ -2025,12 +2029,10 @@ hipError_t upload_operators_n(const double *divT, const double *interp) {
 namespace gocfd {
 namespace dev {
 
-template <int N, class S>
-using MultiC = typename std::conditional<(sizeof(S) == 8 || N <= 1), double, float>::type;
-
-// KIND 0: stage 0 (input q0), 1: stages 1-3, 2: stage 4. Two waves per SIMD:
+// FP64 only: an FP32 kernel of all orders spilled vector registers, which this
+// compiler can place wrongly (see StageWaves). KIND 0: stage 0 (input q0), 1: stages 1-3, 2: stage 4. Two waves per SIMD:
 // the five orders' bodies in one kernel spill vector registers at three.
-template <class S, int FLUX, int KIND, bool GEN>
+template <int FLUX, int KIND, bool GEN>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
 k_stage_multi(MultiArgs m) {
   const int t = tile_of_block(m.xcd_tiles);
@@ -2042,23 +2044,22 @@ k_stage_multi(MultiArgs m) {
   const StageLaunch l{st, m.l.step_index, m.l.ring, m.l.par2, m.l.hpar,
                       st == 0 ? a.q0 : st == 1 ? a.q1 : st == 2 ? a.q2 : st == 3 ? a.q3 : a.q4, 0., nullptr};
   const int tile = t - m.g[g].tile0;
-  using SIN = typename std::conditional<KIND == 0, double, S>::type;
   constexpr bool LAST = KIND == 2;
   switch (m.g[g].N) {
-    case 0: stage_tile<0, S, SIN, MultiC<0, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
-    case 1: stage_tile<1, S, SIN, MultiC<1, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
-    case 2: stage_tile<2, S, SIN, MultiC<2, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
-    case 3: stage_tile<3, S, SIN, MultiC<3, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
-    default: stage_tile<4, S, SIN, MultiC<4, S>, FLUX, LAST, false, GEN>(a, l, tile); break;
+    case 0: stage_tile<0, double, double, double, FLUX, LAST, false, GEN>(a, l, tile); break;
+    case 1: stage_tile<1, double, double, double, FLUX, LAST, false, GEN>(a, l, tile); break;
+    case 2: stage_tile<2, double, double, double, FLUX, LAST, false, GEN>(a, l, tile); break;
+    case 3: stage_tile<3, double, double, double, FLUX, LAST, false, GEN>(a, l, tile); break;
+    default: stage_tile<4, double, double, double, FLUX, LAST, false, GEN>(a, l, tile); break;
   }
 }
 
-template <class S, int FLUX, int KIND, bool GEN>
+template <int FLUX, int KIND, bool GEN>
 static hipError_t launch_multi_k(const MultiArgs &m, hipStream_t s) {
   size_t lds = 0;
   for (int g = 0; g < m.ngroups; ++g) {
     const MultiGroup &G = m.g[g];
-    const size_t cs = sizeof(S) == 8 || G.N <= 1 ? sizeof(double) : sizeof(float);
+    const size_t cs = sizeof(double);
     size_t b = 0;
     switch (G.N) {
       case 0: b = lds_bytes_n<0>(cs, 0, G.Fmax, G.WXints, G.lts != 0); break;
@@ -2071,29 +2072,27 @@ static hipError_t launch_multi_k(const MultiArgs &m, hipStream_t s) {
   }
   static size_t attr_bytes = 0;  // dynamic LDS the kernel is currently allowed
   if (lds > 64 * 1024 && lds > attr_bytes) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_stage_multi<S, FLUX, KIND, GEN>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&k_stage_multi<FLUX, KIND, GEN>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
     attr_bytes = lds;
   }
   const int q = (m.ntiles + 7) / 8;
-  hipLaunchKernelGGL((k_stage_multi<S, FLUX, KIND, GEN>), dim3(8 * q), dim3(kThreads), lds, s, m);
+  hipLaunchKernelGGL((k_stage_multi<FLUX, KIND, GEN>), dim3(8 * q), dim3(kThreads), lds, s, m);
   return hipGetLastError();
 }
 
 template <>
 hipError_t launch_stage_multi_f<GOCFD_MULTI_FLUX>(int prec, const MultiArgs &m, hipStream_t s) {
-  // FP64 only: the FP32 variant (switched off) spilled vector registers,
-  // which this compiler can place wrongly; see StageWaves
   if (prec != 0) return hipErrorNotSupported;
   for (int g = 0; g < m.ngroups; ++g)
     if (m.g[g].Fmax > kThreads || m.g[g].WXints > 3 * kThreads) return hipErrorInvalidValue;
   const int kind = m.l.stage == 0 ? 0 : m.l.stage == 4 ? 2 : 1;
   if (kind == 0)
-    return m.gen ? launch_multi_k<double, GOCFD_MULTI_FLUX, 0, true>(m, s) : launch_multi_k<double, GOCFD_MULTI_FLUX, 0, false>(m, s);
+    return m.gen ? launch_multi_k<GOCFD_MULTI_FLUX, 0, true>(m, s) : launch_multi_k<GOCFD_MULTI_FLUX, 0, false>(m, s);
   if (kind == 2)
-    return m.gen ? launch_multi_k<double, GOCFD_MULTI_FLUX, 2, true>(m, s) : launch_multi_k<double, GOCFD_MULTI_FLUX, 2, false>(m, s);
-  return m.gen ? launch_multi_k<double, GOCFD_MULTI_FLUX, 1, true>(m, s) : launch_multi_k<double, GOCFD_MULTI_FLUX, 1, false>(m, s);
+    return m.gen ? launch_multi_k<GOCFD_MULTI_FLUX, 2, true>(m, s) : launch_multi_k<GOCFD_MULTI_FLUX, 2, false>(m, s);
+  return m.gen ? launch_multi_k<GOCFD_MULTI_FLUX, 1, true>(m, s) : launch_multi_k<GOCFD_MULTI_FLUX, 1, false>(m, s);
 }
 
 template <>
