@@ -431,14 +431,15 @@ __device__ __forceinline__ double ssp_mid(const SspCoef &k, double q0, double qs
 // per wave, and the combination E is lane-local. Whole runs with their state
 // transfers, boundary lists included: order 2 FP64, 320,000 elements, 50 steps
 // 106 -> 33.7 ms; order 4, 80,000 elements, 100 steps in FP64 66.1 -> 32.9 ms,
-// in FP32 58.4 -> 25.6 ms.
+// in FP32 58.4 -> 25.6 ms (25.8 with the boundary state of BcForm::Ref).
 // What is left is latency and instructions: a tile's phases are chains of
 // loads and FP64 arithmetic with barriers between, 10 us for a tile alone.
 // Phase E's operands are therefore loaded under phase C, face points are taken
 // four at a time, the stage's coefficients are chosen once, and one Riemann
 // evaluation serves owners and others. Stage (FP64 unless said) before -> after
 // these: order 1, 3,034 elements 12.8 -> 12.0 us; order 2, 320,000 elements
-// 96.3 -> 90.6; order 4, 80,000 elements 55.3 -> 50.7, FP32 38.2 -> 37.3;
+// 96.3 -> 90.6; order 4, 80,000 elements 55.3 -> 50.7, FP32 38.2 -> 37.3 (38.9
+// with BcForm::Ref);
 // shock capturing at order 2, 249,386 elements 98.3 -> 85.4.
 // S: storage of the stage states q1..q4; SIN: storage of this stage's
 // input (q0 at stage 0 and for the RHS evaluation, else S). q0 and the
